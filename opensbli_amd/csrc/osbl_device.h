@@ -143,32 +143,45 @@ __device__ __forceinline__ void st_once(double v, double* p, int nt) {
   else *p = v;
 }
 
-// a/b (a of either sign) and 1/b for positive normal b far from the
-// overflow range:
-// the hardware reciprocal estimate refined by a Newton-Raphson step, the
-// quotient then corrected once by its residual (Markstein's method); within
-// an ulp of the correctly rounded result, in about half the instructions of
-// the IEEE division sequence, which must also handle scaling and special
-// operands.
+// Quotients and roots of positive normal operands far from the overflow range,
+// from the hardware estimates (measured: v_rcp_f64 within 2^-24.4, v_rsq_f64
+// within 2^-24.2), in about half the instructions of the IEEE sequences, which
+// must also handle scaling and special operands.
+//
+// a/b: one Newton-Raphson step for the reciprocal, the quotient then corrected
+// once by its residual (Markstein's method); within an ulp of the correctly
+// rounded result.
 __device__ __forceinline__ double quot_pos(double a, double b) {
   double r = __builtin_amdgcn_rcp(b);
   r = __fma_rn(__fma_rn(-b, r, 1.0), r, r);
   const double q = a * r;
   return __fma_rn(__fma_rn(-b, q, a), r, q);
 }
-// sqrt(x) for positive normal x: the hardware reciprocal-square-root
-// estimate refined by a Newton-Raphson step, then y = x r corrected once by
-// its residual, y + r (x - y^2)/2; within an ulp of the correctly rounded root.
-__device__ __forceinline__ double sqrt_pos(double x) {
-  double r = __builtin_amdgcn_rsq(x);
-  r = r * __fma_rn(-0.5 * x * r, r, 1.5);
-  const double y = x * r;
-  return __fma_rn(0.5 * r, __fma_rn(-y, y, x), y);
+// The following add the first two terms of the series in the estimate's error
+// e (2^-24, so e^3 is below rounding) in one step: 1/(1-e) = 1 + e + e^2 and
+// 1/sqrt(1-2e) = 1 + e + 3/2 e^2; within an ulp or so, one or two
+// instructions shorter than two refinements.
+__device__ __forceinline__ double quot_near(double a, double b) {
+  const double r = __builtin_amdgcn_rcp(b);
+  const double e = __fma_rn(-b, r, 1.0), q = a * r;
+  return __fma_rn(q, __fma_rn(e, e, e), q);
 }
 __device__ __forceinline__ double recip_pos(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  r = __fma_rn(__fma_rn(-b, r, 1.0), r, r);
-  return __fma_rn(__fma_rn(-b, r, 1.0), r, r);
+  const double r = __builtin_amdgcn_rcp(b);
+  const double e = __fma_rn(-b, r, 1.0);
+  return __fma_rn(r, __fma_rn(e, e, e), r);
+}
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double y = x * r;
+  const double e = __fma_rn(-0.5 * r, y, 0.5);
+  return __fma_rn(y, __fma_rn(1.5 * e, e, e), y);
+}
+// max(m, |x|) in one instruction (fmax first quiets its operands)
+__device__ __forceinline__ double max_abs(double m, double x) {
+  double r;
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(x));
+  return r;
 }
 
 // Every operation is rounded on its own (no contraction into FMAs), so a
@@ -249,7 +262,7 @@ struct RoeF {
 template <int ND>
 __device__ __forceinline__ void roe_factors(const Pt<ND>& P, double& sq, double& h) {
   sq = sqrt_pos(P.q[0]);
-  h = (P.q[ND + 1] + P.p) * quot_pos(sq, P.q[0]);
+  h = (P.q[ND + 1] + P.p) * quot_near(sq, P.q[0]);
 }
 
 template <int ND>
@@ -510,12 +523,6 @@ __device__ __forceinline__ void weno5z_nd(double fm2, double fm1, double f0, dou
   den = 6.0 * (A0 + A1 + A2);
 }
 
-__device__ __forceinline__ double weno5z(double fm2, double fm1, double f0, double f1, double f2) {
-  double n, d;
-  weno5z_nd(fm2, fm1, f0, f1, f2, n, d);
-  return n / d;
-}
-
 // n1/d1 + n2/d2 with one division: (n1 d2 + n2 d1)/(d1 d2).  The weights'
 // denominators grow like beta^6 (at least ~1e-85 from eps), so d1 d2 is a
 // normal number unless |f| exceeds ~1e12; then the two quotients are formed
@@ -545,12 +552,6 @@ __device__ __forceinline__ void weno5js_nd(double fm2, double fm1, double f0, do
   const double r2 = 2.0 * fm2 - 7.0 * fm1 + 11.0 * f0;
   num = A0 * r0 + A1 * r1 + A2 * r2;
   den = 6.0 * (A0 + A1 + A2);
-}
-
-__device__ __forceinline__ double weno5js(double fm2, double fm1, double f0, double f1, double f2) {
-  double n, d;
-  weno5js_nd(fm2, fm1, f0, f1, f2, n, d);
-  return n / d;
 }
 
 // WENO5-JS as above, also returning the shock sensor of its non-linear
@@ -690,73 +691,9 @@ __device__ __forceinline__ void teno_nd(double fm2, double fm1, double f0, doubl
   }
 }
 
-// The same with one division per quotient (kernels that keep their stencil
-// in registers: the shared-division form needs more registers than they
-// have); the quotients are all of positive operands (eps + beta > 0, sums of
-// weights >= 1), formed by quot_pos / recip_pos.
-template <bool SIX, bool QUIRK>
-__device__ __forceinline__ double teno(double fm2, double fm1, double f0, double f1, double f2, double f3,
-                                       double eps, double ct) {
-  constexpr double C13 = 13.0 / 12.0;
-  double q;
-  q = fm1 - f1;
-  double b0 = 0.25 * q * q;
-  q = fm1 - 2.0 * f0 + f1;
-  b0 += C13 * q * q;
-  q = 3.0 * f0 - 4.0 * f1 + f2;
-  double b1 = 0.25 * q * q;
-  q = f0 - 2.0 * f1 + f2;
-  b1 += C13 * q * q;
-  q = fm2 - 4.0 * fm1 + 3.0 * f0;
-  double b2 = 0.25 * q * q;
-  q = fm2 - 2.0 * fm1 + f0;
-  b2 += C13 * q * q;
-  constexpr double S6 = 1.0 / 6.0;
-  const double r0 = (-fm1 + 5.0 * f0 + 2.0 * f1) * S6;
-  const double r1 = (2.0 * f0 + 5.0 * f1 - f2) * S6;
-  const double r2 = (2.0 * fm2 - 7.0 * fm1 + 11.0 * f0) * S6;
-  if constexpr (SIX) {
-    q = -11.0 * f0 + 18.0 * f1 - 9.0 * f2 + 2.0 * f3;
-    double b3 = (1.0 / 36.0) * q * q;
-    q = 2.0 * f0 - 5.0 * f1 + 4.0 * f2 - f3;
-    b3 += C13 * q * q;
-    q = -f0 + 3.0 * f1 - 3.0 * f2 + f3;
-    if constexpr (QUIRK) b3 += (781.0 / 720.0) * q;
-    else b3 += (781.0 / 720.0) * q * q;
-    const double r3 = (3.0 * f0 + 13.0 * f1 - 5.0 * f2 + f3) * (1.0 / 12.0);
-    const double tau = fabs(b3 - (b0 + b2 - 4.0 * b1) * S6);
-    const double a0 = pow6(1.0 + quot_pos(tau, eps + b0));
-    const double a1 = pow6(1.0 + quot_pos(tau, eps + b1));
-    const double a2 = pow6(1.0 + quot_pos(tau, eps + b2));
-    const double a3 = pow6(1.0 + quot_pos(tau, eps + b3));
-    const double ias = recip_pos(a0 + a1 + a2 + a3);
-    const double d0 = (a0 * ias < ct) ? 0.0 : 1.0;
-    const double d1 = (a1 * ias < ct) ? 0.0 : 1.0;
-    const double d2 = (a2 * ias < ct) ? 0.0 : 1.0;
-    const double d3 = (a3 * ias < ct) ? 0.0 : 1.0;
-    constexpr double D0 = 231.0 / 500.0, D1 = 3.0 / 10.0, D2 = 27.0 / 500.0, D3 = 23.0 / 125.0;
-    const double w0 = D0 * d0, w1 = D1 * d1, w2 = D2 * d2, w3 = D3 * d3;
-    const double iws = recip_pos(w0 + w1 + w2 + w3);
-    return (w0 * r0 + w1 * r1 + w2 * r2 + w3 * r3) * iws;
-  } else {
-    const double tau = fabs(b0 - b2);
-    const double a0 = pow6(1.0 + quot_pos(tau, eps + b0));
-    const double a1 = pow6(1.0 + quot_pos(tau, eps + b1));
-    const double a2 = pow6(1.0 + quot_pos(tau, eps + b2));
-    const double ias = recip_pos(a0 + a1 + a2);
-    const double d0 = (a0 * ias < ct) ? 0.0 : 1.0;
-    const double d1 = (a1 * ias < ct) ? 0.0 : 1.0;
-    const double d2 = (a2 * ias < ct) ? 0.0 : 1.0;
-    constexpr double D0 = 11.0 / 20.0, D1 = 4.0 / 10.0, D2 = 1.0 / 20.0;
-    const double w0 = D0 * d0, w1 = D1 * d1, w2 = D2 * d2;
-    const double iws = recip_pos(w0 + w1 + w2);
-    return (w0 * r0 + w1 * r1 + w2 * r2) * iws;
-  }
-}
-
 // Sum of the right reconstruction of f+ and the left reconstruction of f-
 // (shock_capturing.py:257-265) for one characteristic field.
-template <int CONV, bool SHARED = true>
+template <int CONV>
 __device__ __forceinline__ double recon_pair(const double fp[6], const double fm[6], double eps, double ct) {
   if constexpr (CONV == OSBL_CONV_WENO_Z) {
     double n1, d1, n2, d2;
@@ -768,12 +705,6 @@ __device__ __forceinline__ double recon_pair(const double fp[6], const double fm
     weno5js_nd(fp[0], fp[1], fp[2], fp[3], fp[4], n1, d1);
     weno5js_nd(fm[5], fm[4], fm[3], fm[2], fm[1], n2, d2);
     return sum_quotients(n1, d1, n2, d2);
-  } else if constexpr (!SHARED && CONV == OSBL_CONV_TENO6) {
-    return teno<true, true>(fp[0], fp[1], fp[2], fp[3], fp[4], fp[5], eps, ct) +
-           teno<true, false>(fm[5], fm[4], fm[3], fm[2], fm[1], fm[0], eps, ct);
-  } else if constexpr (!SHARED) {
-    return teno<false, false>(fp[0], fp[1], fp[2], fp[3], fp[4], fp[5], eps, ct) +
-           teno<false, false>(fm[5], fm[4], fm[3], fm[2], fm[1], fm[0], eps, ct);
   } else if constexpr (CONV == OSBL_CONV_TENO6) {
     double n1, d1, n2, d2;
     teno_nd<true, true>(fp[0], fp[1], fp[2], fp[3], fp[4], fp[5], eps, ct, n1, d1);
@@ -825,16 +756,326 @@ struct LdsWindow {
   }
 };
 
+// The same from LDS with the fields of a point next to each other, STRIDE
+// doubles from point to point: with an odd stride the lanes of a wave, on
+// consecutive points, hit different banks, and one address with constant
+// offsets reaches every value of the six points.
+template <int ND, int STRIDE>
+struct LdsPoints {
+  static constexpr bool STREAM = true;
+  const double* s;  // field 0 of point 0
+  __device__ __forceinline__ double f(int p, int e) const { return s[p * STRIDE + e]; }
+  __device__ __forceinline__ double q(int p, int m) const { return f(p, m); }
+  __device__ __forceinline__ double u(int p, int m) const { return f(p, ND + 2 + m); }
+  __device__ __forceinline__ double pr(int p) const { return f(p, 2 * ND + 2); }
+  __device__ __forceinline__ double a(int p) const { return f(p, 2 * ND + 3); }
+  __device__ __forceinline__ void point(int p, Pt<ND>& out) const {
+#pragma unroll
+    for (int m = 0; m < ND + 2; ++m) out.q[m] = q(p, m);
+#pragma unroll
+    for (int m = 0; m < ND; ++m) out.u[m] = u(p, m);
+    out.p = pr(p);
+    out.a = a(p);
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Reconstructions in difference form.  A reconstruction at i+1/2 is the value
+// at the upwind point plus a combination of the differences of neighbouring
+// points, so it is evaluated from the differences A = f[-1]-f[-2],
+// B = f[0]-f[-1], C = f[1]-f[0], Dd = f[2]-f[1] (and E = f[3]-f[2], TENO6) of
+// the stencil alone: the candidates are f[0] + c_r/6 with
+//   c_0 = 4C - Dd, c_1 = B + 2C, c_2 = 5B - 2A,
+// and *_gap return sum(omega_r c_r) as num/den.  The left reconstruction
+// (weno.py side -1, of f- on the mirrored points) is the right one of the
+// mirrored differences with the sign turned -- except for TENO6, whose
+// right-side fourth indicator has the unsquared 781/720 term
+// (teno.py:166-167), hence the QUIRK flag.
+// ---------------------------------------------------------------------------
+
+// WENO5-Z (weno.py:283-338, eps = 1e-14, p = 2) and WENO5-JS
+// (weno.py:341-369, eps = 1e-6).  The indicators are taken 12/13 times:
+// t^2 + 3/13 s^2, with eps 12/13 times to match.  The weights
+// d_r (1 + tau^2/e_r^2) (Z) and d_r/e_r^2 (JS) are multiplied by
+// 10 e_0^2 e_1^2 e_2^2, which leaves omega_r unchanged and needs no division.
+template <bool Z>
+__device__ __forceinline__ void weno5_gap(double A, double B, double C, double Dd, double eps, double& num,
+                                          double& den) {
+  constexpr double K = 3.0 / 13.0;
+  const double t0 = Dd - C, t1 = C - B, t2 = B - A;
+  const double s0 = __fma_rn(-2.0, C, t0), s1 = B + C, s2 = __fma_rn(2.0, B, t2);
+  const double e0 = __fma_rn(t0, t0, __fma_rn(K * s0, s0, eps));
+  const double e1 = __fma_rn(t1, t1, __fma_rn(K * s1, s1, eps));
+  const double e2 = __fma_rn(t2, t2, __fma_rn(K * s2, s2, eps));
+  const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
+  double a0 = q1 * q2, a1 = q0 * q2, a2 = q0 * q1;
+  if constexpr (Z) {
+    const double tau = e0 - e2;
+    const double tt = tau * tau, q = a2 * q2;
+    a0 = __fma_rn(tt, a0, q);
+    a1 = __fma_rn(tt, a1, q);
+    a2 = __fma_rn(tt, a2, q);
+  }
+  a0 *= 3.0;
+  a1 *= 6.0;
+  num = a0 * __fma_rn(4.0, C, -Dd) + a1 * __fma_rn(2.0, C, B) + a2 * __fma_rn(5.0, B, -2.0 * A);
+  den = a0 + a1 + a2;
+}
+
+// TENO5 / TENO6 (teno.py:57-234, 407-465): alpha_r = (1 + tau/e_r)^6,
+// e_r = eps + beta_r; delta_r = 0 where alpha_r < C_T sum(alpha), and
+// omega_r = d_r delta_r / sum(d delta).  The quotients tau/e_r share one
+// division by the product of the e_r.  eps comes at least 1e-70 (osbl_create),
+// so the product stays normal for differences up to ~1e37.
+template <bool SIX, bool QUIRK>
+__device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd, double E, double eps, double ct,
+                                         double& num, double& den) {
+  constexpr double C13 = 13.0 / 12.0;
+  const double t0 = C - B, s0 = B + C;
+  const double t1 = Dd - C, s1 = __fma_rn(-2.0, C, t1);
+  const double t2 = B - A, s2 = __fma_rn(2.0, B, t2);
+  const double b0 = C13 * t0 * t0 + 0.25 * s0 * s0;
+  const double b1 = C13 * t1 * t1 + 0.25 * s1 * s1;
+  const double b2 = C13 * t2 * t2 + 0.25 * s2 * s2;
+  const double e0 = eps + b0, e1 = eps + b1, e2 = eps + b2;
+  const double c0 = __fma_rn(2.0, C, B), c1 = __fma_rn(4.0, C, -Dd), c2 = __fma_rn(5.0, B, -2.0 * A);
+  if constexpr (SIX) {
+    const double p3 = 11.0 * C - 7.0 * Dd + 2.0 * E;
+    const double r3 = 3.0 * Dd - 2.0 * C - E;
+    const double q3 = C - 2.0 * Dd + E;
+    double b3 = (1.0 / 36.0) * p3 * p3 + C13 * r3 * r3;
+    // f+- are half the differences that come in: the unsquared term counts double
+    if constexpr (QUIRK) b3 += 2.0 * (781.0 / 720.0) * q3;
+    else b3 += (781.0 / 720.0) * q3 * q3;
+    const double c3 = 4.5 * C - 2.0 * Dd + 0.5 * E;
+    const double tau = fabs(b3 - (b0 + b2 - 4.0 * b1) * (1.0 / 6.0));
+    const double e3 = eps + b3;
+    const double p01 = e0 * e1, p23 = e2 * e3;
+    const double tp = quot_near(tau, p01 * p23);
+    const double a0 = pow6(__fma_rn(e1 * p23, tp, 1.0)), a1 = pow6(__fma_rn(e0 * p23, tp, 1.0));
+    const double a2 = pow6(__fma_rn(e3 * p01, tp, 1.0)), a3 = pow6(__fma_rn(e2 * p01, tp, 1.0));
+    const double cut = ct * (a0 + a1 + a2 + a3);
+    const double w0 = a0 < cut ? 0.0 : 231.0 / 500.0, w1 = a1 < cut ? 0.0 : 3.0 / 10.0;
+    const double w2 = a2 < cut ? 0.0 : 27.0 / 500.0, w3 = a3 < cut ? 0.0 : 23.0 / 125.0;
+    num = w0 * c0 + w1 * c1 + w2 * c2 + w3 * c3;
+    den = w0 + w1 + w2 + w3;
+  } else {
+    const double tau = fabs(b0 - b2);
+    const double p01 = e0 * e1;
+    const double tp = quot_near(tau, p01 * e2);
+    const double a0 = pow6(__fma_rn(e1 * e2, tp, 1.0)), a1 = pow6(__fma_rn(e0 * e2, tp, 1.0));
+    const double a2 = pow6(__fma_rn(p01, tp, 1.0));
+    const double cut = ct * (a0 + a1 + a2);
+    const double w0 = a0 < cut ? 0.0 : 11.0 / 20.0, w1 = a1 < cut ? 0.0 : 4.0 / 10.0, w2 = a2 < cut ? 0.0 : 1.0 / 20.0;
+    num = w0 * c0 + w1 * c1 + w2 * c2;
+    den = w0 + w1 + w2;
+  }
+}
+
+// Twice the reconstructed value of one characteristic field less the sum of
+// its flux at the interface's two points: the right reconstruction of
+// f+ = (cf + lam cs)/2 and the left one of f- = (cf - lam cs)/2
+// (shock_capturing.py:257-265) from the differences dcs, dcf of cs and cf
+// between the six points; the halves are left out (eps counts four times).
+template <int CONV>
+__device__ __forceinline__ double recon_gap(const double dcs[5], const double dcf[5], double lam, double eps,
+                                            double ct) {
+  double p[5], m[5];
+#pragma unroll
+  for (int g = 0; g < 5; ++g) {
+    p[g] = __fma_rn(lam, dcs[g], dcf[g]);
+    m[g] = __fma_rn(-lam, dcs[g], dcf[g]);
+  }
+  if constexpr (CONV == CONV_WFILTER) {
+    // the filter flux, which vanishes on equal values, of the variables less their first
+    double fp[6], fm[6], cf[6];
+    fp[0] = fm[0] = cf[0] = 0.0;
+#pragma unroll
+    for (int g = 0; g < 5; ++g) {
+      fp[g + 1] = fp[g] + 0.5 * p[g];
+      fm[g + 1] = fm[g] + 0.5 * m[g];
+      cf[g + 1] = cf[g] + dcf[g];
+    }
+    return 2.0 * weno_filter_flux(fp, fm, cf);
+  } else {
+    double n1, d1, n2, d2;
+    if constexpr (CONV == OSBL_CONV_WENO_Z || CONV == OSBL_CONV_WENO_JS) {
+      constexpr bool Z = CONV == OSBL_CONV_WENO_Z;
+      weno5_gap<Z>(p[0], p[1], p[2], p[3], eps, n1, d1);
+      weno5_gap<Z>(m[4], m[3], m[2], m[1], eps, n2, d2);
+    } else {
+      constexpr bool SIX = CONV == OSBL_CONV_TENO6;
+      teno_gap<SIX, true>(p[0], p[1], p[2], p[3], p[4], eps, ct, n1, d1);
+      teno_gap<SIX, false>(m[4], m[3], m[2], m[1], m[0], eps, ct, n2, d2);
+    }
+    return __fma_rn(1.0 / 6.0, quot_near(n1, d1) - quot_near(n2, d2), -lam * dcs[2]);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // LLF characteristic flux at the interface between window points 2 and 3
-// (shock_capturing.py:357-448).  CF_k = L_k . F is formed from CS_k = L_k . Q
-// through F = u_D Q + p (e_{1+D} + u_D e_last), which holds exactly for the
-// Euler flux vector.
+// (shock_capturing.py:357-448), as the mean of the two points' fluxes plus
+// R times the rest of the reconstructions: R L = 1, so the values that the
+// reconstructions start from (f+ at point 2, f- at point 3) add up to that
+// mean and -lam (cs_3 - cs_2)/2, and only differences between points have to
+// be projected.  They are projected in the frame that moves with the
+// averaged velocity v.u, where the eigenvectors lose most entries: with
+// m' = m - v.u rho and E' = E - v.u.m + rho v.u^2/2,
+//   entropy   rho - (gama-1)/a^2 E'
+//   acoustic  s (E' +- a/(gama-1) m'_D), s = (gama-1)/(sqrt2 rho a)
+//             (1-D: (gama-1)/(2 a^2))
+//   shear     +-m'_c/rho
+// and the flux in that frame is (m_D, u_D m'_c, u_D m'_D + p,
+// u_D E' + p (u_D - v.u_D)).
+//
+// The sweeps are bound by FP64 issue (and the clock that its power allows):
+// against projecting every point on the full rows of L this takes the y
+// sweep of WENO5-Z, Roe, 3-D, from ~1300 to ~980 VALU instructions per cell;
+// 256^3: y 0.785 -> 0.64 ms, z with the RK update 0.83 -> 0.70, x 0.89 ->
+// 0.75 (the step 8.9 -> 7.7 ms; TENO6 at 131x97x75 18 % faster).
 // ---------------------------------------------------------------------------
+template <int ND, int D, int CONV, class W>
+__device__ __forceinline__ void char_fields(const W& w, const Avg<ND>& v, const Phys& ph, double ct,
+                                            double fh[ND + 2]) {
+  constexpr int NV = ND + 2, E = NV - 1;
+  // WENO's indicators are taken 12/13 times
+  constexpr bool WENO = CONV == OSBL_CONV_WENO_Z || CONV == OSBL_CONV_WENO_JS;
+  const double eps = 4.0 * (WENO ? 12.0 / 13.0 * (CONV == OSBL_CONV_WENO_Z ? 1.0e-14 : 1.0e-6) : ph.eps);
+  // the points are re-read per use from a streamed window, and a field's
+  // reconstruction is finished before the next one starts, so that little of
+  // either stays in registers across the fields
+  auto reload = [] {
+    if constexpr (W::STREAM) asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto finish = [&](double& x) {
+    asm volatile("" : "+v"(x));
+    reload();
+  };
+  double l0 = 0.0, lp = 0.0, lm = 0.0;
+#pragma unroll
+  for (int p = 0; p < 6; ++p) {
+    const double ud = w.u(p, D), a = w.a(p);
+    l0 = max_abs(l0, ud);
+    lp = max_abs(lp, ud + a);
+    lm = max_abs(lm, ud - a);
+  }
+  double hu = 0.0;  // v.u^2/2
+#pragma unroll
+  for (int m = 0; m < ND; ++m) hu = __fma_rn(0.5 * v.u[m], v.u[m], hu);
+#pragma unroll
+  for (int m = 0; m < NV; ++m) fh[m] = 0.0;
+  reload();
+  sfor<0, ND>([&](auto cc) {
+    constexpr int c = decltype(cc)::value;
+    if constexpr (c != D) {
+      constexpr double sg = ND == 3 ? (double)eps3(D, 3 - D - c, c) : (D == 0 ? -1.0 : 1.0);
+      const double lc = sg * v.ir, lr = -lc * v.u[c];
+      double dcs[5], dcf[5], ps = 0.0, pf = 0.0;
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        const double cs = __fma_rn(lr, w.q(p, 0), lc * w.q(p, 1 + c));
+        const double cf = w.u(p, D) * cs;
+        if (p > 0) {
+          dcs[p - 1] = cs - ps;
+          dcf[p - 1] = cf - pf;
+        }
+        ps = cs;
+        pf = cf;
+      }
+      double h = 0.5 * sg * v.rho * recon_gap<CONV>(dcs, dcf, l0, eps, ct);
+      finish(h);
+      fh[1 + c] += h;
+      fh[E] = __fma_rn(v.u[c], h, fh[E]);
+    }
+  });
+  // differences of s E', m'_D and of their fluxes
+  const double ia2 = v.ia * v.ia;
+  const double s = ND == 1 ? 0.5 * ph.gm1 * ia2 : v.bta * ph.gm1;
+  const double kap = ND == 1 ? 0.5 * v.ia : v.bta * v.a;  // s a/(gama-1)
+  double dE[5], gE[5], dm[5], gm[5];
+  {
+    double pE = 0.0, pg = 0.0, pm = 0.0, pn = 0.0;
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+      const double r = w.q(p, 0), ud = w.u(p, D), pr = w.pr(p);
+      const double mD = __fma_rn(-v.u[D], r, w.q(p, 1 + D));
+      double En = __fma_rn(hu, r, w.q(p, E));
+#pragma unroll
+      for (int m = 0; m < ND; ++m) En = __fma_rn(-v.u[m], w.q(p, 1 + m), En);
+      const double fD = __fma_rn(ud, mD, pr);
+      const double fE = __fma_rn(pr, ud - v.u[D], ud * En);
+      if (p > 0) {
+        dE[p - 1] = s * (En - pE);
+        gE[p - 1] = s * (fE - pg);
+        dm[p - 1] = mD - pm;
+        gm[p - 1] = fD - pn;
+      }
+      pE = En;
+      pg = fE;
+      pm = mD;
+      pn = fD;
+      if constexpr (W::STREAM) {
+        if (p & 1) {
+          asm volatile("" : "+v"(pE), "+v"(pg), "+v"(pm), "+v"(pn));
+          reload();
+        }
+      }
+    }
+  }
+  reload();
+  double w0, wp, wm;
+  double cs[5], cf[5];
+  {
+    // -(gama-1)/a^2 / s
+    const double ce = ND == 1 ? -2.0 : -1.41421356237309504880 * v.rho * v.ia;
+#pragma unroll
+    for (int g = 0; g < 5; ++g) {
+      cs[g] = __fma_rn(ce, dE[g], w.q(g + 1, 0) - w.q(g, 0));
+      cf[g] = __fma_rn(ce, gE[g], w.q(g + 1, 1 + D) - w.q(g, 1 + D));
+    }
+    w0 = 0.5 * recon_gap<CONV>(cs, cf, l0, eps, ct);
+  }
+  finish(w0);
+  // R's first entries: alpha (1-D: 1)
+  const double ha = ND == 1 ? 0.5 : 0.5 * v.alpha;
+#pragma unroll
+  for (int g = 0; g < 5; ++g) {
+    cs[g] = __fma_rn(kap, dm[g], dE[g]);
+    cf[g] = __fma_rn(kap, gm[g], gE[g]);
+  }
+  wp = ha * recon_gap<CONV>(cs, cf, lp, eps, ct);
+  finish(wp);
+#pragma unroll
+  for (int g = 0; g < 5; ++g) {
+    cs[g] = __fma_rn(-kap, dm[g], dE[g]);
+    cf[g] = __fma_rn(-kap, gm[g], gE[g]);
+  }
+  wm = ha * recon_gap<CONV>(cs, cf, lm, eps, ct);
+  finish(wm);
+  const double S = wp + wm, G = w0 + S, M = v.a * (wp - wm);
+  fh[0] += G;
+#pragma unroll
+  for (int m = 0; m < ND; ++m) fh[1 + m] = __fma_rn(v.u[m], G, fh[1 + m]);
+  fh[1 + D] += M;
+  fh[E] = __fma_rn(hu, G, fh[E]);
+  fh[E] = __fma_rn(v.a * v.a * ph.igm1, S, fh[E]);
+  fh[E] = __fma_rn(v.u[D], M, fh[E]);
+  if constexpr (CONV != CONV_WFILTER) {
+    const double u2 = 0.5 * w.u(2, D), u3 = 0.5 * w.u(3, D), p2 = w.pr(2), p3 = w.pr(3);
+    fh[0] += 0.5 * (w.q(2, 1 + D) + w.q(3, 1 + D));
+#pragma unroll
+    for (int m = 0; m < ND; ++m) {
+      const double f = __fma_rn(u2, w.q(2, 1 + m), u3 * w.q(3, 1 + m));
+      fh[1 + m] += m == D ? __fma_rn(0.5, p2 + p3, f) : f;
+    }
+    fh[E] += __fma_rn(u2, w.q(2, E) + p2, u3 * (w.q(3, E) + p3));
+  }
+}
+
 template <int ND, int D, int CONV, int AVG, bool CACHED = false, class W>
 __device__ __forceinline__ void char_flux_w(const W& w, const Phys& ph, double fh[ND + 2], double ct,
                                             const RoeF& rf = RoeF{}) {
-  constexpr int NV = ND + 2;
   Avg<ND> v;
   {
     Pt<ND> L, R;
@@ -847,53 +1088,7 @@ __device__ __forceinline__ void char_flux_w(const W& w, const Phys& ph, double f
       interface_state<ND, AVG>(v, L, R, ph);
     }
   }
-#pragma unroll
-  for (int m = 0; m < NV; ++m) fh[m] = 0.0;
-  sfor<0, NV>([&](auto kc) {
-    constexpr int K = decltype(kc)::value;
-    constexpr unsigned LM = lmask<ND, D, K>();
-    constexpr unsigned RM = rmask<ND, D, K>();
-    double l[NV];
-    lrow<ND, D, K>(v, ph, l);
-    // the split fluxes 1/2 (CF +- lam CS) are formed from the half row L_k/2:
-    // halving is exact, so CS/2 and CF/2 come out exactly and the two
-    // products by 1/2 per point disappear
-#pragma unroll
-    for (int m = 0; m < NV; ++m) l[m] *= 0.5;
-    double lam = 0.0;
-#pragma unroll
-    for (int p = 0; p < 6; ++p) lam = fmax(lam, abs_lambda_ua<ND, D, K>(w.u(p, D), w.a(p)));
-    // coefficient of p in L_k . F - u_D L_k . Q
-    double fp[6], fm[6];
-    [[maybe_unused]] double cfa[6];
-#pragma unroll
-    for (int p = 0; p < 6; ++p) {
-      double hcs = 0.0;
-      sfor<0, NV>([&](auto mc) {
-        constexpr int M = decltype(mc)::value;
-        if constexpr ((LM >> M) & 1u) hcs += l[M] * w.q(p, M);
-      });
-      const double ud = w.u(p, D);
-      double hlp = 0.0;
-      if constexpr ((LM >> (1 + D)) & 1u) hlp = l[1 + D];
-      if constexpr ((LM >> (NV - 1)) & 1u) hlp += ud * l[NV - 1];
-      const double hcf = ud * hcs + w.pr(p) * hlp;
-      fp[p] = __fma_rn(lam, hcs, hcf);
-      fm[p] = __fma_rn(-lam, hcs, hcf);
-      if constexpr (CONV == CONV_WFILTER) cfa[p] = 2.0 * hcf;
-    }
-    double rc;
-    if constexpr (CONV == CONV_WFILTER) rc = weno_filter_flux(fp, fm, cfa);
-    else rc = recon_pair<CONV, W::STREAM>(fp, fm, ph.eps, ct);
-    double r[NV];
-    rcol<ND, D, K>(v, ph, r);
-    sfor<0, NV>([&](auto mc) {
-      constexpr int M = decltype(mc)::value;
-      if constexpr ((RM >> M) & 1u) fh[M] += r[M] * rc;
-    });
-    // LDS window: the next field reloads its points (nothing stays live across fields)
-    if constexpr (W::STREAM) asm volatile("" ::: "memory");
-  });
+  char_fields<ND, D, CONV>(w, v, ph, ct, fh);
 }
 
 template <int ND, int D, int CONV, int AVG, bool CACHED = false>

@@ -198,10 +198,10 @@ __global__ void __launch_bounds__(256) k_char_sweep(const double* __restrict__ Q
     if (f >= c0) {
       const int x = off + 2 * st;
       // a stretched direction scales the flux difference by D_dd (opensblifunctions.py:607-616)
-      const double gm = met ? met[f] : 1.0;
+      const double gi = met ? met[f] * inv : inv;
 #pragma unroll
       for (int m = 0; m < NV; ++m) {
-        const double v = met ? -(gm * ((fh[m] - fprev[m]) * inv)) : -(fh[m] - fprev[m]) * inv;
+        const double v = (fprev[m] - fh[m]) * gi;
         if constexpr (RKM == 0) {
           const double r = (EARLY ? rin[m] : R[m * g.fs + x]) + v;
           const double qo = rk.first ? w[2].q[m] : (EARLY ? qoin[m] : rk.Qo[m * g.fs + x]);
@@ -251,11 +251,13 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
   constexpr int NV = ND + 2;
   constexpr bool ROE = AVG == OSBL_AVG_ROE;
   constexpr int NF = NV + ND + 2 + (ROE ? 2 : 0);  // q, u, p, a (, sqrt(rho), sqrt(rho) H)
-  __shared__ double sh[XW][NF][XP];
+  constexpr int NS = NF | 1;                       // odd stride: no bank conflicts
+  __shared__ double sh[XW][XP][NS];
+  __shared__ double edge[XW][2][NV];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int row = blockIdx.x * XW + wv;
   if (row >= nrows) return;  // whole waves only: no block-wide barrier below
-  double (*S)[XP] = sh[wv];
+  double (*S)[NS] = sh[wv];
   const int base = g.idx(0, row % g.n[1], row / g.n[1]);
   const int N = g.n[0];
   const double inv = ph.inv_delta[0];
@@ -263,24 +265,24 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
     Pt<ND> p;
     load_pt<ND>(p, Q, g.fs, base + x, ph);
 #pragma unroll
-    for (int m = 0; m < NV; ++m) S[m][slot] = p.q[m];
+    for (int m = 0; m < NV; ++m) S[slot][m] = p.q[m];
 #pragma unroll
-    for (int m = 0; m < ND; ++m) S[NV + m][slot] = p.u[m];
-    S[NV + ND][slot] = p.p;
-    S[NV + ND + 1][slot] = p.a;
-    if constexpr (ROE) roe_factors<ND>(p, S[NV + ND + 2][slot], S[NV + ND + 3][slot]);
+    for (int m = 0; m < ND; ++m) S[slot][NV + m] = p.u[m];
+    S[slot][NV + ND] = p.p;
+    S[slot][NV + ND + 1] = p.a;
+    if constexpr (ROE) roe_factors<ND>(p, S[slot][NV + ND + 2], S[slot][NV + ND + 3]);
   };
   // flux at interface x0 + lane + 1/2 (points x0+lane-2 .. x0+lane+3 = slots lane .. lane+5)
   const int xmax = N + g.h[0] - 1;  // last stored point of the line
   auto flux = [&](double fh[NV], int xi) {
-    const LdsWindow<ND> w{&S[0][lane], XP};
+    const LdsPoints<ND, NS> w{S[lane]};
     const double ct = theta ? adaptive_ct(theta[base + min(xi, xmax)], ph) : ph.teno_ct;
     [[maybe_unused]] RoeF rf{};
     if constexpr (ROE) {
-      rf.sL = S[NV + ND + 2][lane + 2];
-      rf.hL = S[NV + ND + 3][lane + 2];
-      rf.sR = S[NV + ND + 2][lane + 3];
-      rf.hR = S[NV + ND + 3][lane + 3];
+      rf.sL = S[lane + 2][NV + ND + 2];
+      rf.hL = S[lane + 2][NV + ND + 3];
+      rf.sR = S[lane + 3][NV + ND + 2];
+      rf.hR = S[lane + 3][NV + ND + 3];
     }
     char_flux_w<ND, 0, CONV, AVG, true>(w, ph, fh, ct, rf);
   };
@@ -295,10 +297,10 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
   auto emit = [&](int x, const double* r) {
-    const double gm = met ? met[x] : 1.0;
+    const double gi = met ? -met[x] * inv : -inv;
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
-      const double v = met ? -(gm * (r[m] * inv)) : -r[m] * inv;
+      const double v = r[m] * gi;
       if constexpr (ACC) st_once(ld_once(&R[m * g.fs + base + x], ph.nt) + v, &R[m * g.fs + base + x], ph.nt);
       else st_once(v, &R[m * g.fs + base + x], ph.nt);
     }
@@ -319,12 +321,12 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
       for (int m = 0; m < NV; ++m) p.q[m] = q[m];
       finish_pt<ND>(p, ph);
 #pragma unroll
-      for (int m = 0; m < NV; ++m) S[m][slot] = p.q[m];
+      for (int m = 0; m < NV; ++m) S[slot][m] = p.q[m];
 #pragma unroll
-      for (int m = 0; m < ND; ++m) S[NV + m][slot] = p.u[m];
-      S[NV + ND][slot] = p.p;
-      S[NV + ND + 1][slot] = p.a;
-      if constexpr (ROE) roe_factors<ND>(p, S[NV + ND + 2][slot], S[NV + ND + 3][slot]);
+      for (int m = 0; m < ND; ++m) S[slot][NV + m] = p.u[m];
+      S[slot][NV + ND] = p.p;
+      S[slot][NV + ND + 1] = p.a;
+      if constexpr (ROE) roe_factors<ND>(p, S[slot][NV + ND + 2], S[slot][NV + ND + 3]);
     };
     auto wave_sync = [&] {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -332,13 +334,13 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
     auto flux_at = [&](double fh[NV]) {
-      const LdsWindow<ND> w{&S[0][lane], XP};
+      const LdsPoints<ND, NS> w{S[lane]};
       [[maybe_unused]] RoeF rf{};
       if constexpr (ROE) {
-        rf.sL = S[NV + ND + 2][lane + 2];
-        rf.hL = S[NV + ND + 3][lane + 2];
-        rf.sR = S[NV + ND + 2][lane + 3];
-        rf.hR = S[NV + ND + 3][lane + 3];
+        rf.sL = S[lane + 2][NV + ND + 2];
+        rf.hL = S[lane + 2][NV + ND + 3];
+        rf.sR = S[lane + 3][NV + ND + 2];
+        rf.hR = S[lane + 3][NV + ND + 3];
       }
       char_flux_w<ND, 0, CONV, AVG, true>(w, ph, fh, ph.teno_ct, rf);
     };
@@ -350,12 +352,6 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
       stage_q(lane, q0);
     }
     fetch_q<ND>(nq, Q, g.fs, base + clampx(x0s - 2 + lane));
-    double prev[NV], first[NV];
-#pragma unroll
-    for (int m = 0; m < NV; ++m) {
-      prev[m] = 0.0;
-      first[m] = 0.0;
-    }
     for (int x0 = x0s; x0 - 5 <= N - 1; x0 += 64) {
       stage_q(5 + lane, nq);
       wave_sync();
@@ -364,29 +360,29 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
       double fh[NV];
       const int I = x0 - 5 + lane;
       flux_at(fh);
-      double left[NV];
+      double r[NV];
 #pragma unroll
       for (int m = 0; m < NV; ++m) {
         const double up = __shfl_up(fh[m], 1);
-        left[m] = lane == 0 ? prev[m] : up;
+        r[m] = fh[m] - (lane == 0 ? edge[wv][0][m] : up);
       }
-      const int last = min(63, N - 1 - (x0 - 5));  // lane holding the line's last interface of the chunk
+      // the line's first and last flux of the chunk wait in LDS (registers are what bounds the kernel)
+      const int last = min(63, N - 1 - (x0 - 5));
+      if (lane == 0 && x0 == x0s) {
 #pragma unroll
-      for (int m = 0; m < NV; ++m) {
-        if (x0 == x0s) first[m] = __shfl(fh[m], 0);
-        prev[m] = __shfl(fh[m], last);
+        for (int m = 0; m < NV; ++m) edge[wv][1][m] = fh[m];
       }
-      if (I >= 0 && I < N && !(periodic && I == 0)) {
-        double r[NV];
+      wave_sync();
+      if (lane == last) {
 #pragma unroll
-        for (int m = 0; m < NV; ++m) r[m] = fh[m] - left[m];
-        emit(I, r);
+        for (int m = 0; m < NV; ++m) edge[wv][0][m] = fh[m];
       }
+      if (I >= 0 && I < N && !(periodic && I == 0)) emit(I, r);
       // slots 64..68 become slots 0..4 of the next chunk
       wave_sync();
       if (lane < 5) {
 #pragma unroll
-        for (int e = 0; e < NF; ++e) S[e][lane] = S[e][64 + lane];
+        for (int e = 0; e < NF; ++e) S[lane][e] = S[64 + lane][e];
       }
       wave_sync();
     }
@@ -394,7 +390,7 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
       // the line's last interface flux is the flux left of cell 0
       double r[NV];
 #pragma unroll
-      for (int m = 0; m < NV; ++m) r[m] = first[m] - prev[m];
+      for (int m = 0; m < NV; ++m) r[m] = edge[wv][1][m] - edge[wv][0][m];
       emit(0, r);
     }
   } else {

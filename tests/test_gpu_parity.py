@@ -45,6 +45,24 @@ def test_rhs_generic3d(conv, oracle):
     check_parity(g.rhs(), r.rhs(), f"rhs generic {conv}")
 
 
+@pytest.mark.parametrize("averaging", ["roe", "simple"])
+@pytest.mark.parametrize("rho_unit,u_unit", [(1e-24, 1e6), (1e3, 1e4)])
+@pytest.mark.parametrize("conv", ["weno_z", "weno_js", "teno6", "teno5"])
+def test_rhs_other_units(conv, rho_unit, u_unit, averaging, oracle):
+    """The residual of the same kind of state in other units: the weights'
+    products of smoothness indicators then span most of the exponent range,
+    and the projections' scalings differ by as much."""
+    from opensbli_amd.problems import taylor_green
+    _say(f"case rhs conv={conv} units {rho_unit} {u_unit} {averaging}")
+    problem, _ = taylor_green(24, conv=conv, viscous="none", averaging=averaging)
+    q0 = generic_state(24, 3, seed=2)
+    q0 = q0 * rho_unit
+    q0[1:4] *= u_unit
+    q0[4] *= u_unit ** 2
+    g, r = _pair(problem, q0, oracle)
+    check_parity(g.rhs(), r.rhs(), f"rhs {conv} in other units")
+
+
 @pytest.mark.parametrize("conv", ["central_skew", "central_cons", "weno_z", "weno_js", "teno6", "teno5"])
 def test_rhs_tgv3d(conv, oracle):
     """The residual at the Taylor-Green vortex's initial state.  Its density
