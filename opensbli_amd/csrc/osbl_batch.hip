@@ -5,12 +5,11 @@
 // Storage: each variable is one array holding every instance's points back
 // to back, each instance with H halo points on both sides.
 //
-// Two executions, same arithmetic as the single-block path (char_flux<1,...>,
-// the same residual and RK formulas), so results are bitwise identical to
-// running every instance alone:
+// Two executions, same arithmetic (line_segment, osbl_line.h), so the results
+// are bitwise identical:
 //  * persistent: one launch; workgroup b integrates instance order[b]
-//    through all its steps and stages, with block barriers between phases.
-//    Threads per workgroup come from a per-size table the autotuner fills.
+//    through all its steps and stages, with a workgroup barrier per stage.
+//    Up to 16 waves share a line; the autotuner can set the threads by size.
 //  * staged: one launch per RK stage covering every instance still running;
 //    the stages of a chunk of steps are captured once into a hipGraph (two,
 //    when a chunk ends on the other ping-pong buffer) and replayed for every
@@ -22,6 +21,7 @@
 #include <vector>
 
 #include "osbl_kernels.h"
+#include "osbl_line.h"
 
 using namespace osbl;
 
@@ -38,59 +38,168 @@ struct Inst {
   double inv_dx;
 };
 
-// one RK stage of the sweep + update for the cells [c0, c1) of one instance
-template <int CONV, int AVG, int MODE>
-__device__ __forceinline__ void stage_segment(const double* __restrict__ Q, double* __restrict__ Qo,
-                                              double* __restrict__ Qn, long long fs, const Inst& in, int c0, int c1,
-                                              const Phys& ph, double cA, double cB, bool first) {
-  constexpr int ND = 1, NV = 3;
-  if (c0 >= c1) return;
-  int off = in.off + c0 - 3;
-  Pt<ND> w[6];
+struct Coeffs {
+  double A[5], B[5];
+  int ns;
+};
+
+// read / write access of line_segment to a line in global memory
+struct GlobalLine {
+  const double* Q;
+  double* Qn;
+  double* Qo;
+  long long fs;
+  int off;
+  __device__ __forceinline__ void ld(int x, double (&q)[3]) const {
 #pragma unroll
-  for (int p = 0; p < 5; ++p) load_pt<ND>(w[p], Q, fs, off + p, ph);
-  // the next point's raw values are fetched one iteration ahead
-  double nxt[NV];
-  fetch_q<ND>(nxt, Q, fs, off + 5);
-  double fprev[NV];
-  for (int f = c0 - 1; f < c1; ++f) {
-#pragma unroll
-    for (int m = 0; m < NV; ++m) w[5].q[m] = nxt[m];
-    finish_pt<ND>(w[5], ph);
-    if (f + 1 < c1) fetch_q<ND>(nxt, Q, fs, off + 6);
-    double fh[NV];
-    // the RK register of this iteration's cell is fetched before the flux so
-    // that the load overlaps its arithmetic; the cell's state is window point 2
-    double qoin[NV];
-#pragma unroll
-    for (int m = 0; m < NV; ++m) qoin[m] = 0.0;
-    if (f >= c0 && !(MODE == 0 && first)) {
-#pragma unroll
-      for (int m = 0; m < NV; ++m) qoin[m] = Qo[m * fs + off + 2];
-    }
-    char_flux<ND, 0, CONV, AVG>(w, ph, fh, ph.teno_ct);
-    if (f >= c0) {
-      const int x = off + 2;
-#pragma unroll
-      for (int m = 0; m < NV; ++m) {
-        const double r = -(fh[m] - fprev[m]) * in.inv_dx;
-        if constexpr (MODE == 0) {
-          const double qo = first ? w[2].q[m] : qoin[m];
-          Qn[m * fs + x] = qo + in.dt * cA * r;
-          Qo[m * fs + x] = qo + in.dt * cB * r;
-        } else {
-          const double tmp = (cA == 0.0 ? 0.0 : cA * qoin[m]) + in.dt * r;
-          Qo[m * fs + x] = tmp;
-          Qn[m * fs + x] = w[2].q[m] + cB * tmp;
-        }
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < NV; ++m) fprev[m] = fh[m];
-#pragma unroll
-    for (int p = 0; p < 5; ++p) w[p] = w[p + 1];
-    ++off;
+    for (int m = 0; m < 3; ++m) q[m] = Q[m * fs + off + x];
   }
+  __device__ __forceinline__ void rk_in(int x, double (&q)[3]) const {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) q[m] = Qo[m * fs + off + x];
+  }
+  __device__ __forceinline__ void put(int x, const double (&qn)[3], const double (&qo)[3]) const {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      Qn[m * fs + off + x] = qn[m];
+      Qo[m * fs + off + x] = qo[m];
+    }
+  }
+};
+
+template <int CONV, int AVG, int MODE>
+__device__ __forceinline__ void line_segment_global(double (*S)[LINE_NF], int lane, const Inst& in, int s0, int s1,
+                                                    const Phys& ph, const Coeffs& rk, int s, const GlobalLine& g) {
+  line_segment<CONV, AVG, MODE>(
+      S, lane, in.n, s0, s1, in.dt, in.inv_dx, ph, rk.A[s], rk.B[s], s == 0,
+      [&](int x, double (&q)[3]) { g.ld(x, q); }, [&](int x, double (&q)[3]) { g.rk_in(x, q); },
+      [&](int x, const double (&qn)[3], const double (&qo)[3]) { g.put(x, qn, qo); });
+}
+
+// LDS of a workgroup of W waves: the waves' staged points, then (for lines
+// that fit) two copies of the state of up to LINE_CELLS * W cells
+__host__ __device__ constexpr size_t line_lds(int W, bool state) {
+  return sizeof(double) * ((size_t)W * LINE_PTS * LINE_NF + (state ? (size_t)W * 6 * LINE_CELLS : 0));
+}
+
+// One line through nsteps iterations by one workgroup, a barrier per stage.
+//
+// A line of at most LINE_CELLS cells per wave stays on the chip: its state in
+// two LDS copies that alternate between the stages, its RK register in the
+// registers of the lanes that own the cells.  What bounds it is the latency
+// of one wave's chunk; a longer line is split into one contiguous part per
+// wave, read from and written to L2, and bound by the CU's FP64 issue.
+template <int CONV, int AVG, int MODE>
+__device__ __forceinline__ void line_run(const Inst& in, int W, double* sm, double* QA, double* QB, double* Qo,
+                                         long long fs, const Phys& ph, const Coeffs& rk) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), T = blockDim.x;
+  double (*S)[LINE_NF] = reinterpret_cast<double (*)[LINE_NF]>(sm + (size_t)wv * LINE_PTS * LINE_NF);
+  // the final state: boundary points and halos filled
+  auto leave = [&](auto&& value) {
+    for (int i = (int)threadIdx.x - BH; i < in.n + BH; i += T) {
+      const int x = max(1, min(i, in.n - 2));
+      double v[3];
+      value(x, v);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) QA[m * fs + in.off + i] = v[m];
+    }
+  };
+  if (in.n <= LINE_CELLS * W) {
+    double* L = sm + (size_t)(T >> 6) * LINE_PTS * LINE_NF;
+    const int ls = LINE_CELLS * (T >> 6);  // doubles per variable
+    for (int i = threadIdx.x; i < in.n; i += T)
+#pragma unroll
+      for (int m = 0; m < 3; ++m) L[m * ls + i] = QA[m * fs + in.off + i];
+    __syncthreads();
+    const int s0 = min(wv * LINE_CELLS, in.n), s1 = min(s0 + LINE_CELLS, in.n);
+    double ro[3] = {0.0, 0.0, 0.0};
+    int cur = 0;
+    for (int step = 0; step < in.nsteps; ++step)
+      for (int s = 0; s < rk.ns; ++s) {
+        const double* Lq = L + cur * 3 * ls;
+        double* Ln = L + (1 - cur) * 3 * ls;
+        if (wv < W)
+          line_segment<CONV, AVG, MODE>(
+              S, lane, in.n, s0, s1, in.dt, in.inv_dx, ph, rk.A[s], rk.B[s], s == 0,
+              [&](int x, double (&q)[3]) {
+#pragma unroll
+                for (int m = 0; m < 3; ++m) q[m] = Lq[m * ls + x];
+              },
+              [&](int, double (&q)[3]) {
+#pragma unroll
+                for (int m = 0; m < 3; ++m) q[m] = ro[m];
+              },
+              [&](int x, const double (&qn)[3], const double (&qo)[3]) {
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                  Ln[m * ls + x] = qn[m];
+                  ro[m] = qo[m];
+                }
+              });
+        __syncthreads();
+        cur ^= 1;
+      }
+    const double* Lq = L + cur * 3 * ls;
+    leave([&](int x, double (&v)[3]) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) v[m] = Lq[m * ls + x];
+    });
+    return;
+  }
+  const int len = (in.n + W - 1) / W;
+  const int s0 = min(wv * len, in.n), s1 = wv < W ? min(s0 + len, in.n) : s0;
+  double* Q = QA;
+  double* Qn = QB;
+  for (int step = 0; step < in.nsteps; ++step)
+    for (int s = 0; s < rk.ns; ++s) {
+      line_segment_global<CONV, AVG, MODE>(S, lane, in, s0, s1, ph, rk, s, GlobalLine{Q, Qn, Qo, fs, in.off});
+      __syncthreads();
+      double* t = Q;
+      Q = Qn;
+      Qn = t;
+    }
+  if (Q != QA) {
+    leave([&](int x, double (&v)[3]) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) v[m] = Q[m * fs + in.off + x];
+    });
+  } else {
+    // the ends only: the rest is in place
+    const int t = threadIdx.x;
+    if (t < 2 * (BH + 1)) {
+      const int i = t <= BH ? t - BH : in.n - 1 + (t - BH - 1);
+      const int x = t <= BH ? 1 : in.n - 2;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) QA[m * fs + in.off + i] = QA[m * fs + in.off + x];
+    }
+  }
+}
+
+template <int CONV, int AVG, int MODE>
+__global__ void __launch_bounds__(1024) k_batch_persistent(const Inst* __restrict__ insts,
+                                                           const int* __restrict__ order, double* __restrict__ QA,
+                                                           double* __restrict__ QB, double* __restrict__ Qo,
+                                                           long long fs, Phys ph, Coeffs rk) {
+  extern __shared__ double sm[];
+  const Inst in = insts[order[blockIdx.x]];
+  line_run<CONV, AVG, MODE>(in, in.threads >> 6, sm, QA, QB, Qo, fs, ph, rk);
+}
+
+// A single 1-D block: the whole run of a line that stays on one chip (one
+// workgroup), or one stage of a longer one, LINE_CELLS cells per wave.
+template <int CONV, int AVG, int MODE>
+__global__ void __launch_bounds__(1024) k_line_run(Inst in, double* __restrict__ Q, double* __restrict__ Q2,
+                                                   double* __restrict__ Qo, long long fs, Phys ph, Coeffs rk) {
+  extern __shared__ double sm[];
+  line_run<CONV, AVG, MODE>(in, blockDim.x >> 6, sm, Q, Q2, Qo, fs, ph, rk);
+}
+template <int CONV, int AVG, int MODE>
+__global__ void __launch_bounds__(64) k_line_stage(Inst in, const double* __restrict__ Q, double* __restrict__ Qo,
+                                                   double* __restrict__ Qn, long long fs, Phys ph, Coeffs rk, int s) {
+  __shared__ double sm[LINE_PTS][LINE_NF];
+  const int c0 = blockIdx.x * LINE_CELLS;
+  line_segment_global<CONV, AVG, MODE>(sm, threadIdx.x, in, c0, min(c0 + LINE_CELLS, in.n), ph, rk, s,
+                                       GlobalLine{Q, Qn, Qo, fs, in.off});
 }
 
 // zeroth-order extrapolation of both ends (extrapolation.py:29-58) by lanes 0, 1
@@ -105,62 +214,29 @@ __device__ __forceinline__ void extrap_ends(double* __restrict__ Q, long long fs
   }
 }
 
-struct Coeffs {
-  double A[5], B[5];
-  int ns;
-};
-
-template <int CONV, int AVG, int MODE>
-__global__ void __launch_bounds__(512) k_batch_persistent(const Inst* __restrict__ insts, const int* __restrict__ order,
-                                                            double* __restrict__ QA, double* __restrict__ QB,
-                                                            double* __restrict__ Qo, long long fs, Phys ph, Coeffs rk) {
-  const Inst in = insts[order[blockIdx.x]];
-  const int T = in.threads;
-  const int t = threadIdx.x;
-  double* Q = QA;
-  double* Qn = QB;
-  const int seg = (in.n + T - 1) / T;
-  const int c0 = min(t * seg, in.n), c1 = min(c0 + seg, in.n);
-  const bool act = t < T;
-  for (int step = 0; step < in.nsteps; ++step) {
-    for (int s = 0; s < rk.ns; ++s) {
-      if (act) extrap_ends(Q, fs, in, t);
-      __syncthreads();
-      if (act) stage_segment<CONV, AVG, MODE>(Q, Qo, Qn, fs, in, c0, c1, ph, rk.A[s], rk.B[s], s == 0);
-      __syncthreads();
-      double* tmp = Q;
-      Q = Qn;
-      Qn = tmp;
-    }
-  }
-  // leave the final state of every instance in QA with filled halos
-  if ((in.nsteps * rk.ns) & 1) {
-    for (int i = t - BH; i < in.n + BH; i += blockDim.x)
-      for (int m = 0; m < 3; ++m) QA[m * fs + in.off + i] = Q[m * fs + in.off + i];
-    __syncthreads();
-  }
-  if (t < 2) extrap_ends(QA, fs, in, t);
-}
-
 // Staged mode.  The step a launch belongs to is *step0 + rel: step0 is a
 // device counter the chunk's last kernel advances, so one captured chunk of
 // steps serves every chunk of the run.
 //
-// one thread per (instance, segment); inactive instances skip
+// one wave per (instance, chunk of LINE_CELLS cells); finished instances skip
+constexpr int SW = 4;  // waves per workgroup
 template <int CONV, int AVG, int MODE>
-__global__ void __launch_bounds__(256) k_batch_stage(const Inst* __restrict__ insts, const int* __restrict__ seg_inst,
-                                                      const int* __restrict__ seg_c0, int nseg, const double* __restrict__ Q,
-                                                      double* __restrict__ Qo, double* __restrict__ Qn, long long fs,
-                                                      Phys ph, double cA, double cB, int first,
-                                                      const int* __restrict__ step0, int rel, int seglen) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nseg) return;
+__global__ void __launch_bounds__(64 * SW) k_batch_stage(const Inst* __restrict__ insts,
+                                                         const int* __restrict__ seg_inst,
+                                                         const int* __restrict__ seg_c0, int nseg,
+                                                         const double* __restrict__ Q, double* __restrict__ Qo,
+                                                         double* __restrict__ Qn, long long fs, Phys ph, Coeffs rk,
+                                                         int s, const int* __restrict__ step0, int rel) {
+  __shared__ double sm[SW][LINE_PTS][LINE_NF];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = blockIdx.x * SW + wv;
+  if (t >= nseg) return;  // whole waves only: no workgroup-wide barrier below
   const Inst in = insts[seg_inst[t]];
   const int step = *step0 + rel;
   if (step >= in.nsteps) return;
   const int c0 = seg_c0[t];
-  const int c1 = min(c0 + seglen, in.n);
-  stage_segment<CONV, AVG, MODE>(Q, Qo, Qn, fs, in, c0, c1, ph, cA, cB, first != 0);
+  line_segment_global<CONV, AVG, MODE>(sm[wv], lane, in, c0, min(c0 + LINE_CELLS, in.n), ph, rk, s,
+                                       GlobalLine{Q, Qn, Qo, fs, in.off});
 }
 
 __global__ void __launch_bounds__(256) k_batch_bc(const Inst* __restrict__ insts, int ninst, double* __restrict__ Q,
@@ -219,7 +295,6 @@ struct osbl_batch {
   double* stage_buf = nullptr;
   hipStream_t stream = nullptr;
   // staged mode
-  int seglen = 16;
   int* d_seg_inst = nullptr;
   int* d_seg_c0 = nullptr;
   int nseg = 0;
@@ -230,9 +305,8 @@ struct osbl_batch {
   int* d_step0 = nullptr;
   // captured chunk of graph_steps steps, by the buffer it starts from (0: QA, 1: QB)
   hipGraphExec_t chunk[2] = {nullptr, nullptr};
-  // per-size thread table: threads for n <= bucket_n[k]
-  std::vector<int> bucket_n{256, 512, 1024, 2048, 4096, 1 << 30};
-  std::vector<int> bucket_t{64, 64, 128, 256, 256, 512};
+  // per-size thread table: threads for n <= bucket_n[k]; empty: a wave per LINE_CELLS cells
+  std::vector<int> bucket_n, bucket_t;
   double last_ms = 0.0;
 };
 
@@ -241,7 +315,7 @@ namespace {
 int pick_threads(const osbl_batch* b, int n) {
   for (size_t k = 0; k < b->bucket_n.size(); ++k)
     if (n <= b->bucket_n[k]) return b->bucket_t[k];
-  return b->bucket_t.back();
+  return 64 * std::min(16, (n + LINE_CELLS - 1) / LINE_CELLS);
 }
 
 int upload_instances(osbl_batch* b) {
@@ -251,28 +325,32 @@ int upload_instances(osbl_batch* b) {
 }
 
 template <int CONV, int AVG>
-void launch_persistent_t(osbl_batch* b) {
+int launch_persistent_t(osbl_batch* b) {
   int maxT = 64;
-  for (auto& in : b->h_inst) maxT = std::max(maxT, in.threads);
-  if (b->mode_rk == 0)
-    k_batch_persistent<CONV, AVG, 0><<<b->ninst, maxT, 0, b->stream>>>(b->d_inst, b->d_order, b->QA, b->QB, b->Qo,
-                                                                       b->fs, b->ph, b->rk);
-  else
-    k_batch_persistent<CONV, AVG, 1><<<b->ninst, maxT, 0, b->stream>>>(b->d_inst, b->d_order, b->QA, b->QB, b->Qo,
-                                                                       b->fs, b->ph, b->rk);
+  bool state = false;
+  for (auto& in : b->h_inst) {
+    maxT = std::max(maxT, in.threads);
+    state |= in.n <= LINE_CELLS * (in.threads >> 6);
+  }
+  const size_t lds = line_lds(maxT >> 6, state);
+  auto go = [&](auto k) -> int {
+    BCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k<<<b->ninst, maxT, lds, b->stream>>>(b->d_inst, b->d_order, b->QA, b->QB, b->Qo, b->fs, b->ph, b->rk);
+    BCHK(hipGetLastError());
+    return OSBL_OK;
+  };
+  return b->mode_rk == 0 ? go(&k_batch_persistent<CONV, AVG, 0>) : go(&k_batch_persistent<CONV, AVG, 1>);
 }
 
 template <int CONV, int AVG>
 void launch_stage_t(osbl_batch* b, const double* Q, double* Qn, int s, int rel) {
-  const unsigned blocks = (unsigned)((b->nseg + 255) / 256);
+  const unsigned blocks = (unsigned)((b->nseg + SW - 1) / SW);
   if (b->mode_rk == 0)
-    k_batch_stage<CONV, AVG, 0><<<blocks, 256, 0, b->stream>>>(b->d_inst, b->d_seg_inst, b->d_seg_c0, b->nseg, Q, b->Qo,
-                                                               Qn, b->fs, b->ph, b->rk.A[s], b->rk.B[s], s == 0,
-                                                               b->d_step0, rel, b->seglen);
+    k_batch_stage<CONV, AVG, 0><<<blocks, 64 * SW, 0, b->stream>>>(b->d_inst, b->d_seg_inst, b->d_seg_c0, b->nseg, Q,
+                                                                   b->Qo, Qn, b->fs, b->ph, b->rk, s, b->d_step0, rel);
   else
-    k_batch_stage<CONV, AVG, 1><<<blocks, 256, 0, b->stream>>>(b->d_inst, b->d_seg_inst, b->d_seg_c0, b->nseg, Q, b->Qo,
-                                                               Qn, b->fs, b->ph, b->rk.A[s], b->rk.B[s], s == 0,
-                                                               b->d_step0, rel, b->seglen);
+    k_batch_stage<CONV, AVG, 1><<<blocks, 64 * SW, 0, b->stream>>>(b->d_inst, b->d_seg_inst, b->d_seg_c0, b->nseg, Q,
+                                                                   b->Qo, Qn, b->fs, b->ph, b->rk, s, b->d_step0, rel);
 }
 
 template <class F>
@@ -291,11 +369,11 @@ void dispatch(int conv, int avg, F&& f) {
 }
 
 int run_persistent(osbl_batch* b) {
+  int rc = OSBL_OK;
   dispatch(b->base.conv, b->base.averaging, [&](auto c, auto a) {
-    launch_persistent_t<decltype(c)::value, decltype(a)::value>(b);
+    rc = launch_persistent_t<decltype(c)::value, decltype(a)::value>(b);
   });
-  BCHK(hipGetLastError());
-  return OSBL_OK;
+  return rc;
 }
 
 void drop_chunks(osbl_batch* b) {
@@ -308,7 +386,6 @@ void drop_chunks(osbl_batch* b) {
 
 // capture one chunk of graph_steps steps starting from buffer `start`
 int capture_chunk(osbl_batch* b, int start) {
-  const unsigned bcb = (unsigned)((2 * b->ninst + 255) / 256);
   const unsigned cpb = (unsigned)((b->npts + 255) / 256);
   double* Q = start ? b->QB : b->QA;
   double* Qn = start ? b->QA : b->QB;
@@ -316,7 +393,6 @@ int capture_chunk(osbl_batch* b, int start) {
   BCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   for (int rel = 0; rel < b->graph_steps; ++rel) {
     for (int s = 0; s < b->rk.ns; ++s) {
-      k_batch_bc<<<bcb, 256, 0, b->stream>>>(b->d_inst, b->ninst, Q, b->fs, b->d_step0, rel);
       dispatch(b->base.conv, b->base.averaging, [&](auto c, auto a) {
         launch_stage_t<decltype(c)::value, decltype(a)::value>(b, Q, Qn, s, rel);
       });
@@ -361,6 +437,46 @@ int run_staged(osbl_batch* b) {
 }
 
 }  // namespace
+
+namespace osbl {
+
+int launch_line_run(int conv, int avg, int mode, double* Q, double* Q2, double* Qo, const Grid& g, const Phys& ph,
+                    const double* A, const double* B, int ns, int nsteps, hipStream_t st) {
+  const int W = (g.n[0] + LINE_CELLS - 1) / LINE_CELLS;
+  const Inst in{g.n[0], g.idx(0, 0, 0), nsteps, 64 * W, ph.dt, ph.inv_delta[0]};
+  Coeffs rk{};
+  rk.ns = ns;
+  for (int i = 0; i < ns; ++i) { rk.A[i] = A[i]; rk.B[i] = B[i]; }
+  const size_t lds = line_lds(W, true);
+  int rc = OSBL_OK;
+  auto go = [&](auto k) -> int {
+    BCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k<<<1, 64 * W, lds, st>>>(in, Q, Q2, Qo, g.fs, ph, rk);
+    BCHK(hipGetLastError());
+    return OSBL_OK;
+  };
+  dispatch(conv, avg, [&](auto c, auto a) {
+    constexpr int C = decltype(c)::value, V = decltype(a)::value;
+    rc = mode == 0 ? go(&k_line_run<C, V, 0>) : go(&k_line_run<C, V, 1>);
+  });
+  return rc;
+}
+
+void launch_line_stage(int conv, int avg, int mode, const double* Q, double* Qo, double* Qn, const Grid& g,
+                       const Phys& ph, const double* A, const double* B, int ns, int s, hipStream_t st) {
+  const Inst in{g.n[0], g.idx(0, 0, 0), 1, 64, ph.dt, ph.inv_delta[0]};
+  Coeffs rk{};
+  rk.ns = ns;
+  for (int i = 0; i < ns; ++i) { rk.A[i] = A[i]; rk.B[i] = B[i]; }
+  const unsigned blocks = (unsigned)((g.n[0] + LINE_CELLS - 1) / LINE_CELLS);
+  dispatch(conv, avg, [&](auto c, auto a) {
+    constexpr int C = decltype(c)::value, V = decltype(a)::value;
+    if (mode == 0) k_line_stage<C, V, 0><<<blocks, 64, 0, st>>>(in, Q, Qo, Qn, g.fs, ph, rk, s);
+    else k_line_stage<C, V, 1><<<blocks, 64, 0, st>>>(in, Q, Qo, Qn, g.fs, ph, rk, s);
+  });
+}
+
+}  // namespace osbl
 
 extern "C" {
 
@@ -419,7 +535,7 @@ int osbl_batch_create(const osbl_config* base, int ninst, const int32_t* n, cons
   // staged mode segment lists
   std::vector<int> si, sc, pi, pp;
   for (int i = 0; i < ninst; ++i) {
-    for (int c = 0; c < n[i]; c += b->seglen) { si.push_back(i); sc.push_back(c); }
+    for (int c = 0; c < n[i]; c += LINE_CELLS) { si.push_back(i); sc.push_back(c); }
     for (int p = -BH; p < n[i] + BH; ++p) { pi.push_back(i); pp.push_back(p); }
   }
   b->nseg = (int)si.size();

@@ -65,6 +65,16 @@ void launch_curv_direction(int nd, int d, int conv, int avg, const double* Q, co
 void launch_curv_metric(int nd, const double* X, double* M, const Grid& g, const Phys& ph, const int e[3],
                         hipStream_t s);
 
+// 1-D block with zeroth-order extrapolation ends: nsteps iterations of a line
+// of at most LINE_RUN_MAX points in one launch (state left in Q, ends filled;
+// Q2 and Qo are scratch), or one stage Q -> Qn of any line (its ends are read
+// as the boundary condition gives them, and left to a later boundary pass)
+constexpr int LINE_RUN_MAX = 16 * 63;
+int launch_line_run(int conv, int avg, int mode, double* Q, double* Q2, double* Qo, const Grid& g, const Phys& ph,
+                    const double* A, const double* B, int ns, int nsteps, hipStream_t s);
+void launch_line_stage(int conv, int avg, int mode, const double* Q, double* Qo, double* Qn, const Grid& g,
+                       const Phys& ph, const double* A, const double* B, int ns, int stage, hipStream_t s);
+
 // record the thread-local message osbl_last_error() returns; returns code
 int set_error(int code, const char* msg);
 

@@ -200,6 +200,7 @@ struct osbl_ctx {
   bool tiled_visc = false;  // 3-D characteristic scheme with viscous terms
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
   bool tiled_central = false;  // 3-D periodic central scheme: tiled convective kernel (+ tiled viscous kernel)
+  bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
   bool general = false;     // closures, metric or Sutherland viscosity: the general update kernel
   bool suth = false;
   Bnd bnd{};
@@ -628,6 +629,8 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->csz = conv3d_segment(c->g);
   c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear &&
                      conv3d_blocks(c->g, c->csz) >= 128;
+  c->line = c->nd == 1 && !is_central(cfg->conv) && cfg->viscous == OSBL_VISC_NONE && !stretched && !ph.has_force &&
+            cfg->bc[0][0] == OSBL_BC_EXTRAP0 && cfg->bc[0][1] == OSBL_BC_EXTRAP0;
   c->need_prims = !c->tiled_central && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   const size_t bundle = (size_t)fs * c->nv * sizeof(double);
@@ -871,6 +874,14 @@ static void iterate(osbl_ctx* c, int mode) {
   // conditions, so the iteration starts with them as the reference's does
   if (c->cfg.filters) apply_bcs(c, Qcur(c));
   for (int s = 0; s < c->nstages; ++s) {
+    if (c->line) {  // (osbl_run applies the boundary conditions at the end)
+      timed(c, F_SWEEP_X, [&] {
+        launch_line_stage(c->cfg.conv, c->cfg.averaging, mode, Qcur(c), c->Qo, c->Qbuf[1 - c->cur], c->g, c->ph, c->A,
+                          c->B, c->nstages, s, c->stream);
+      });
+      c->cur ^= 1;
+      continue;
+    }
     stage(c, mode, c->A[s], c->B[s], s == 0);
     c->cur ^= 1;
     apply_bcs(c, Qcur(c));
@@ -902,6 +913,18 @@ int osbl_run(osbl_ctx* c, int64_t niter) {
   if (niter < 0) return fail(OSBL_E_ARG, "niter must be non-negative");
   if (int rc = check_ready(c)) return rc;
   const int mode = c->cfg.rk == OSBL_RK3 ? 0 : 1;
+  if (c->line && c->g.n[0] <= LINE_RUN_MAX) {
+    // (launches of a few milliseconds at most)
+    for (int64_t it = 0; it < niter; it += 1024) {
+      int rc = OSBL_OK;
+      timed(c, F_SWEEP_X, [&] {
+        rc = launch_line_run(c->cfg.conv, c->cfg.averaging, mode, Qcur(c), c->Qbuf[1 - c->cur], c->Qo, c->g, c->ph,
+                             c->A, c->B, c->nstages, (int)std::min<int64_t>(1024, niter - it), c->stream);
+      });
+      if (rc) return rc;
+    }
+    return OSBL_OK;
+  }
   if (niter > 0) apply_bcs(c, Qcur(c));
   if ((c->cfg.filters & OSBL_FILTER_SFD) && niter > 0) {
     // "Initialize the filter" before the time loop: vfilt = v (SFD.py:50-61)
@@ -933,6 +956,7 @@ int osbl_run(osbl_ctx* c, int64_t niter) {
     }
   }
   for (; it < niter; ++it) iterate(c, mode);
+  if (c->line && niter > 0) apply_bcs(c, Qcur(c));
   HIPCHK(hipGetLastError());
   return OSBL_OK;
 }
