@@ -229,23 +229,41 @@ __global__ void __launch_bounds__(256) k_char_sweep(const double* __restrict__ Q
 
 // ---------------------------------------------------------------------------
 // Characteristic sweep along x with the lanes of a wave along x.  A wave owns
-// one grid line (one (y, z) row) and walks it in chunks of 64 cells: the
-// chunk's 69 points (x0-2 .. x0+66) are loaded with coalesced reads, their
-// constituent relations computed once and kept in LDS, then lane l evaluates
-// the flux at interface x0+l+1/2 from LDS and the residual of
-// cell x0+l is its difference with lane l-1's flux (a shuffle; lane 0 takes
-// the previous chunk's last flux).  Stores are coalesced 512-byte rows.  On a
-// periodic line the flux left of cell 0 is the line's last interface flux, so
-// cell 0 is finished after the walk; otherwise it is evaluated first.
+// `cells` consecutive cells of one (y, z) row and walks them in chunks of 64
+// interfaces: the 69 points around a chunk are staged in LDS with their
+// constituent relations, lane l evaluates the flux at interface base + l + 1/2
+// from LDS, and the residual of cell base + l is its difference with lane
+// l-1's flux (a shuffle; lane 0 takes the previous chunk's last flux).  Stores
+// are coalesced 512-byte rows.  On a periodic row of one wave the flux left of
+// cell 0 is the row's last interface flux, so cell 0 is finished after the
+// walk; otherwise the walk starts with the flux left of the first cell.
+//
+// Slot s of a chunk holds point base - 2 + s; slots 0..4 are slots 64..68 of
+// the chunk before, so each chunk stages one new point per lane, whose raw
+// values are fetched while the previous chunk evaluates its fluxes.
 // ---------------------------------------------------------------------------
-constexpr int XW = 4;             // waves (lines) per block
+constexpr int XW = 4;             // waves per block
 constexpr int XP = 64 + 5;        // points staged per chunk
 
-// (at least three waves per SIMD: TENO6 needs ~178 VGPRs otherwise and
-// would run two; held to 168 it spills four and is 6 % faster)
+// Cells per wave: the whole row when the rows alone fill the GPU (1024 SIMDs
+// times the three waves the registers allow), else 64 k - 1 cells (k chunks
+// and the flux left of the first cell) with k as large as that number of
+// waves allows.  400^2 (400 rows, 7 waves each): 21 -> 9 us.
+static int sweep_xl_cells(const Grid& g) {
+  const long long rows = (long long)g.n[1] * g.n[2];
+  const int n = g.n[0];
+  if (rows >= 3072 || n <= 63) return n;
+  for (int k = (n + 63) / 64; k > 1; --k) {
+    const int cells = 64 * k - 1;
+    if (rows * ((n + cells - 1) / cells) >= 3072) return cells >= n ? n : cells;
+  }
+  return 63;
+}
+
+// (at least three waves per SIMD)
 template <int ND, int CONV, int AVG, bool ACC>
 __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __restrict__ Q, double* __restrict__ R,
-                                                          Grid g, Phys ph, int nrows, int periodic,
+                                                          Grid g, Phys ph, int nwaves, int cells, int periodic,
                                                           const double* __restrict__ met,
                                                           const double* __restrict__ theta) {
   constexpr int NV = ND + 2;
@@ -255,15 +273,22 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
   __shared__ double sh[XW][XP][NS];
   __shared__ double edge[XW][2][NV];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int row = blockIdx.x * XW + wv;
-  if (row >= nrows) return;  // whole waves only: no block-wide barrier below
+  const int id = __builtin_amdgcn_readfirstlane(blockIdx.x * XW + wv);
+  if (id >= nwaves) return;  // whole waves only: no block-wide barrier below
   double (*S)[NS] = sh[wv];
-  const int base = g.idx(0, row % g.n[1], row / g.n[1]);
   const int N = g.n[0];
+  const int nseg = (N + cells - 1) / cells;
+  const int row = id / nseg, s0 = (id % nseg) * cells, s1 = min(s0 + cells, N);
+  const int line = g.idx(0, row % g.n[1], row / g.n[1]);
   const double inv = ph.inv_delta[0];
-  auto stage_point = [&](int slot, int x) {
+  const bool wrap = periodic && nseg == 1;
+  const int xmax = N + g.h[0] - 1;  // last stored point of the row
+  auto clampx = [&](int x) { return max(-g.h[0], min(x, xmax)); };
+  auto stage_q = [&](int slot, const double (&q)[NV]) {
     Pt<ND> p;
-    load_pt<ND>(p, Q, g.fs, base + x, ph);
+#pragma unroll
+    for (int m = 0; m < NV; ++m) p.q[m] = q[m];
+    finish_pt<ND>(p, ph);
 #pragma unroll
     for (int m = 0; m < NV; ++m) S[slot][m] = p.q[m];
 #pragma unroll
@@ -272,26 +297,7 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
     S[slot][NV + ND + 1] = p.a;
     if constexpr (ROE) roe_factors<ND>(p, S[slot][NV + ND + 2], S[slot][NV + ND + 3]);
   };
-  // flux at interface x0 + lane + 1/2 (points x0+lane-2 .. x0+lane+3 = slots lane .. lane+5)
-  const int xmax = N + g.h[0] - 1;  // last stored point of the line
-  auto flux = [&](double fh[NV], int xi) {
-    const LdsPoints<ND, NS> w{S[lane]};
-    const double ct = theta ? adaptive_ct(theta[base + min(xi, xmax)], ph) : ph.teno_ct;
-    [[maybe_unused]] RoeF rf{};
-    if constexpr (ROE) {
-      rf.sL = S[lane + 2][NV + ND + 2];
-      rf.hL = S[lane + 2][NV + ND + 3];
-      rf.sR = S[lane + 3][NV + ND + 2];
-      rf.hR = S[lane + 3][NV + ND + 3];
-    }
-    char_flux_w<ND, 0, CONV, AVG, true>(w, ph, fh, ct, rf);
-  };
-  auto stage_chunk = [&](int x0) {
-    // slots 0..68 hold points x0-2 .. x0+66 (clamped to the stored line: the
-    // clamped slots only feed lanes whose cells lie beyond the line)
-    __builtin_amdgcn_wave_barrier();
-    stage_point(lane, min(x0 - 2 + lane, xmax));
-    if (lane < XP - 64) stage_point(64 + lane, min(x0 + 62 + lane, xmax));
+  auto wave_sync = [&] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -301,39 +307,26 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
       const double v = r[m] * gi;
-      if constexpr (ACC) st_once(ld_once(&R[m * g.fs + base + x], ph.nt) + v, &R[m * g.fs + base + x], ph.nt);
-      else st_once(v, &R[m * g.fs + base + x], ph.nt);
+      if constexpr (ACC) st_once(ld_once(&R[m * g.fs + line + x], ph.nt) + v, &R[m * g.fs + line + x], ph.nt);
+      else st_once(v, &R[m * g.fs + line + x], ph.nt);
     }
   };
-  if constexpr (CONV == OSBL_CONV_WENO_Z || CONV == OSBL_CONV_WENO_JS) {
-    // Pipelined walk (the WENO sweeps have the registers for it): slot s
-    // holds point x0 - 7 + s, lane l evaluates the flux at interface
-    // I = x0 - 5 + l (points I-2 .. I+3 = slots l .. l+5) and finishes cell
-    // I.  Slots 0..4 of a chunk are slots 64..68 of the one before, so each
-    // chunk stages one new point per lane, whose raw values are fetched while
-    // the previous chunk evaluates its fluxes.  Periodic lines start at I = 0
-    // (the flux left of cell 0 is the line's last one, used after the walk),
-    // others at I = -1.
-    auto clampx = [&](int x) { return max(-g.h[0], min(x, xmax)); };
-    auto stage_q = [&](int slot, const double (&q)[NV]) {
-      Pt<ND> p;
-#pragma unroll
-      for (int m = 0; m < NV; ++m) p.q[m] = q[m];
-      finish_pt<ND>(p, ph);
-#pragma unroll
-      for (int m = 0; m < NV; ++m) S[slot][m] = p.q[m];
-#pragma unroll
-      for (int m = 0; m < ND; ++m) S[slot][NV + m] = p.u[m];
-      S[slot][NV + ND] = p.p;
-      S[slot][NV + ND + 1] = p.a;
-      if constexpr (ROE) roe_factors<ND>(p, S[slot][NV + ND + 2], S[slot][NV + ND + 3]);
-    };
-    auto wave_sync = [&] {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    auto flux_at = [&](double fh[NV]) {
+  int base = wrap ? s0 : s0 - 1;
+  double nq[NV];
+  if (lane < 5) {
+    double q0[NV];
+    fetch_q<ND>(q0, Q, g.fs, line + clampx(base - 2 + lane));
+    stage_q(lane, q0);
+  }
+  fetch_q<ND>(nq, Q, g.fs, line + clampx(base + 3 + lane));
+  for (bool start = true; base < s1; base += 64, start = false) {
+    stage_q(5 + lane, nq);
+    wave_sync();
+    // the next chunk's point, in flight while this chunk's fluxes are evaluated
+    fetch_q<ND>(nq, Q, g.fs, line + clampx(base + 67 + lane));
+    const int I = base + lane;
+    double fh[NV];
+    {
       const LdsPoints<ND, NS> w{S[lane]};
       [[maybe_unused]] RoeF rf{};
       if constexpr (ROE) {
@@ -342,99 +335,41 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
         rf.sR = S[lane + 3][NV + ND + 2];
         rf.hR = S[lane + 3][NV + ND + 3];
       }
-      char_flux_w<ND, 0, CONV, AVG, true>(w, ph, fh, ph.teno_ct, rf);
-    };
-    const int x0s = periodic ? 5 : 4;
-    double nq[NV];
+      const double ct = theta ? adaptive_ct(theta[line + min(I, xmax)], ph) : ph.teno_ct;
+      char_flux_w<ND, 0, CONV, AVG, true>(w, ph, fh, ct, rf);
+    }
+    double r[NV];
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      const double up = __shfl_up(fh[m], 1);
+      r[m] = fh[m] - (lane == 0 ? edge[wv][0][m] : up);
+    }
+    // the first flux and the chunk's last one wait in LDS (registers are what bounds the kernel)
+    const int last = min(63, s1 - 1 - base);
+    if (lane == 0 && start) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m) edge[wv][1][m] = fh[m];
+    }
+    wave_sync();
+    if (lane == last) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m) edge[wv][0][m] = fh[m];
+    }
+    if (I >= s0 && I < s1 && !(wrap && I == 0)) emit(I, r);
+    // slots 64..68 become slots 0..4 of the next chunk
+    wave_sync();
     if (lane < 5) {
-      double q0[NV];
-      fetch_q<ND>(q0, Q, g.fs, base + clampx(x0s - 7 + lane));
-      stage_q(lane, q0);
-    }
-    fetch_q<ND>(nq, Q, g.fs, base + clampx(x0s - 2 + lane));
-    for (int x0 = x0s; x0 - 5 <= N - 1; x0 += 64) {
-      stage_q(5 + lane, nq);
-      wave_sync();
-      // the next chunk's point, in flight while this chunk's fluxes are evaluated
-      fetch_q<ND>(nq, Q, g.fs, base + clampx(x0 + 62 + lane));
-      double fh[NV];
-      const int I = x0 - 5 + lane;
-      flux_at(fh);
-      double r[NV];
 #pragma unroll
-      for (int m = 0; m < NV; ++m) {
-        const double up = __shfl_up(fh[m], 1);
-        r[m] = fh[m] - (lane == 0 ? edge[wv][0][m] : up);
-      }
-      // the line's first and last flux of the chunk wait in LDS (registers are what bounds the kernel)
-      const int last = min(63, N - 1 - (x0 - 5));
-      if (lane == 0 && x0 == x0s) {
+      for (int e = 0; e < NF; ++e) S[lane][e] = S[64 + lane][e];
+    }
+    wave_sync();
+  }
+  if (wrap && lane == 0) {
+    // the row's last interface flux is the flux left of cell 0
+    double r[NV];
 #pragma unroll
-        for (int m = 0; m < NV; ++m) edge[wv][1][m] = fh[m];
-      }
-      wave_sync();
-      if (lane == last) {
-#pragma unroll
-        for (int m = 0; m < NV; ++m) edge[wv][0][m] = fh[m];
-      }
-      if (I >= 0 && I < N && !(periodic && I == 0)) emit(I, r);
-      // slots 64..68 become slots 0..4 of the next chunk
-      wave_sync();
-      if (lane < 5) {
-#pragma unroll
-        for (int e = 0; e < NF; ++e) S[lane][e] = S[64 + lane][e];
-      }
-      wave_sync();
-    }
-    if (periodic && lane == 0) {
-      // the line's last interface flux is the flux left of cell 0
-      double r[NV];
-#pragma unroll
-      for (int m = 0; m < NV; ++m) r[m] = edge[wv][1][m] - edge[wv][0][m];
-      emit(0, r);
-    }
-  } else {
-    double prev[NV];  // flux left of the chunk's first cell (valid in every lane)
-    double first[NV];
-    if (!periodic) {
-      // flux at interface -1/2 (points -3..2): lane 0 of a chunk staged at x0 = -1
-      stage_chunk(-1);
-      double fh[NV];
-      flux(fh, -1 + lane);
-  #pragma unroll
-      for (int m = 0; m < NV; ++m) prev[m] = __shfl(fh[m], 0);
-    }
-    for (int x0 = 0; x0 < N; x0 += 64) {
-      stage_chunk(x0);
-      double fh[NV];
-      flux(fh, x0 + lane);
-      const int x = x0 + lane;
-      double left[NV];
-  #pragma unroll
-      for (int m = 0; m < NV; ++m) {
-        const double up = __shfl_up(fh[m], 1);
-        left[m] = lane == 0 ? prev[m] : up;
-      }
-      const int last = min(63, N - 1 - x0);  // lane holding the chunk's last valid interface
-  #pragma unroll
-      for (int m = 0; m < NV; ++m) {
-        if (x0 == 0) first[m] = fh[m];
-        prev[m] = __shfl(fh[m], last);
-      }
-      if (x < N && !(periodic && x == 0)) {
-        double r[NV];
-  #pragma unroll
-        for (int m = 0; m < NV; ++m) r[m] = fh[m] - left[m];
-        emit(x, r);
-      }
-    }
-    if (periodic && lane == 0) {
-      // the line's last interface flux is the flux left of cell 0
-      double r[NV];
-  #pragma unroll
-      for (int m = 0; m < NV; ++m) r[m] = first[m] - prev[m];
-      emit(0, r);
-    }
+    for (int m = 0; m < NV; ++m) r[m] = edge[wv][1][m] - edge[wv][0][m];
+    emit(0, r);
   }
 }
 
@@ -1179,12 +1114,15 @@ template <int ND, int D, int CONV, int AVG>
 static void launch_sweep_t(const double* Q, double* R, const Grid& g, const Phys& ph, int seg, bool acc,
                            const double* met, const double* theta, hipStream_t s) {
   if constexpr (D == 0 && ND >= 2) {
-    const int nrows = g.n[1] * g.n[2];
-    const unsigned blocks = (unsigned)((nrows + XW - 1) / XW);
+    const int cells = sweep_xl_cells(g);
+    const int nwaves = g.n[1] * g.n[2] * ((g.n[0] + cells - 1) / cells);
+    const unsigned blocks = (unsigned)((nwaves + XW - 1) / XW);
     if (acc)
-      k_char_sweep_xl<ND, CONV, AVG, true><<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nrows, g.periodic_x, met, theta);
+      k_char_sweep_xl<ND, CONV, AVG, true>
+          <<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nwaves, cells, g.periodic_x, met, theta);
     else
-      k_char_sweep_xl<ND, CONV, AVG, false><<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nrows, g.periodic_x, met, theta);
+      k_char_sweep_xl<ND, CONV, AVG, false>
+          <<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nwaves, cells, g.periodic_x, met, theta);
     return;
   }
   long long lines = 1;

@@ -1,0 +1,59 @@
+"""Block shapes at which the 2-D and 3-D kernels split their work differently
+(rows of one wave or several, chunks of 64 interfaces, tiles and their
+remainders), against the oracle: residual and five steps, relative L2 <= 1e-10
+per variable."""
+import numpy as np
+import pytest
+
+from conftest import check_parity
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(n, conv, bc, averaging="roe", rk="rk3", viscous="none", seed=0):
+    """A block of order-one variables, smooth and periodic, on [0, 1)^d."""
+    nd = len(n)
+    x = np.meshgrid(*[np.arange(k) / k for k in reversed(n)], indexing="ij")
+    rs = np.random.RandomState(seed)
+
+    def wave(amp):
+        return amp * sum(np.sin(2 * np.pi * (rs.randint(1, 3) * c + rs.rand())) for c in x)
+    rho = 1.0 + wave(0.1)
+    u = [0.3 + wave(0.1) for _ in range(nd)]
+    p = 1.0 + wave(0.1)
+    q0 = np.stack([rho] + [rho * v for v in u] + [p / 0.4 + 0.5 * rho * sum(v * v for v in u)])
+    delta = [1.0 / k for k in n]
+    problem = dict(ndim=nd, n=list(n), delta=delta, conv=conv, averaging=averaging, viscous=viscous, rk=rk,
+                   bc=[[bc, bc]] * nd, gama=1.4, Minf=1.0, Re=100.0, Pr=0.71, dt=0.1 * min(delta), eps=1e-16,
+                   teno_ct=1e-6)
+    return problem, q0
+
+
+def _check(problem, q0, oracle, what):
+    from opensbli_amd.native import Block
+    print("case", what, flush=True)
+    g, r = Block(problem), oracle.RefSolver(problem)
+    g.set_state(q0)
+    r.set_state(q0)
+    check_parity(g.rhs(), r.rhs(), what + " residual")
+    g.set_state(q0)
+    r.set_state(q0)
+    g.run(5)
+    r.run(5)
+    check_parity(g.get_state(), r.get_state(), what)
+
+
+@pytest.mark.parametrize("bc", ["periodic", "extrap0"])
+@pytest.mark.parametrize("conv,averaging,rk", [("weno_z", "roe", "rk3"), ("weno_js", "simple", "ls3"),
+                                               ("teno5", "roe", "rk3"), ("teno6", "roe", "ls3")])
+@pytest.mark.parametrize("n", [(8, 8), (62, 9), (63, 17), (64, 16), (65, 33), (127, 8), (190, 40), (64, 3100)])
+def test_2d_shapes(n, conv, averaging, rk, bc, oracle):
+    problem, q0 = _block(n, conv, bc, averaging, rk)
+    _check(problem, q0, oracle, f"2-D {n} {conv} {averaging} {rk} {bc}")
+
+
+@pytest.mark.parametrize("conv", ["weno_z", "teno6"])
+@pytest.mark.parametrize("n", [(8, 8, 8), (63, 9, 10), (66, 17, 9), (130, 12, 33)])
+def test_3d_shapes(n, conv, oracle):
+    problem, q0 = _block(n, conv, "periodic", viscous="const")
+    _check(problem, q0, oracle, f"3-D {n} {conv}")
