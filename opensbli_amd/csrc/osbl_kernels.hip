@@ -525,7 +525,6 @@ __device__ __forceinline__ void central_convective(const double* __restrict__ Q,
 //   MODE 1: low-storage stage (rk_LS.py:155-166): Qo = cA*Qo + dt*R,
 //           Qn = Q + cB*Qo (Qo not read when cA == 0).
 //   MODE 2: residual only (written to R).
-//   MODE 3 (k_visc_update3d only): the viscous terms alone, assigned to R.
 // For characteristic schemes the convective residual is already in R.
 // ---------------------------------------------------------------------------
 template <int ND, int CONV, bool VISC, int MODE>
@@ -587,10 +586,8 @@ constexpr int VTX = 64, VTY = 8, VPX = VTX + 4, VPY = VTY + 4, VPL = VPX * VPY;
 constexpr int VNT = VTX * VTY;                 // threads per block
 constexpr int VPP = (VPL + VNT - 1) / VNT;     // staged points per thread and plane
 
-template <int MODE>
-__global__ void __launch_bounds__(VNT, 2) k_visc_update3d(const double* __restrict__ Q, double* __restrict__ R,
-                                                       double* __restrict__ Qo, double* __restrict__ Qn, Grid g,
-                                                       Phys ph, double cA, double cB, int first, int sz) {
+__global__ void __launch_bounds__(VNT, 2) k_visc_update3d(const double* __restrict__ Q, double* __restrict__ R, Grid g,
+                                                       Phys ph, int sz) {
   __shared__ double sp[4][4][VPL];
   const int tx = threadIdx.x, ty = threadIdx.y;
   const int tid = ty * VTX + tx;
@@ -689,19 +686,11 @@ __global__ void __launch_bounds__(VNT, 2) k_visc_update3d(const double* __restri
     const bool more = z + 1 < z1;  // plane z+3 feeds the next plane's queue entry
     if (more) fetch(z + 3);
     const int o = g.idx(x, y, z);
-    // the cell's residual and RK registers, in flight during the arithmetic
-    double rin[5], qa[5], qb[5];
+    // the cell's residual, in flight during the arithmetic
+    double rin[5];
     if (inside) {
 #pragma unroll
-      for (int m = 0; m < 5; ++m) {
-        if constexpr (MODE == 2) rin[m] = ld_once(&R[m * g.fs + o], ph.nt);
-        if constexpr (MODE == 0 || MODE == 1) rin[m] = ld_once(&R[m * g.fs + o], ph.nt);
-        if constexpr (MODE == 0) qa[m] = first ? Q[m * g.fs + o] : ld_once(&Qo[m * g.fs + o], ph.nt);
-        if constexpr (MODE == 1) {
-          qa[m] = cA == 0.0 ? 0.0 : ld_once(&Qo[m * g.fs + o], ph.nt);
-          qb[m] = Q[m * g.fs + o];
-        }
-      }
+      for (int m = 0; m < 5; ++m) rin[m] = ld_once(&R[m * g.fs + o], ph.nt);
       const int sl = slot_of(z);
       const double* U[3] = {sp[sl][0], sp[sl][1], sp[sl][2]};
       const double* T = sp[sl][3];
@@ -765,27 +754,8 @@ __global__ void __launch_bounds__(VNT, 2) k_visc_update3d(const double* __restri
         r[1 + m] = visc;
       }
       r[4] = energy;
-      if constexpr (MODE != 3) {
 #pragma unroll
-        for (int m = 0; m < 5; ++m) r[m] = rin[m] + r[m];
-      }
-      if constexpr (MODE == 2 || MODE == 3) {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) st_once(r[m], &R[m * g.fs + o], ph.nt);
-      } else if constexpr (MODE == 0) {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) {
-          st_once(qa[m] + ph.dt * cA * r[m], &Qn[m * g.fs + o], ph.nt);
-          st_once(qa[m] + ph.dt * cB * r[m], &Qo[m * g.fs + o], ph.nt);
-        }
-      } else {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) {
-          const double tmp = (cA == 0.0 ? 0.0 : cA * qa[m]) + ph.dt * r[m];
-          st_once(tmp, &Qo[m * g.fs + o], ph.nt);
-          st_once(qb[m] + cB * tmp, &Qn[m * g.fs + o], ph.nt);
-        }
-      }
+      for (int m = 0; m < 5; ++m) st_once(rin[m] + r[m], &R[m * g.fs + o], ph.nt);
     }
     if (more) {
       // plane z+3 replaces plane z-1 (last read before the previous barrier)
@@ -800,67 +770,70 @@ __global__ void __launch_bounds__(VNT, 2) k_visc_update3d(const double* __restri
   }
 }
 
-void launch_visc_update3d(int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g, const Phys& ph,
-                          double cA, double cB, int first, int sz, hipStream_t s) {
+void launch_visc_update3d(const double* Q, double* R, const Grid& g, const Phys& ph, int sz, hipStream_t s) {
   dim3 grid((g.n[0] + VTX - 1) / VTX, (g.n[1] + VTY - 1) / VTY, (g.n[2] + sz - 1) / sz);
-  dim3 block(VTX, VTY);
-  if (mode == 0) k_visc_update3d<0><<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz);
-  else if (mode == 1) k_visc_update3d<1><<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz);
-  else if (mode == 2) k_visc_update3d<2><<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz);
-  else k_visc_update3d<3><<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz);
+  k_visc_update3d<<<grid, dim3(VTX, VTY), 0, s>>>(Q, R, g, ph, sz);
 }
 
 // ---------------------------------------------------------------------------
-// 3-D central convective terms, tiled 2.5-D.  Skew-symmetric (Blaisdell) form
-// (parsing.py:75-111, scheme.py:187-252) or the conservative flux form
-// (parsing.py:189-216), with the formulas of central_convective.  A CTX x CTY
-// block of (x, y) columns marches along z.  The plane being evaluated is
-// staged in LDS (Q, u_x, u_y, p with a 2-point x/y halo, the x/y stencils);
-// each thread keeps a register queue of its own column's Q, u_z, p over the
-// five planes z-2..z+2 (the z stencils).  Software pipeline: the raw Q of the
-// next plane's staged points and of the column point three planes ahead are
-// loaded at the top of an iteration and consumed after its arithmetic; two
-// LDS slots alternate, one barrier per plane.
-//   MODE 0/1: RK update (no viscous terms); MODE 2: the terms are assigned to
-//   R (the viscous kernel then adds its terms and applies the update).
+// One stage of a 3-D central scheme in one kernel: convective terms in the
+// skew-symmetric (Blaisdell) form (parsing.py:75-111, scheme.py:187-252) or
+// the conservative flux form (parsing.py:189-216), constant-viscosity terms
+// (scheme.py:299-387) and the RK update, with the formulas of
+// central_convective and viscous_terms.
+//
+// A 64 x TY block of (x, y) columns marches along z.  When plane z+2 is in
+// LDS (conservative and primitive variables with a 2-point x/y halo), each
+// thread evaluates everything that needs only that plane for its column --
+// the x and y terms, added up in r -- and keeps in a register queue over
+// five planes what the z stencils need: Q, 1/rho and the inner derivatives
+// D_x u_0 + D_y u_1, D_x u_2, D_y u_2 of the mixed terms.  Then plane z is
+// complete.  With the sums folded, the viscous terms need nothing else kept:
+//   rhou_m: (1/Re) (lap u_m + D_m(div u)/3)
+//   rhoE:   u . the above + (1/Re) (2 sum_m (D_m u_m)^2 - 2/3 (div u)^2
+//           + sum_{m<j} (D_m u_j + D_j u_m)^2) + cq lap T
+// The raw Q of the next plane is in flight during the arithmetic; two LDS
+// slots alternate, one barrier per plane.  On a block periodic in every
+// direction (`wrap`) the staged points are read at their periodic images, so
+// the halos need not be filled between stages.
+//
+// The stage moves Q, the register and the new state once: 160 B per cell
+// against 280 for a convective kernel that leaves R to a viscous kernel.
+//   MODE 0/1: RK update; MODE 2: the residual alone, into R.
 // ---------------------------------------------------------------------------
-constexpr int CTX = 64, CTY = 4, CPX = CTX + 4, CPY = CTY + 4, CPL = CPX * CPY;
-constexpr int CNT = CTX * CTY;                 // threads per block
-constexpr int CPP = (CPL + CNT - 1) / CNT;     // staged points per thread and plane
-constexpr int CNF = 8;                         // staged fields: Q0..Q4, u_x, u_y, p
-
-template <int CONV, int MODE>
-__global__ void __launch_bounds__(CNT, 2) k_conv3d(const double* __restrict__ Q, double* __restrict__ R,
-                                                   double* __restrict__ Qo, double* __restrict__ Qn, Grid g, Phys ph,
-                                                   double cA, double cB, int first, int sz) {
-  constexpr int NV = 5;
-  __shared__ double sp[2][CNF][CPL];
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int tid = ty * CTX + tx;
+template <int CONV, bool VISC, int MODE, int TX, int TY>
+__global__ void __launch_bounds__(TX * TY, 2)
+    k_central3d(const double* __restrict__ Q, double* __restrict__ R, double* __restrict__ Qo,
+                double* __restrict__ Qn, Grid g, Phys ph, double cA, double cB, int first, int sz, int wrap) {
+  constexpr int NV = 5, PX = TX + 4, PY = TY + 4, PL = PX * PY, NT = TX * TY;
+  constexpr int PP = (PL + NT - 1) / NT;     // staged points per thread and plane
+  constexpr int NF = VISC ? 11 : 9;          // Q0..Q4, u0, u1, u2, p (, T, pad): odd, no bank conflicts
+  constexpr int NQ = VISC ? 9 : 6;           // queue: Q0..Q4, 1/rho (, D_x u0 + D_y u1, D_x u2, D_y u2)
+  __shared__ double sp[2][PL][NF];
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
   int bx, by, bz;
   xcd_tile(bx, by, bz);
-  const int x0 = bx * CTX, y0 = by * CTY;
-  const int z0 = bz * sz;
-  const int z1 = min(z0 + sz, g.n[2]);
+  const int x0 = bx * TX, y0 = by * TY, z0 = bz * sz, z1 = min(z0 + sz, g.n[2]);
   const int x = x0 + tx, y = y0 + ty;
   const bool inside = x < g.n[0] && y < g.n[1];
+  const double ix = ph.inv_delta[0], iy = ph.inv_delta[1], iz = ph.inv_delta[2];
+  const double cT = ph.gama * ph.Minf * ph.Minf;
 
-  int sidx[CPP], soff[CPP];
-  bool sval[CPP];
+  auto image = [&](int i, int n) { return !wrap ? i : (i < 0 ? i + n : (i >= n ? i - n : i)); };
+  int soff[PP];
+  bool sval[PP];
 #pragma unroll
-  for (int k = 0; k < CPP; ++k) {
-    const int p = tid + k * CNT;
-    const int xx = p % CPX, yy = p / CPX;
-    const int gx = x0 - 2 + xx, gy = y0 - 2 + yy;
-    sidx[k] = p;
-    sval[k] = p < CPL && gx < g.n[0] + g.h[0] && gy < g.n[1] + g.h[1];
-    soff[k] = sval[k] ? g.idx(gx, gy, 0) : 0;
+  for (int k = 0; k < PP; ++k) {
+    const int pt = tid + k * NT;
+    const int gx = x0 - 2 + pt % PX, gy = y0 - 2 + pt / PX;
+    sval[k] = pt < PL && gx < g.n[0] + 2 && gy < g.n[1] + 2;
+    soff[k] = sval[k] ? g.idx(image(gx, g.n[0]), image(gy, g.n[1]), 0) : 0;
   }
-  double pq[CPP][NV];  // raw Q of the next plane's staged points
+  double pq[PP][NV];  // raw Q of the plane in flight
   auto fetch = [&](int zp) {
-    const int zo = zp * g.plane;
+    const int zo = image(zp, g.n[2]) * g.plane;
 #pragma unroll
-    for (int k = 0; k < CPP; ++k)
+    for (int k = 0; k < PP; ++k)
       if (sval[k]) {
 #pragma unroll
         for (int m = 0; m < NV; ++m) pq[k][m] = Q[m * g.fs + soff[k] + zo];
@@ -868,173 +841,222 @@ __global__ void __launch_bounds__(CNT, 2) k_conv3d(const double* __restrict__ Q,
   };
   auto store = [&](int slot) {
 #pragma unroll
-    for (int k = 0; k < CPP; ++k)
+    for (int k = 0; k < PP; ++k)
       if (sval[k]) {
+        const int pt = tid + k * NT;
         const double rho = pq[k][0];
         const double ir = recip_pos(rho);
         const double u0 = pq[k][1] * ir, u1 = pq[k][2] * ir, u2 = pq[k][3] * ir;
         const double pr = ph.gm1 * (pq[k][4] - 0.5 * rho * (u0 * u0 + u1 * u1 + u2 * u2));
-        const int p = sidx[k];
 #pragma unroll
-        for (int m = 0; m < NV; ++m) sp[slot][m][p] = pq[k][m];
-        sp[slot][5][p] = u0;
-        sp[slot][6][p] = u1;
-        sp[slot][7][p] = pr;
+        for (int m = 0; m < NV; ++m) sp[slot][pt][m] = pq[k][m];
+        sp[slot][pt][5] = u0;
+        sp[slot][pt][6] = u1;
+        sp[slot][pt][7] = u2;
+        sp[slot][pt][8] = pr;
+        if constexpr (VISC) sp[slot][pt][9] = cT * pr * ir;
       }
   };
-  // this thread's column: raw Q of one plane, and its queue entries Q0..Q4, u_z, p
-  const int col = inside ? g.idx(x, y, 0) : 0;
-  double oq[NV];
-  auto fetch_col = [&](int zp) {
-    if (inside) {
-      const int o = col + zp * g.plane;
+  const int c = (ty + 2) * PX + tx + 2;  // this thread's column in a slot
+  auto d1 = [](double fm2, double fm1, double fp1, double fp2) {
+    return (1.0 / 12.0) * (fm2 - fp2) + (2.0 / 3.0) * (fp1 - fm1);
+  };
+  auto d2 = [](double fm2, double fm1, double f0, double fp1, double fp2) {
+    return (-1.0 / 12.0) * (fm2 + fp2) + (4.0 / 3.0) * (fm1 + fp1) - 2.5 * f0;
+  };
+  // derivatives of field f about the point `o` of a slot, along stride st
+  auto at1 = [&](const double (*S)[NF], int f, int o, int st) {
+    return d1(S[o - 2 * st][f], S[o - st][f], S[o + st][f], S[o + 2 * st][f]);
+  };
+  auto at2 = [&](const double (*S)[NF], int f, int o, int st) {
+    return d2(S[o - 2 * st][f], S[o - st][f], S[o][f], S[o + st][f], S[o + 2 * st][f]);
+  };
+  // convective terms along one direction: values of Q_m, u_j, p at the
+  // offsets -2, -1, 1, 2 through fq, fu, fp; the cell's own Q and u_j
+  auto convect = [&](int j, double inv, auto&& fq, auto&& fu, auto&& fp, const double (&q0)[NV], double u0, double* r) {
+    double qv[4][NV], uv[4], pv[4];
 #pragma unroll
-      for (int m = 0; m < NV; ++m) oq[m] = Q[m * g.fs + o];
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m) qv[s][m] = fq(s, m);
+      uv[s] = fu(s);
+      pv[s] = fp(s);
+    }
+    const double dp = inv * d1(pv[0], pv[1], pv[2], pv[3]);
+    if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
+      const double hi = -0.5 * inv, hu = hi * u0;
+      const double du = hi * d1(uv[0], uv[1], uv[2], uv[3]);
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        const double dru = d1(qv[0][m] * uv[0], qv[1][m] * uv[1], qv[2][m] * uv[2], qv[3][m] * uv[3]);
+        const double dq = d1(qv[0][m], qv[1][m], qv[2][m], qv[3][m]);
+        r[m] += hi * dru + hu * dq + q0[m] * du;
+        if (m == 1 + j) r[m] -= dp;
+      }
+      r[4] -= inv * d1(pv[0] * uv[0], pv[1] * uv[1], pv[2] * uv[2], pv[3] * uv[3]);
+    } else {
+      r[0] -= inv * d1(qv[0][1 + j], qv[1][1 + j], qv[2][1 + j], qv[3][1 + j]);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        r[1 + m] -= inv * d1(qv[0][1 + m] * uv[0], qv[1][1 + m] * uv[1], qv[2][1 + m] * uv[2], qv[3][1 + m] * uv[3]);
+        if (m == j) r[1 + m] -= dp;
+      }
+      r[4] -= inv * d1((qv[0][4] + pv[0]) * uv[0], (qv[1][4] + pv[1]) * uv[1], (qv[2][4] + pv[2]) * uv[2],
+                       (qv[3][4] + pv[3]) * uv[3]);
     }
   };
-  auto col_entry = [&](double* e) {
-    const double rho = oq[0];
-    const double ir = recip_pos(rho);
-    const double u0 = oq[1] * ir, u1 = oq[2] * ir, u2 = oq[3] * ir;
+
+  // (what has been added up so far is finished before the next terms' values
+  // are read from LDS: the registers hold one direction's at a time)
+  auto settle = [](double* r) {
 #pragma unroll
-    for (int m = 0; m < NV; ++m) e[m] = oq[m];
-    e[5] = u2;
-    e[6] = ph.gm1 * (oq[4] - 0.5 * rho * (u0 * u0 + u1 * u1 + u2 * u2));
+    for (int m = 0; m < NV; ++m) asm volatile("" : "+v"(r[m]) : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
-  const int c = (ty + 2) * CPX + tx + 2;  // this thread's point in a slot
 
-  double zq[5][7];  // planes z-2..z+2 of this column
-  // prologue: the queue for z0 (planes z0-2 .. z0+2), plane z0 staged
-  for (int k = 0; k < 5; ++k) {
-    fetch_col(z0 - 2 + k);
-    if (inside) col_entry(zq[k]);
-  }
-  fetch(z0);
+  double zq[5][NQ];   // planes z-2 .. z+2 of this column
+  double rr[3][NV];   // the in-plane sums of planes z, z+1, z+2
+  fetch(z0 - 2);
   store(z0 & 1);
-  if (z0 + 1 < z1) {  // in flight during the first plane
-    fetch(z0 + 1);
-    fetch_col(z0 + 3);
-  }
   __syncthreads();
-
-  constexpr double W1A = 1.0 / 12.0, W1B = 2.0 / 3.0;
-  for (int z = z0; z < z1; ++z) {
-    const bool more = z + 1 < z1;
+  for (int zp = z0 - 2; zp < z1 + 2; ++zp) {
+    const int z = zp - 2;  // the plane that plane zp completes
+    const bool more = zp + 1 < z1 + 2;
+    if (more) fetch(zp + 1);
     const int o = g.idx(x, y, z);
-    if (inside) {
-      // RK registers of the cell, in flight during the arithmetic
-      [[maybe_unused]] double qa[NV], qb[NV];
+    [[maybe_unused]] double qa[NV];
+    if (inside && z >= z0) {
 #pragma unroll
       for (int m = 0; m < NV; ++m) {
         if constexpr (MODE == 0) qa[m] = first ? 0.0 : ld_once(&Qo[m * g.fs + o], ph.nt);
         if constexpr (MODE == 1) qa[m] = cA == 0.0 ? 0.0 : ld_once(&Qo[m * g.fs + o], ph.nt);
       }
-      const int sl = z & 1;
-      double r[NV];
-#pragma unroll
-      for (int m = 0; m < NV; ++m) r[m] = 0.0;
-      // x and y from LDS (stride 1 and CPX), then z from the queue
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double inv = ph.inv_delta[j];
-        const double wts[4] = {W1A, -W1B, W1B, -W1A};
-        auto qv = [&](int q, int m) -> double {  // Q_m at stencil point q (offsets -2,-1,+1,+2)
-          if (j == 2) return zq[q < 2 ? q : q + 1][m];
-          const int st = j == 0 ? 1 : CPX;
-          const int off = (q < 2 ? q - 2 : q - 1) * st;
-          return sp[sl][m][c + off];
-        };
-        auto uv = [&](int q) -> double {  // u_j at stencil point q
-          if (j == 2) return zq[q < 2 ? q : q + 1][5];
-          const int st = j == 0 ? 1 : CPX;
-          const int off = (q < 2 ? q - 2 : q - 1) * st;
-          return sp[sl][5 + j][c + off];
-        };
-        auto pv = [&](int q) -> double {
-          if (j == 2) return zq[q < 2 ? q : q + 1][6];
-          const int st = j == 0 ? 1 : CPX;
-          const int off = (q < 2 ? q - 2 : q - 1) * st;
-          return sp[sl][7][c + off];
-        };
-        if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
-          double d_ru[NV], d_q[NV], d_uj = 0.0, d_p = 0.0, d_puj = 0.0;
-#pragma unroll
-          for (int m = 0; m < NV; ++m) { d_ru[m] = 0.0; d_q[m] = 0.0; }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const double w = wts[q];
-            const double uj = uv(q);
-            const double pp = pv(q);
-#pragma unroll
-            for (int m = 0; m < NV; ++m) {
-              const double qm = qv(q, m);
-              d_ru[m] += w * (qm * uj);
-              d_q[m] += w * qm;
-            }
-            d_uj += w * uj;
-            d_p += w * pp;
-            d_puj += w * (pp * uj);
-          }
-          const double uj = j == 2 ? zq[2][5] : sp[sl][5 + j][c];
-          const double duj = inv * d_uj;
-#pragma unroll
-          for (int m = 0; m < NV; ++m) {
-            const double qm = zq[2][m];
-            double t = -0.5 * (inv * d_ru[m] + uj * (inv * d_q[m]) + qm * duj);
-            if (m == 1 + j) t -= inv * d_p;
-            if (m == NV - 1) t -= inv * d_puj;
-            r[m] += t;
-          }
-        } else {
-          double dF[NV];
-#pragma unroll
-          for (int m = 0; m < NV; ++m) dF[m] = 0.0;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const double w = wts[q];
-            const double uj = uv(q);
-            const double pp = pv(q);
-            dF[0] += w * qv(q, 1 + j);
-#pragma unroll
-            for (int m = 0; m < 3; ++m) dF[1 + m] += w * (qv(q, 1 + m) * uj + (m == j ? pp : 0.0));
-            dF[NV - 1] += w * ((pp + qv(q, NV - 1)) * uj);
-          }
-#pragma unroll
-          for (int m = 0; m < NV; ++m) r[m] -= inv * dF[m];
-        }
-      }
-      if constexpr (MODE == 2) {
-#pragma unroll
-        for (int m = 0; m < NV; ++m) st_once(r[m], &R[m * g.fs + o], ph.nt);
-      } else if constexpr (MODE == 0) {
-#pragma unroll
-        for (int m = 0; m < NV; ++m) {
-          const double qo = first ? zq[2][m] : qa[m];
-          st_once(qo + ph.dt * cA * r[m], &Qn[m * g.fs + o], ph.nt);
-          st_once(qo + ph.dt * cB * r[m], &Qo[m * g.fs + o], ph.nt);
-        }
-      } else {
-#pragma unroll
-        for (int m = 0; m < NV; ++m) {
-          const double tmp = (cA == 0.0 ? 0.0 : cA * qa[m]) + ph.dt * r[m];
-          st_once(tmp, &Qo[m * g.fs + o], ph.nt);
-          st_once(zq[2][m] + cB * tmp, &Qn[m * g.fs + o], ph.nt);
-        }
-      }
     }
-    if (more) {
-      // plane z+1 goes into the slot plane z-1 left (last read before the
-      // previous barrier); the queue moves on by one plane
-      store((z + 1) & 1);
+    const double (*S)[NF] = sp[zp & 1];
+    if (inside) {
+      double* e = zq[4];
+#pragma unroll
+      for (int m = 0; m < NV; ++m) e[m] = S[c][m];
+      e[5] = recip_pos(e[0]);
+      [[maybe_unused]] double ux, vy;
+      if constexpr (VISC) {
+        ux = ix * at1(S, 5, c, 1);
+        vy = iy * at1(S, 6, c, PX);
+        e[6] = ux + vy;
+        e[7] = ix * at1(S, 7, c, 1);
+        e[8] = iy * at1(S, 7, c, PX);
+      }
+      if (zp >= z0 && zp < z1) {
+        double* r = rr[2];
+#pragma unroll
+        for (int m = 0; m < NV; ++m) r[m] = 0.0;
+        const double q0[NV] = {e[0], e[1], e[2], e[3], e[4]};
+        const double u0 = S[c][5], u1 = S[c][6];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int st = j == 0 ? 1 : PX;
+          auto off = [&](int s) { return c + (s < 2 ? s - 2 : s - 1) * st; };
+          convect(
+              j, j == 0 ? ix : iy, [&](int s, int m) { return S[off(s)][m]; },
+              [&](int s) { return S[off(s)][5 + j]; }, [&](int s) { return S[off(s)][8]; }, q0, j == 0 ? u0 : u1, r);
+          settle(r);
+        }
+        if constexpr (VISC) {
+          const double u2 = S[c][7];
+          auto mixed = [&](int f) {  // D_y(D_x f)
+            return ix * iy *
+                   d1(at1(S, f, c - 2 * PX, 1), at1(S, f, c - PX, 1), at1(S, f, c + PX, 1), at1(S, f, c + 2 * PX, 1));
+          };
+          const double xx = ix * ix, yy = iy * iy;
+          const double p0 = (4.0 / 3.0) * xx * at2(S, 5, c, 1) + yy * at2(S, 5, c, PX) + (1.0 / 3.0) * mixed(6);
+          double sh = iy * at1(S, 5, c, PX);
+          r[1] += ph.inv_re * p0;
+          r[4] += ph.inv_re * (u0 * p0 + 2.0 * (ux * ux + vy * vy));
+          asm volatile("" : "+v"(sh));
+          settle(r);
+          const double p1 = xx * at2(S, 6, c, 1) + (4.0 / 3.0) * yy * at2(S, 6, c, PX) + (1.0 / 3.0) * mixed(5);
+          sh += ix * at1(S, 6, c, 1);
+          r[2] += ph.inv_re * p1;
+          r[4] += ph.inv_re * (u1 * p1 + sh * sh);
+          settle(r);
+          const double p2 = xx * at2(S, 7, c, 1) + yy * at2(S, 7, c, PX);
+          r[3] += ph.inv_re * p2;
+          r[4] += ph.inv_re * (u2 * p2) + ph.cq * (xx * at2(S, 9, c, 1) + yy * at2(S, 9, c, PX));
+          settle(r);
+        }
+      }
+      if (z >= z0) {
+        double r[NV];
+#pragma unroll
+        for (int m = 0; m < NV; ++m) r[m] = rr[0][m];
+        const double* k0 = zq[2];
+        const double q0[NV] = {k0[0], k0[1], k0[2], k0[3], k0[4]};
+        // velocities and pressure of the column
+        double u[5][3], p[5];
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+          double ke = 0.0;
+#pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            u[s][m] = zq[s][1 + m] * zq[s][5];
+            ke += u[s][m] * zq[s][1 + m];
+          }
+          p[s] = ph.gm1 * (zq[s][4] - 0.5 * ke);
+        }
+        auto pl = [](int s) { return s < 2 ? s : s + 1; };
+        convect(
+            2, iz, [&](int s, int m) { return zq[pl(s)][m]; }, [&](int s) { return u[pl(s)][2]; },
+            [&](int s) { return p[pl(s)]; }, q0, u[2][2], r);
+        settle(r);
+        if constexpr (VISC) {
+          double T[5], du[3], ddu[3];
+#pragma unroll
+          for (int s = 0; s < 5; ++s) T[s] = cT * p[s] * zq[s][5];
+          const double zz = iz * iz;
+#pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            du[m] = iz * d1(u[0][m], u[1][m], u[3][m], u[4][m]);
+            ddu[m] = zz * d2(u[0][m], u[1][m], u[2][m], u[3][m], u[4][m]);
+          }
+          auto dz = [&](int i) { return iz * d1(zq[0][i], zq[1][i], zq[3][i], zq[4][i]); };
+          const double p0 = ddu[0] + (1.0 / 3.0) * dz(7);
+          const double p1 = ddu[1] + (1.0 / 3.0) * dz(8);
+          const double p2 = (4.0 / 3.0) * ddu[2] + (1.0 / 3.0) * dz(6);
+          const double div = k0[6] + du[2], sx = du[0] + k0[7], sy = du[1] + k0[8];
+          r[1] += ph.inv_re * p0;
+          r[2] += ph.inv_re * p1;
+          r[3] += ph.inv_re * p2;
+          r[4] += ph.inv_re * (u[2][0] * p0 + u[2][1] * p1 + u[2][2] * p2 + 2.0 * du[2] * du[2] -
+                               (2.0 / 3.0) * div * div + sx * sx + sy * sy) +
+                  ph.cq * zz * d2(T[0], T[1], T[2], T[3], T[4]);
+        }
+#pragma unroll
+        for (int m = 0; m < NV; ++m) {
+          if constexpr (MODE == 2) {
+            st_once(r[m], &R[m * g.fs + o], ph.nt);
+          } else if constexpr (MODE == 0) {
+            const double qo = first ? q0[m] : qa[m];
+            st_once(qo + ph.dt * cA * r[m], &Qn[m * g.fs + o], ph.nt);
+            st_once(qo + ph.dt * cB * r[m], &Qo[m * g.fs + o], ph.nt);
+          } else {
+            const double tmp = cA * qa[m] + ph.dt * r[m];
+            st_once(tmp, &Qo[m * g.fs + o], ph.nt);
+            st_once(q0[m] + cB * tmp, &Qn[m * g.fs + o], ph.nt);
+          }
+        }
+      }
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int e = 0; e < 7; ++e) zq[k][e] = zq[k + 1][e];
-      if (inside) col_entry(zq[4]);
-      if (z + 2 < z1) {  // planes up to z1 + 1 are read
-        fetch(z + 2);
-        fetch_col(z + 4);
+        for (int i = 0; i < NQ; ++i) zq[k][i] = zq[k + 1][i];
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        rr[0][m] = rr[1][m];
+        rr[1][m] = rr[2][m];
       }
+    }
+    if (more) {
+      store((zp + 1) & 1);  // (last read before the previous barrier)
       __syncthreads();
     }
   }
@@ -1045,7 +1067,7 @@ __global__ void __launch_bounds__(CNT, 2) k_conv3d(const double* __restrict__ Q,
 // The viscous kernels (one 512-thread block per CU, bound by their 104-130 KB
 // of LDS) take 64-plane segments from 512 blocks on: each segment stages four
 // planes beyond its own, and at 256^3 two rounds of 64 planes beat four of 32
-// (0.684 -> 0.673 ms for the central viscous + RK kernel).
+// (0.684 -> 0.673 ms for a viscous + RK kernel).
 static int tile_segment(const Grid& g, int tx, int ty, long long want, int start) {
   const long long tiles = (long long)((g.n[0] + tx - 1) / tx) * ((g.n[1] + ty - 1) / ty);
   int sz = start;
@@ -1053,26 +1075,56 @@ static int tile_segment(const Grid& g, int tx, int ty, long long want, int start
   return sz;
 }
 int visc3d_segment(const Grid& g) { return tile_segment(g, VTX, VTY, 512, 64); }
-int conv3d_segment(const Grid& g) { return tile_segment(g, CTX, CTY, 1024, 32); }
-long long conv3d_blocks(const Grid& g, int sz) {
-  return (long long)((g.n[0] + CTX - 1) / CTX) * ((g.n[1] + CTY - 1) / CTY) * ((g.n[2] + sz - 1) / sz);
+
+// Tile and z segment of k_central3d.  A segment stages four planes beyond its
+// own, and every plane costs a block about the same time whatever the others
+// do, so the launch takes rounds * (segment + overhead).  Measured (us, skew +
+// viscous): 64 x 8 tiles, one block per CU (144 KB of LDS), 4.9 per plane + 11
+// per segment; 32 x 8 tiles, two per CU, 5.3 and 12, or 3.5 and 10 while there
+// are no more blocks than CUs.  The cheapest of all is taken: 256^3 64 x 8 x
+// 128 (0.88 ms; 0.91 with 32 planes, 0.96 with 32-wide tiles), 128^3 64 x 8 x
+// 16 (113 us; 142 with 4), 24x30x40 32 x 8 x 2 (17 us; 21 with 64-wide tiles).
+void central3d_tiles(const Grid& g, int* tx, int* sz) {
+  double best = 1.0e300;
+  for (int w = 64; w >= 32; w -= 32) {
+    const long long tiles = (long long)((g.n[0] + w - 1) / w) * ((g.n[1] + 7) / 8);
+    for (int p = 2; p <= 256; ++p) {
+      const long long blocks = tiles * ((g.n[2] + p - 1) / p);
+      double t;
+      if (w == 64) t = (double)((blocks + 255) / 256) * (4.9 * p + 11.0);
+      else t = blocks <= 256 ? 3.5 * p + 10.0 : (double)((blocks + 511) / 512) * (5.3 * p + 12.0);
+      if (t < best) {
+        best = t;
+        *tx = w;
+        *sz = p;
+      }
+      if (p >= g.n[2]) break;
+    }
+  }
 }
 
-void launch_conv3d(int conv, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
-                   const Phys& ph, double cA, double cB, int first, int sz, hipStream_t s) {
-  dim3 grid((g.n[0] + CTX - 1) / CTX, (g.n[1] + CTY - 1) / CTY, (g.n[2] + sz - 1) / sz);
-  dim3 block(CTX, CTY);
-#define OSBL_CONV3D(C, M) k_conv3d<C, M><<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz)
-  if (conv == OSBL_CONV_CENTRAL_SKEW) {
-    if (mode == 0) OSBL_CONV3D(OSBL_CONV_CENTRAL_SKEW, 0);
-    else if (mode == 1) OSBL_CONV3D(OSBL_CONV_CENTRAL_SKEW, 1);
-    else OSBL_CONV3D(OSBL_CONV_CENTRAL_SKEW, 2);
-  } else {
-    if (mode == 0) OSBL_CONV3D(OSBL_CONV_CENTRAL_CONS, 0);
-    else if (mode == 1) OSBL_CONV3D(OSBL_CONV_CENTRAL_CONS, 1);
-    else OSBL_CONV3D(OSBL_CONV_CENTRAL_CONS, 2);
-  }
-#undef OSBL_CONV3D
+void launch_central3d(int conv, bool visc, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
+                      const Phys& ph, double cA, double cB, int first, int tx, int sz, int wrap, hipStream_t s) {
+  const dim3 grid((g.n[0] + tx - 1) / tx, (g.n[1] + 7) / 8, (g.n[2] + sz - 1) / sz), block(tx, 8);
+  auto go = [&](auto cc, auto vv, auto mm, auto xx, auto yy) {
+    k_central3d<decltype(cc)::value, decltype(vv)::value, decltype(mm)::value, decltype(xx)::value, decltype(yy)::value>
+        <<<grid, block, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, sz, wrap);
+  };
+  auto with_tile = [&](auto cc, auto vv, auto mm) {
+    if (tx == 64) go(cc, vv, mm, std::integral_constant<int, 64>{}, std::integral_constant<int, 8>{});
+    else go(cc, vv, mm, std::integral_constant<int, 32>{}, std::integral_constant<int, 8>{});
+  };
+  auto with_mode = [&](auto cc, auto vv) {
+    if (mode == 0) with_tile(cc, vv, std::integral_constant<int, 0>{});
+    else if (mode == 1) with_tile(cc, vv, std::integral_constant<int, 1>{});
+    else with_tile(cc, vv, std::integral_constant<int, 2>{});
+  };
+  auto with_visc = [&](auto cc) {
+    if (visc) with_mode(cc, std::true_type{});
+    else with_mode(cc, std::false_type{});
+  };
+  if (conv == OSBL_CONV_CENTRAL_SKEW) with_visc(std::integral_constant<int, OSBL_CONV_CENTRAL_SKEW>{});
+  else with_visc(std::integral_constant<int, OSBL_CONV_CENTRAL_CONS>{});
 }
 
 // interior <-> contiguous copies
@@ -1221,12 +1273,14 @@ static void launch_update_nd(int conv, bool visc, int mode, const double* Q, con
                              hipStream_t s) {
   const bool central = conv == OSBL_CONV_CENTRAL_SKEW || conv == OSBL_CONV_CENTRAL_CONS;
   if (central) {
+    if constexpr (ND < 3) {  // 3-D: k_central3d
     if (conv == OSBL_CONV_CENTRAL_SKEW) {
       if (visc) launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
       else launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
     } else {
       if (visc) launch_update_m<ND, OSBL_CONV_CENTRAL_CONS, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
       else launch_update_m<ND, OSBL_CONV_CENTRAL_CONS, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
+    }
     }
   } else {
     if (visc) launch_update_m<ND, OSBL_CONV_WENO_Z, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);

@@ -195,11 +195,12 @@ struct osbl_ctx {
   double A[5]{}, B[5]{};
   int seg = 32;
   int vsz = 32;             // z segment of the tiled viscous kernels
-  int csz = 32;             // z segment of the tiled central convective kernel
+  int ctx = 64, csz = 64;   // tile width and z segment of the tiled central kernel
   bool need_prims = false;
   bool tiled_visc = false;  // 3-D characteristic scheme with viscous terms
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
-  bool tiled_central = false;  // 3-D periodic central scheme: tiled convective kernel (+ tiled viscous kernel)
+  bool tiled_central = false;  // 3-D central scheme in one tiled kernel
+  bool haloless = false;    // its periodic images are read in place: no boundary pass in the time loop
   bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
   bool general = false;     // closures, metric or Sutherland viscosity: the general update kernel
   bool suth = false;
@@ -285,10 +286,14 @@ int bc_halos(const osbl_ctx* c, int side) {
   return central ? 2 : (side == 0 ? 3 : 4);
 }
 
+bool all_periodic(const osbl_ctx* c) {
+  bool p = true;
+  for (int d = 0; d < c->nd; ++d) p &= c->cfg.bc[d][0] == OSBL_BC_PERIODIC;
+  return p;
+}
+
 void apply_bcs(osbl_ctx* c, double* Q) {
-  bool all_periodic = true;
-  for (int d = 0; d < c->nd; ++d) all_periodic &= c->cfg.bc[d][0] == OSBL_BC_PERIODIC;
-  if (all_periodic) {
+  if (all_periodic(c)) {
     // one pass that gives every halo point its periodic image
     timed(c, F_BC, [&] { launch_halo_periodic(Q, c->nv, c->g, c->stream); });
     return;
@@ -312,6 +317,12 @@ void apply_bcs(osbl_ctx* c, double* Q) {
       }
     }
   }
+}
+
+// the boundary conditions of the time loop (none where the stages read their
+// periodic images in place; what reads halos itself calls apply_bcs)
+void loop_bcs(osbl_ctx* c) {
+  if (!c->haloless) apply_bcs(c, Qcur(c));
 }
 
 // spatial residual of the current state into R (characteristic part only),
@@ -353,17 +364,11 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
     return;
   }
   if (c->tiled_central) {
-    // 3-D central scheme: the tiled convective kernel applies the RK update,
-    // or, with viscous terms, assigns R and the tiled viscous kernel adds its
-    // terms and applies the update (mode 2: residual only, left in R)
-    const bool visc = c->cfg.viscous != OSBL_VISC_NONE;
+    // 3-D central scheme: everything in one kernel (mode 2: the residual, left in R)
     timed(c, F_CENTRAL, [&] {
-      launch_conv3d(conv, visc ? 2 : mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->csz, c->stream);
+      launch_central3d(conv, c->cfg.viscous != OSBL_VISC_NONE, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first,
+                       c->ctx, c->csz, all_periodic(c), c->stream);
     });
-    if (visc)
-      timed(c, F_UPDATE, [&] {
-        launch_visc_update3d(mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->vsz, c->stream);
-      });
     return;
   }
   if (c->tiled_visc && mode != 2) {
@@ -374,7 +379,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
       launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, c->Theta, false,
                    c->stream);
     });
-    timed(c, F_UPDATE, [&] { launch_visc_update3d(2, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->vsz, c->stream); });
+    timed(c, F_UPDATE, [&] { launch_visc_update3d(Q, c->R, c->g, c->ph, c->vsz, c->stream); });
     timed(c, F_SWEEP_Y, [&] {
       launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, c->Theta, true,
                    c->stream);
@@ -420,10 +425,8 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
       launch_update_gen(c->nd, conv, visc, mode, Q, c->P, c->R, c->Qo, Qn, c->g, c->ph, c->bnd, cA, cB, first,
                         c->suth ? 1 : 0, c->stream);
     });
-  } else if (c->tiled_visc) {
-    timed(c, F_UPDATE, [&] {
-      launch_visc_update3d(mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->vsz, c->stream);
-    });
+  } else if (c->tiled_visc) {  // mode 2
+    timed(c, F_UPDATE, [&] { launch_visc_update3d(Q, c->R, c->g, c->ph, c->vsz, c->stream); });
   } else {
     timed(c, F_UPDATE, [&] {
       launch_update(c->nd, conv, visc, mode, Q, c->P, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->stream);
@@ -622,13 +625,10 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->tiled_visc = !c->general && c->nd == 3 && !is_central(cfg->conv) && cfg->viscous != OSBL_VISC_NONE;
   c->tiled_gen = c->general && c->nd == 3 && !is_central(cfg->conv) && cfg->viscous != OSBL_VISC_NONE &&
                  !c->bnd.mod[2][0] && !c->bnd.mod[2][1] && !cfg->stretch[2];
-  // the tiled central kernels march columns along z in segments short
-  // enough to give the GPU ~1024 blocks; a grid with too few tiles even then
-  // (below ~32^3) keeps the per-point kernels
   c->vsz = visc3d_segment(c->g);
-  c->csz = conv3d_segment(c->g);
-  c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear &&
-                     conv3d_blocks(c->g, c->csz) >= 128;
+  c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear;
+  central3d_tiles(c->g, &c->ctx, &c->csz);
+  c->haloless = c->tiled_central && all_periodic(c) && !cfg->filters;
   c->line = c->nd == 1 && !is_central(cfg->conv) && cfg->viscous == OSBL_VISC_NONE && !stretched && !ph.has_force &&
             cfg->bc[0][0] == OSBL_BC_EXTRAP0 && cfg->bc[0][1] == OSBL_BC_EXTRAP0;
   c->need_prims = !c->tiled_central && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
@@ -884,7 +884,7 @@ static void iterate(osbl_ctx* c, int mode) {
     }
     stage(c, mode, c->A[s], c->B[s], s == 0);
     c->cur ^= 1;
-    apply_bcs(c, Qcur(c));
+    loop_bcs(c);
   }
   if (c->cfg.filters) filters(c);
 }
@@ -925,7 +925,7 @@ int osbl_run(osbl_ctx* c, int64_t niter) {
     }
     return OSBL_OK;
   }
-  if (niter > 0) apply_bcs(c, Qcur(c));
+  if (niter > 0) loop_bcs(c);
   if ((c->cfg.filters & OSBL_FILTER_SFD) && niter > 0) {
     // "Initialize the filter" before the time loop: vfilt = v (SFD.py:50-61)
     for (int m = 0; m < c->nv; ++m) {
@@ -1158,7 +1158,7 @@ int osbl_use_graphs(osbl_ctx* c, int enable) {
 int osbl_rhs(osbl_ctx* c, double* residual_host) {
   if (!c || !residual_host) return fail(OSBL_E_ARG, "null argument");
   if (int rc = check_ready(c)) return rc;
-  apply_bcs(c, Qcur(c));
+  loop_bcs(c);
   stage(c, 2, 0.0, 0.0, 0);
   HIPCHK(hipGetLastError());
   const long long n = cells(c);
@@ -1261,17 +1261,12 @@ int osbl_kernel_work(osbl_ctx* c, int family, double* bytes, double* flops) {
       f = (interface_flops(c) + (c->tiled_visc || c->tiled_gen ? 6.0 * nv : 0.0)) * n;
       break;
     case F_FILTER: b = 16.0 * nv * n; break;
-    case F_CENTRAL:
-      // read Q; write R (viscous terms follow) or read the register and write Q and the register
-      b = (c->cfg.viscous != OSBL_VISC_NONE ? 16.0 : 32.0) * nv * n;
-      f = (c->nd * central_flops(c) + (c->cfg.viscous != OSBL_VISC_NONE ? 0.0 : 6.0 * nv)) * n;
+    case F_CENTRAL:  // the whole stage of the tiled central scheme: read Q and the register, write both
+      b = 32.0 * nv * n;
+      f = (c->nd * central_flops(c) + viscous_flops(c) + 6.0 * nv) * n;
       break;
     case F_UPDATE: {
-      if (c->tiled_central) {  // viscous terms + RK update: read Q, R, the register; write Q and the register
-        b = 40.0 * nv * n;
-        f = (viscous_flops(c) + 6.0 * nv) * n;
-        break;
-      }
+      if (c->tiled_central) break;  // no kernel of its own
       if (c->tiled_visc || c->tiled_gen) {  // viscous terms only: read Q (or the CRs), RMW R
         b = 24.0 * nv * n;
         f = viscous_flops(c) * n;
@@ -1510,12 +1505,12 @@ int osbl_step_stages_dev(osbl_ctx* c, double* stages_dev) {
   if (!c || !stages_dev) return fail(OSBL_E_ARG, "null argument");
   const long long n = cells(c);
   const int mode = c->cfg.rk == OSBL_RK3 ? 0 : 1;
-  apply_bcs(c, Qcur(c));
+  loop_bcs(c);
   for (int s = 0; s < c->nstages; ++s) {
     launch_pack_all(Qcur(c), stages_dev + (long long)s * c->nv * n, c->g, c->nv, c->stream);
     stage(c, mode, c->A[s], c->B[s], s == 0);
     c->cur ^= 1;
-    apply_bcs(c, Qcur(c));
+    loop_bcs(c);
   }
   HIPCHK(hipGetLastError());
   return OSBL_OK;

@@ -30,7 +30,7 @@ FAMILIES = [
     ("k_char_vjp", "adjoint"),
     ("k_adj_", "adjoint"),
     ("k_visc_vjp", "adjoint"),
-    ("k_conv3d", "central_convective"),
+    ("k_central3d", "central_convective"),
     ("k_visc_update3d", "residual_rk_update"),
     ("k_visc_gen3d", "residual_rk_update"),
     ("k_visc_shell", "residual_rk_update"),

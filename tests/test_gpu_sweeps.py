@@ -57,3 +57,12 @@ def test_2d_shapes(n, conv, averaging, rk, bc, oracle):
 def test_3d_shapes(n, conv, oracle):
     problem, q0 = _block(n, conv, "periodic", viscous="const")
     _check(problem, q0, oracle, f"3-D {n} {conv}")
+
+
+@pytest.mark.parametrize("bc", ["periodic", "symmetry"])
+@pytest.mark.parametrize("conv,rk,viscous", [("central_skew", "ls3", "const"), ("central_skew", "rk3", "none"),
+                                             ("central_cons", "rk3", "const"), ("central_cons", "ls3", "none")])
+@pytest.mark.parametrize("n", [(8, 8, 8), (31, 9, 10), (33, 16, 11), (64, 8, 40), (65, 17, 9), (130, 12, 70)])
+def test_3d_central_shapes(n, conv, rk, viscous, bc, oracle):
+    problem, q0 = _block(n, conv, bc, rk=rk, viscous=viscous)
+    _check(problem, q0, oracle, f"3-D {n} {conv} {rk} {viscous} {bc}")
