@@ -798,7 +798,11 @@ void launch_visc_update3d(const double* Q, double* R, const Grid& g, const Phys&
 // the halos need not be filled between stages.
 //
 // The stage moves Q, the register and the new state once: 160 B per cell
-// against 280 for a convective kernel that leaves R to a viscous kernel.
+// against 280 for a convective kernel that leaves R to a viscous kernel.  What
+// bounds it now is a block's chain per plane (LDS reads, two waves per SIMD,
+// a barrier) and, at 256^3, HBM: 0.75 ms a stage, 3.6 TB/s of those 160 B;
+// the two kernels and the halo pass took 1.36 ms.  Reading a point's fields
+// two at a time (ds_read_b128) and adding up point by point took it from 0.88.
 //   MODE 0/1: RK update; MODE 2: the residual alone, into R.
 // ---------------------------------------------------------------------------
 template <int CONV, bool VISC, int MODE, int TX, int TY>
@@ -807,9 +811,11 @@ __global__ void __launch_bounds__(TX * TY, 2)
                 double* __restrict__ Qn, Grid g, Phys ph, double cA, double cB, int first, int sz, int wrap) {
   constexpr int NV = 5, PX = TX + 4, PY = TY + 4, PL = PX * PY, NT = TX * TY;
   constexpr int PP = (PL + NT - 1) / NT;     // staged points per thread and plane
-  constexpr int NF = VISC ? 11 : 9;          // Q0..Q4, u0, u1, u2, p (, T, pad): odd, no bank conflicts
+  constexpr int NF = 10;                     // Q0..Q4, p, u0, u1, u2, T
   constexpr int NQ = VISC ? 9 : 6;           // queue: Q0..Q4, 1/rho (, D_x u0 + D_y u1, D_x u2, D_y u2)
-  __shared__ double sp[2][PL][NF];
+  // a point's fields lie next to each other and are read two at a time: at a
+  // stride of 80 bytes 16 lanes' 16-byte reads cover the 64 banks once
+  __shared__ __align__(16) double sp[2][PL][NF];
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
   int bx, by, bz;
   xcd_tile(bx, by, bz);
@@ -850,11 +856,13 @@ __global__ void __launch_bounds__(TX * TY, 2)
         const double pr = ph.gm1 * (pq[k][4] - 0.5 * rho * (u0 * u0 + u1 * u1 + u2 * u2));
 #pragma unroll
         for (int m = 0; m < NV; ++m) sp[slot][pt][m] = pq[k][m];
-        sp[slot][pt][5] = u0;
-        sp[slot][pt][6] = u1;
-        sp[slot][pt][7] = u2;
-        sp[slot][pt][8] = pr;
-        if constexpr (VISC) sp[slot][pt][9] = cT * pr * ir;
+        sp[slot][pt][5] = pr;
+        sp[slot][pt][6] = u0;
+        sp[slot][pt][7] = u1;
+        if constexpr (VISC) {
+          sp[slot][pt][8] = u2;
+          sp[slot][pt][9] = cT * pr * ir;
+        }
       }
   };
   const int c = (ty + 2) * PX + tx + 2;  // this thread's column in a slot
@@ -864,14 +872,68 @@ __global__ void __launch_bounds__(TX * TY, 2)
   auto d2 = [](double fm2, double fm1, double f0, double fp1, double fp2) {
     return (-1.0 / 12.0) * (fm2 + fp2) + (4.0 / 3.0) * (fm1 + fp1) - 2.5 * f0;
   };
-  // derivatives of field f about the point `o` of a slot, along stride st
-  auto at1 = [&](const double (*S)[NF], int f, int o, int st) {
-    return d1(S[o - 2 * st][f], S[o - st][f], S[o + st][f], S[o + 2 * st][f]);
+  struct alignas(16) Two {
+    double a, b;
   };
-  auto at2 = [&](const double (*S)[NF], int f, int o, int st) {
-    return d2(S[o - 2 * st][f], S[o - st][f], S[o][f], S[o + st][f], S[o + 2 * st][f]);
+  // fields 2 i and 2 i + 1 of the point o of a slot
+  auto two = [](const double (*S)[NF], int o, int i) { return *reinterpret_cast<const Two*>(&S[o][2 * i]); };
+  // sums over the points -2, -1, 1, 2 of a direction: first differences of
+  // Q u_j, Q, p, p u_j, u_0..u_2 and second ones of u_0..u_2, T
+  struct Sums {
+    double qu[NV], q[NV], p, pu, u[3], uu[3], TT;
   };
-  // convective terms along one direction: values of Q_m, u_j, p at the
+  auto gather = [&](const double (*S)[NF], int j, int st) {
+    Sums a{};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int o = c + (s < 2 ? s - 2 : s - 1) * st;
+      const double w = s == 0 ? 1.0 / 12.0 : (s == 1 ? -2.0 / 3.0 : (s == 2 ? 2.0 / 3.0 : -1.0 / 12.0));
+      const double w2 = (s == 0 || s == 3) ? -1.0 / 12.0 : 4.0 / 3.0;
+      const Two f0 = two(S, o, 0), f1 = two(S, o, 1), f2 = two(S, o, 2), f3 = two(S, o, 3);
+      const double q[NV] = {f0.a, f0.b, f1.a, f1.b, f2.a}, p = f2.b;
+      const double uj = j == 0 ? f3.a : f3.b, wu = w * uj;
+      if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
+#pragma unroll
+        for (int m = 0; m < NV; ++m) {
+          a.qu[m] = __fma_rn(wu, q[m], a.qu[m]);
+          a.q[m] = __fma_rn(w, q[m], a.q[m]);
+        }
+      } else {
+        a.q[0] = __fma_rn(w, q[1 + j], a.q[0]);
+#pragma unroll
+        for (int m = 1; m < NV; ++m) a.qu[m] = __fma_rn(wu, q[m], a.qu[m]);
+      }
+      a.p = __fma_rn(w, p, a.p);
+      a.pu = __fma_rn(wu, p, a.pu);
+      if constexpr (VISC) {
+        const Two f4 = two(S, o, 4);
+        a.u[0] = __fma_rn(w, f3.a, a.u[0]);
+        a.u[1] = __fma_rn(w, f3.b, a.u[1]);
+        a.u[2] = __fma_rn(w, f4.a, a.u[2]);
+        a.uu[0] = __fma_rn(w2, f3.a, a.uu[0]);
+        a.uu[1] = __fma_rn(w2, f3.b, a.uu[1]);
+        a.uu[2] = __fma_rn(w2, f4.a, a.uu[2]);
+        a.TT = __fma_rn(w2, f4.b, a.TT);
+      } else {
+        a.u[j] = __fma_rn(w, uj, a.u[j]);
+      }
+    }
+    return a;
+  };
+  auto add_convect = [](const Sums& a, int j, double inv, const double (&q0)[NV], double u0, double* r) {
+    if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
+      const double hi = -0.5 * inv, hu = hi * u0, du = hi * a.u[j];
+#pragma unroll
+      for (int m = 0; m < NV; ++m) r[m] += hi * a.qu[m] + hu * a.q[m] + q0[m] * du;
+    } else {
+      r[0] -= inv * a.q[0];
+#pragma unroll
+      for (int m = 1; m < NV; ++m) r[m] -= inv * a.qu[m];
+    }
+    r[1 + j] -= inv * a.p;
+    r[4] -= inv * a.pu;
+  };
+  // convective terms along z: values of Q_m, u_j, p at the
   // offsets -2, -1, 1, 2 through fq, fu, fp; the cell's own Q and u_j
   auto convect = [&](int j, double inv, auto&& fq, auto&& fu, auto&& fp, const double (&q0)[NV], double u0, double* r) {
     double qv[4][NV], uv[4], pv[4];
@@ -935,55 +997,74 @@ __global__ void __launch_bounds__(TX * TY, 2)
     const double (*S)[NF] = sp[zp & 1];
     if (inside) {
       double* e = zq[4];
-#pragma unroll
-      for (int m = 0; m < NV; ++m) e[m] = S[c][m];
+      const Two f0 = two(S, c, 0), f1 = two(S, c, 1), f2 = two(S, c, 2), f3 = two(S, c, 3);
+      e[0] = f0.a;
+      e[1] = f0.b;
+      e[2] = f1.a;
+      e[3] = f1.b;
+      e[4] = f2.a;
       e[5] = recip_pos(e[0]);
-      [[maybe_unused]] double ux, vy;
-      if constexpr (VISC) {
-        ux = ix * at1(S, 5, c, 1);
-        vy = iy * at1(S, 6, c, PX);
-        e[6] = ux + vy;
-        e[7] = ix * at1(S, 7, c, 1);
-        e[8] = iy * at1(S, 7, c, PX);
-      }
       if (zp >= z0 && zp < z1) {
         double* r = rr[2];
 #pragma unroll
         for (int m = 0; m < NV; ++m) r[m] = 0.0;
         const double q0[NV] = {e[0], e[1], e[2], e[3], e[4]};
-        const double u0 = S[c][5], u1 = S[c][6];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int st = j == 0 ? 1 : PX;
-          auto off = [&](int s) { return c + (s < 2 ? s - 2 : s - 1) * st; };
-          convect(
-              j, j == 0 ? ix : iy, [&](int s, int m) { return S[off(s)][m]; },
-              [&](int s) { return S[off(s)][5 + j]; }, [&](int s) { return S[off(s)][8]; }, q0, j == 0 ? u0 : u1, r);
-          settle(r);
-        }
+        const Sums ax = gather(S, 0, 1);
+        add_convect(ax, 0, ix, q0, f3.a, r);
         if constexpr (VISC) {
-          const double u2 = S[c][7];
-          auto mixed = [&](int f) {  // D_y(D_x f)
-            return ix * iy *
-                   d1(at1(S, f, c - 2 * PX, 1), at1(S, f, c - PX, 1), at1(S, f, c + PX, 1), at1(S, f, c + 2 * PX, 1));
-          };
           const double xx = ix * ix, yy = iy * iy;
-          const double p0 = (4.0 / 3.0) * xx * at2(S, 5, c, 1) + yy * at2(S, 5, c, PX) + (1.0 / 3.0) * mixed(6);
-          double sh = iy * at1(S, 5, c, PX);
-          r[1] += ph.inv_re * p0;
-          r[4] += ph.inv_re * (u0 * p0 + 2.0 * (ux * ux + vy * vy));
-          asm volatile("" : "+v"(sh));
+          const Two f4 = two(S, c, 4);
+          // second derivatives and shears, x first
+          double p0 = (4.0 / 3.0) * xx * (ax.uu[0] - 2.5 * f3.a), p1 = xx * (ax.uu[1] - 2.5 * f3.b);
+          double p2 = xx * (ax.uu[2] - 2.5 * f4.a), TT = xx * (ax.TT - 2.5 * f4.b);
+          double ux = ix * ax.u[0], sh = ix * ax.u[1];
+          e[7] = ix * ax.u[2];
+          asm volatile("" : "+v"(p0), "+v"(p1), "+v"(p2), "+v"(TT), "+v"(ux), "+v"(sh), "+v"(e[7]));
           settle(r);
-          const double p1 = xx * at2(S, 6, c, 1) + (4.0 / 3.0) * yy * at2(S, 6, c, PX) + (1.0 / 3.0) * mixed(5);
-          sh += ix * at1(S, 6, c, 1);
-          r[2] += ph.inv_re * p1;
-          r[4] += ph.inv_re * (u1 * p1 + sh * sh);
-          settle(r);
-          const double p2 = xx * at2(S, 7, c, 1) + yy * at2(S, 7, c, PX);
+          const Sums ay = gather(S, 1, PX);
+          add_convect(ay, 1, iy, q0, f3.b, r);
+          p0 += yy * (ay.uu[0] - 2.5 * f3.a);
+          p1 += (4.0 / 3.0) * yy * (ay.uu[1] - 2.5 * f3.b);
+          p2 += yy * (ay.uu[2] - 2.5 * f4.a);
+          TT += yy * (ay.TT - 2.5 * f4.b);
+          const double vy = iy * ay.u[1];
+          sh += iy * ay.u[0];
+          e[6] = ux + vy;
+          e[8] = iy * ay.u[2];
           r[3] += ph.inv_re * p2;
-          r[4] += ph.inv_re * (u2 * p2) + ph.cq * (xx * at2(S, 9, c, 1) + yy * at2(S, 9, c, PX));
+          r[4] += ph.inv_re * (f4.a * p2 + 2.0 * (ux * ux + vy * vy) + sh * sh) + ph.cq * TT;
+          asm volatile("" : "+v"(p0), "+v"(p1), "+v"(e[6]), "+v"(e[8]));
+          settle(r);
+          // D_y(D_x u_1) and D_y(D_x u_0)
+          double m0 = 0.0, m1 = 0.0;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const int o = c + (s < 2 ? s - 2 : s - 1) * PX;
+            const double w = s == 0 ? 1.0 / 12.0 : (s == 1 ? -2.0 / 3.0 : (s == 2 ? 2.0 / 3.0 : -1.0 / 12.0));
+            const Two a = two(S, o - 2, 3), b = two(S, o - 1, 3), d = two(S, o + 1, 3), f = two(S, o + 2, 3);
+            m0 = __fma_rn(w, d1(a.a, b.a, d.a, f.a), m0);
+            m1 = __fma_rn(w, d1(a.b, b.b, d.b, f.b), m1);
+          }
+          const double k = (1.0 / 3.0) * ix * iy;
+          p0 += k * m1;
+          p1 += k * m0;
+          r[1] += ph.inv_re * p0;
+          r[2] += ph.inv_re * p1;
+          r[4] += ph.inv_re * (f3.a * p0 + f3.b * p1);
+          settle(r);
+        } else {
+          settle(r);
+          add_convect(gather(S, 1, PX), 1, iy, q0, f3.b, r);
           settle(r);
         }
+      } else if constexpr (VISC) {
+        // a plane that only the z stencils read
+        auto at1 = [&](int f, int st) {
+          return d1(S[c - 2 * st][f], S[c - st][f], S[c + st][f], S[c + 2 * st][f]);
+        };
+        e[6] = ix * at1(6, 1) + iy * at1(7, PX);
+        e[7] = ix * at1(8, 1);
+        e[8] = iy * at1(8, PX);
       }
       if (z >= z0) {
         double r[NV];
@@ -1079,11 +1160,11 @@ int visc3d_segment(const Grid& g) { return tile_segment(g, VTX, VTY, 512, 64); }
 // Tile and z segment of k_central3d.  A segment stages four planes beyond its
 // own, and every plane costs a block about the same time whatever the others
 // do, so the launch takes rounds * (segment + overhead).  Measured (us, skew +
-// viscous): 64 x 8 tiles, one block per CU (144 KB of LDS), 4.9 per plane + 11
-// per segment; 32 x 8 tiles, two per CU, 5.3 and 12, or 3.5 and 10 while there
+// viscous): 64 x 8 tiles, one block per CU (131 KB of LDS), 4.0 per plane + 10
+// per segment; 32 x 8 tiles, two per CU, 4.2 and 9, or 3.05 and 8 while there
 // are no more blocks than CUs.  The cheapest of all is taken: 256^3 64 x 8 x
-// 128 (0.88 ms; 0.91 with 32 planes, 0.96 with 32-wide tiles), 128^3 64 x 8 x
-// 16 (113 us; 142 with 4), 24x30x40 32 x 8 x 2 (17 us; 21 with 64-wide tiles).
+// 128 (0.75 ms; 0.78 with 32 planes), 128^3 about 91 us (101 with 64 x 8 x 8),
+// 24x30x40 32 x 8 x 2 (14 us; 18 with 64-wide tiles).
 void central3d_tiles(const Grid& g, int* tx, int* sz) {
   double best = 1.0e300;
   for (int w = 64; w >= 32; w -= 32) {
@@ -1091,8 +1172,8 @@ void central3d_tiles(const Grid& g, int* tx, int* sz) {
     for (int p = 2; p <= 256; ++p) {
       const long long blocks = tiles * ((g.n[2] + p - 1) / p);
       double t;
-      if (w == 64) t = (double)((blocks + 255) / 256) * (4.9 * p + 11.0);
-      else t = blocks <= 256 ? 3.5 * p + 10.0 : (double)((blocks + 511) / 512) * (5.3 * p + 12.0);
+      if (w == 64) t = (double)((blocks + 255) / 256) * (4.0 * p + 10.0);
+      else t = blocks <= 256 ? 3.05 * p + 8.0 : (double)((blocks + 511) / 512) * (4.2 * p + 9.0);
       if (t < best) {
         best = t;
         *tx = w;
