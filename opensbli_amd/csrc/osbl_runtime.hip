@@ -200,7 +200,8 @@ struct osbl_ctx {
   bool tiled_visc = false;  // 3-D characteristic scheme with viscous terms
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
   bool tiled_central = false;  // 3-D central scheme in one tiled kernel
-  bool haloless = false;    // its periodic images are read in place: no boundary pass in the time loop
+  bool plain2d = false;     // 2-D characteristic Euler block: the whole stage in one tiled kernel
+  bool haloless = false;    // periodic blocks of these two: read in place, no boundary pass in the time loop
   bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
   bool general = false;     // closures, metric or Sutherland viscosity: the general update kernel
   bool suth = false;
@@ -411,7 +412,13 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
     });
     return;
   }
-  if (!is_central(conv)) {
+  if (!is_central(conv) && c->nd == 2) {
+    timed(c, F_SWEEP_X, [&] {
+      launch_char_tile2d(conv, c->cfg.averaging, c->plain2d ? mode : 2, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB,
+                         first, c->bnd.dm[0], c->bnd.dm[1], c->Theta, c->haloless ? 1 : 0, c->stream);
+    });
+    if (c->plain2d) return;
+  } else if (!is_central(conv)) {
     for (int d = 0; d < c->nd; ++d) {
       timed(c, F_SWEEP_X + d, [&] {
         launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], c->Theta, d > 0,
@@ -628,7 +635,9 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->vsz = visc3d_segment(c->g);
   c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear;
   central3d_tiles(c->g, &c->ctx, &c->csz);
-  c->haloless = c->tiled_central && all_periodic(c) && !cfg->filters;
+  c->plain2d = c->nd == 2 && !is_central(cfg->conv) && !cfg->curvilinear && cfg->viscous == OSBL_VISC_NONE &&
+               !ph.has_force;
+  c->haloless = (c->tiled_central || c->plain2d) && all_periodic(c) && !cfg->filters && !cfg->sensor;
   c->line = c->nd == 1 && !is_central(cfg->conv) && cfg->viscous == OSBL_VISC_NONE && !stretched && !ph.has_force &&
             cfg->bc[0][0] == OSBL_BC_EXTRAP0 && cfg->bc[0][1] == OSBL_BC_EXTRAP0;
   c->need_prims = !c->tiled_central && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
@@ -847,7 +856,13 @@ static void filters(osbl_ctx* c) {
     double* Q = Qcur(c);
     const bool ducros = c->cfg.wf_sensor == OSBL_WF_DUCROS;
     if (ducros) timed(c, F_FILTER, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
-    for (int d = 0; d < c->nd; ++d) {
+    if (c->nd == 2) {
+      timed(c, F_FILTER, [&] {
+        launch_char_tile2d(CONV_WFILTER, OSBL_AVG_SIMPLE, 2, Q, c->R, nullptr, nullptr, c->g, c->ph, 0.0, 0.0, 0,
+                           c->bnd.dm[0], c->bnd.dm[1], nullptr, 0, c->stream);
+      });
+    }
+    for (int d = 0; d < c->nd && c->nd == 3; ++d) {
       timed(c, F_FILTER, [&] {
         launch_sweep(c->nd, d, CONV_WFILTER, OSBL_AVG_SIMPLE, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], nullptr,
                      d > 0, c->stream);
@@ -1253,7 +1268,11 @@ int osbl_kernel_work(osbl_ctx* c, int family, double* bytes, double* flops) {
   switch (family) {
     case F_BC: b = 16.0 * nv * (double)halo_points(c->g); break;
     case F_PRIMS: b = 8.0 * (nv + c->nd + 2) * n; f = 6.0 * nv * n; break;
-    case F_SWEEP_X: b = 16.0 * nv * n; f = interface_flops(c) * n; break;
+    case F_SWEEP_X:
+      // 2-D: both directions, with the RK update on Euler blocks
+      b = (c->plain2d ? 32.0 : 16.0) * nv * n;
+      f = (c->nd == 2 && !c->curv ? 2.0 * interface_flops(c) + (c->plain2d ? 6.0 * nv : 0.0) : interface_flops(c)) * n;
+      break;
     case F_SWEEP_Y: b = 24.0 * nv * n; f = interface_flops(c) * n; break;
     case F_SWEEP_Z:
       // with the fused RK update: read Q, R and the register, write Q and the register
