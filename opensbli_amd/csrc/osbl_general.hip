@@ -11,6 +11,7 @@
 // fused with the RK update.  The characteristic fluxes come from the sweeps of
 // osbl_kernels.hip, which apply the metric to their flux differences.
 #include "osbl_kernels.h"
+#include "osbl_visc.h"
 
 namespace osbl {
 
@@ -70,12 +71,6 @@ __device__ __forceinline__ double dxi(const Bnd& b, int d, int c, int N, int x, 
 // computational coordinates and transformed on stretched directions:
 // D_j -> G_j D, D_jj -> G_j^2 D2 + G_j S_j D, D_a D_b -> G_a G_b D_b(D_a).
 // P holds u_0..u_{ND-1}, p, T, mu.
-template <int ND>
-__device__ __forceinline__ void viscous_assemble(double mu, const double um_[3], const double (&DU)[ND][ND],
-                                                 const double (&DD)[ND][ND][ND], const double (&D2T)[ND],
-                                                 const double (&DT)[ND], const double (&DMU)[ND], const Phys& ph,
-                                                 bool suth, double vr[ND + 2]);
-
 template <int ND>
 __device__ __forceinline__ void viscous_gen(const double* __restrict__ P, long long fs, int x, const int st[3],
                                             const int ci[3], const Grid& g, const Bnd& b, const Phys& ph, bool suth,
@@ -143,52 +138,6 @@ __device__ __forceinline__ void viscous_gen(const double* __restrict__ P, long l
   }
   const double um[3] = {U[0][x], ND > 1 ? U[1][x] : 0.0, ND > 2 ? U[2][x] : 0.0};
   viscous_assemble<ND>(suth ? MU[x] : 1.0, um, DU, DD, D2T, DT, DMU, ph, suth, vr);
-}
-
-// The viscous residual from the transformed derivatives at a point (the
-// second half of viscous_gen, shared with the tiled kernel).
-template <int ND>
-__device__ __forceinline__ void viscous_assemble(double mu, const double um_[3], const double (&DU)[ND][ND],
-                                                 const double (&DD)[ND][ND][ND], const double (&D2T)[ND],
-                                                 const double (&DT)[ND], const double (&DMU)[ND], const Phys& ph,
-                                                 bool suth, double vr[ND + 2]) {
-  double divu = 0.0;
-#pragma unroll
-  for (int k = 0; k < ND; ++k) divu += DU[k][k];
-  double energy = 0.0;
-#pragma unroll
-  for (int j = 0; j < ND; ++j) {
-    if (suth) energy += ph.cq * (mu * D2T[j] + DMU[j] * DT[j]);
-    else energy += ph.cq * D2T[j];
-  }
-#pragma unroll
-  for (int m = 0; m < ND; ++m) {
-    const double um = um_[m];
-    double visc = 0.0;
-#pragma unroll
-    for (int j = 0; j < ND; ++j) {
-      double tt = DD[m][j][j] + DD[j][m][j];
-      if (j == m) {
-        double sk = 0.0;
-#pragma unroll
-        for (int k = 0; k < ND; ++k) sk += DD[k][m][k];
-        tt -= (2.0 / 3.0) * sk;
-      }
-      const double sr = DU[m][j] + DU[j][m] - (j == m ? (2.0 / 3.0) * divu : 0.0);
-      double dtau, tau;
-      if (suth) {
-        dtau = ph.inv_re * mu * tt + ph.inv_re * DMU[j] * sr;
-        tau = ph.inv_re * mu * sr;
-      } else {
-        dtau = ph.inv_re * tt;
-        tau = ph.inv_re * sr;
-      }
-      visc += dtau;
-      energy += DU[m][j] * tau + um * dtau;
-    }
-    vr[1 + m] += visc;
-  }
-  vr[ND + 1] += energy;
 }
 
 // Central convective terms with the closures and metric: the skew form
@@ -749,7 +698,7 @@ static void launch_gen_nd(int conv, bool visc, const double* Q, const double* P,
   } else if (conv == OSBL_CONV_CENTRAL_CONS) {
     if (visc) launch_gen_t<ND, OSBL_CONV_CENTRAL_CONS, true>(Q, P, R, Qo, Qn, g, ph, b, cA, cB, first, mode, suth, s);
     else launch_gen_t<ND, OSBL_CONV_CENTRAL_CONS, false>(Q, P, R, Qo, Qn, g, ph, b, cA, cB, first, mode, suth, s);
-  } else {
+  } else if constexpr (ND != 2) {  // 2-D: k_char_tile2d
     if (visc) launch_gen_t<ND, OSBL_CONV_WENO_Z, true>(Q, P, R, Qo, Qn, g, ph, b, cA, cB, first, mode, suth, s);
     else launch_gen_t<ND, OSBL_CONV_WENO_Z, false>(Q, P, R, Qo, Qn, g, ph, b, cA, cB, first, mode, suth, s);
   }

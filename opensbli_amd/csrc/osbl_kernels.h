@@ -10,11 +10,13 @@ void launch_extrap0(double* Q, int nv, const Grid& g, int d, int side, hipStream
 void launch_prims(int nd, const double* Q, double* P, const Grid& g, const Phys& ph, hipStream_t s);
 void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
                   const double* met, const double* theta, bool acc, hipStream_t s);
-// both sweeps of a 2-D block (mode 0/1: with the RK update; 2: assigned to R);
-// wrap: periodic in both directions, halos not read
-void launch_char_tile2d(int conv, int avg, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
-                        const Phys& ph, double cA, double cB, int first, const double* met0, const double* met1,
-                        const double* theta, int wrap, hipStream_t s);
+// one stage of a 2-D characteristic block (osbl_tile2d.hip); theta: the
+// adaptive TENO's sensor is formed and left there; wrap: periodic in both
+// directions, halos not read.  conv CONV_WFILTER, mode 2: the WENO filter's
+// flux differences into R
+void launch_char_tile2d(int conv, int avg, int mode, bool visc, const double* Q, double* R, double* Qo, double* Qn,
+                        const Grid& g, const Phys& ph, const Bnd& b, double cA, double cB, int first, double* theta,
+                        int suth, int wrap, hipStream_t s);
 void launch_sweep_z_rk(int conv, int avg, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
                        const Phys& ph, int seg, const double* theta, double cA, double cB, int first, hipStream_t s);
 void launch_sensor(int nd, const double* Q, double* theta, const Grid& g, const Phys& ph, const Bnd& b, hipStream_t s);

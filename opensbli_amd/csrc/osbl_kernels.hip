@@ -374,116 +374,6 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
 }
 
 // ---------------------------------------------------------------------------
-// Both characteristic sweeps of a 2-D block in one kernel, for MODE 0/1 with
-// the RK update (MODE as k_update; MODE 2 assigns the flux differences to R).
-// A workgroup takes 15 x 15 cells: the points around them are staged in LDS
-// with their constituent relations once for both directions; thread (i, j)
-// evaluates the flux left of cell i in row j (x) and below cell j in column
-// i - 1 (y), 16 interfaces per 15 cells, and finishes cell (i - 1, j): its
-// left flux comes from the lane below, its upper one through LDS.  The
-// residual stays in registers.
-//
-// wrap: periodic in both directions, points are read at their periodic images
-// and the halos need not be filled.  met0, met1: D_dd of stretched directions.
-// ---------------------------------------------------------------------------
-constexpr int T2C = 15, T2P = T2C + 6;  // cells and staged points per side
-
-template <int CONV, int AVG, int MODE>
-__global__ void __launch_bounds__(256, 3) k_char_tile2d(const double* __restrict__ Q, double* __restrict__ R,
-                                                        double* __restrict__ Qo, double* __restrict__ Qn, Grid g,
-                                                        Phys ph, double cA, double cB, int first,
-                                                        const double* __restrict__ met0,
-                                                        const double* __restrict__ met1,
-                                                        const double* __restrict__ theta, int wrap) {
-  constexpr int ND = 2, NV = 4;
-  constexpr bool ROE = AVG == OSBL_AVG_ROE;
-  constexpr int NF = NV + ND + 2 + (ROE ? 2 : 0);  // q, u, p, a (, sqrt(rho), sqrt(rho) H)
-  constexpr int NS = NF | 1;                       // odd stride: no bank conflicts along x
-  __shared__ double S[T2P * T2P][NS];
-  __shared__ double Fy[NV][256];
-  const int t = threadIdx.x, i = t & 15, j = t >> 4;
-  const int x0 = blockIdx.x * T2C, y0 = blockIdx.y * T2C;
-  auto image = [&](int a, int n) { return !wrap ? a : (a < 0 ? a + n : (a >= n ? a - n : a)); };
-  // point (px, py) of the tile is (x0 - 3 + px, y0 - 3 + py); those beyond
-  // the block's reach (n + 2) feed no cell
-  double nq[2][NV];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int p = min(t + 256 * k, T2P * T2P - 1);
-    const int gx = min(x0 - 3 + p % T2P, g.n[0] + 2), gy = min(y0 - 3 + p / T2P, g.n[1] + 2);
-    fetch_q<ND>(nq[k], Q, g.fs, g.idx(image(gx, g.n[0]), image(gy, g.n[1]), 0));
-  }
-  const int cx = x0 + i - 1, cy = y0 + j;
-  const int x = g.idx(cx, cy, 0);
-  const bool own = i > 0 && j < T2C && cx < g.n[0] && cy < g.n[1];
-  [[maybe_unused]] double qo[NV] = {0.0, 0.0, 0.0, 0.0};
-  if constexpr (MODE != 2)
-    if (own && !(MODE == 0 ? first : cA == 0.0)) {
-#pragma unroll
-      for (int m = 0; m < NV; ++m) qo[m] = Qo[m * g.fs + x];
-    }
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int p = t + 256 * k;
-    Pt<ND> s;
-#pragma unroll
-    for (int m = 0; m < NV; ++m) s.q[m] = nq[k][m];
-    finish_pt<ND>(s, ph);
-    double sq = 0.0, h = 0.0;
-    if constexpr (ROE) roe_factors<ND>(s, sq, h);
-    if (p < T2P * T2P) {
-#pragma unroll
-      for (int m = 0; m < NV; ++m) S[p][m] = s.q[m];
-      S[p][4] = s.u[0];
-      S[p][5] = s.u[1];
-      S[p][6] = s.p;
-      S[p][7] = s.a;
-      if constexpr (ROE) {
-        S[p][8] = sq;
-        S[p][9] = h;
-      }
-    }
-  }
-  __syncthreads();
-  auto flux = [&](auto dc, int p0, int left, double (&fh)[NV]) {
-    constexpr int D = decltype(dc)::value, ST = D == 0 ? NS : T2P * NS, PS = D == 0 ? 1 : T2P;
-    [[maybe_unused]] RoeF rf{};
-    if constexpr (ROE) rf = RoeF{S[p0 + 2 * PS][8], S[p0 + 2 * PS][9], S[p0 + 3 * PS][8], S[p0 + 3 * PS][9]};
-    const double ct = theta ? adaptive_ct(theta[left], ph) : ph.teno_ct;
-    char_flux_w<ND, D, CONV, AVG, true>(LdsPoints<ND, ST>{S[p0]}, ph, fh, ct, rf);
-  };
-  // the sensor at the left point of an interface, kept on the block
-  auto at = [&](int a, int b) { return g.idx(min(a, g.n[0]), min(b, g.n[1]), 0); };
-  double r[NV], f[NV];
-  flux(std::integral_constant<int, 0>{}, min(j, T2C - 1) * T2P + 3 * T2P + i, at(x0 + i - 1, y0 + min(j, T2C - 1)), f);
-  const double g0 = met0 && own ? ph.inv_delta[0] * met0[cx] : ph.inv_delta[0];
-#pragma unroll
-  for (int m = 0; m < NV; ++m) r[m] = (__shfl_up(f[m], 1) - f[m]) * g0;
-  flux(std::integral_constant<int, 1>{}, j * T2P + max(i, 1) + 2, at(x0 + max(i, 1) - 1, y0 + j - 1), f);
-#pragma unroll
-  for (int m = 0; m < NV; ++m) Fy[m][t] = f[m];
-  __syncthreads();
-  if (!own) return;
-  const double g1 = met1 ? ph.inv_delta[1] * met1[cy] : ph.inv_delta[1];
-  const int pc = (j + 3) * T2P + i + 2;
-#pragma unroll
-  for (int m = 0; m < NV; ++m) {
-    r[m] = __fma_rn(f[m] - Fy[m][t + 16], g1, r[m]);
-    if constexpr (MODE == 2) {
-      R[m * g.fs + x] = r[m];
-    } else if constexpr (MODE == 0) {
-      const double o = first ? S[pc][m] : qo[m];
-      Qn[m * g.fs + x] = __fma_rn(ph.dt * cA, r[m], o);
-      Qo[m * g.fs + x] = __fma_rn(ph.dt * cB, r[m], o);
-    } else {
-      const double tmp = __fma_rn(ph.dt, r[m], cA * qo[m]);
-      Qo[m * g.fs + x] = tmp;
-      Qn[m * g.fs + x] = __fma_rn(cB, tmp, S[pc][m]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Central fourth-order stencils (scheme.py:81-85): D1 weights
 // [1/12, -2/3, 0, 2/3, -1/12], D2 weights [-1/12, 4/3, -5/2, 4/3, -1/12].
 // ---------------------------------------------------------------------------
@@ -1443,36 +1333,6 @@ void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, 
     else launch_sweep_conv<3, 2>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
   } else {
     launch_sweep_conv<1, 0>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
-  }
-}
-
-void launch_char_tile2d(int conv, int avg, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
-                        const Phys& ph, double cA, double cB, int first, const double* met0, const double* met1,
-                        const double* theta, int wrap, hipStream_t s) {
-  const dim3 grid((g.n[0] + T2C - 1) / T2C, (g.n[1] + T2C - 1) / T2C);
-  auto go = [&](auto cc, auto aa, auto mm) {
-    k_char_tile2d<decltype(cc)::value, decltype(aa)::value, decltype(mm)::value>
-        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, met0, met1, theta, wrap);
-  };
-  if (conv == CONV_WFILTER) {  // SimpleAverage (WENO_filter.py:324)
-    go(std::integral_constant<int, CONV_WFILTER>{}, std::integral_constant<int, OSBL_AVG_SIMPLE>{},
-       std::integral_constant<int, 2>{});
-    return;
-  }
-  auto with_mode = [&](auto cc, auto aa) {
-    if (mode == 0) go(cc, aa, std::integral_constant<int, 0>{});
-    else if (mode == 1) go(cc, aa, std::integral_constant<int, 1>{});
-    else go(cc, aa, std::integral_constant<int, 2>{});
-  };
-  auto with_avg = [&](auto cc) {
-    if (avg == OSBL_AVG_ROE) with_mode(cc, std::integral_constant<int, OSBL_AVG_ROE>{});
-    else with_mode(cc, std::integral_constant<int, OSBL_AVG_SIMPLE>{});
-  };
-  switch (conv) {
-    case OSBL_CONV_WENO_JS: with_avg(std::integral_constant<int, OSBL_CONV_WENO_JS>{}); break;
-    case OSBL_CONV_WENO_Z: with_avg(std::integral_constant<int, OSBL_CONV_WENO_Z>{}); break;
-    case OSBL_CONV_TENO5: with_avg(std::integral_constant<int, OSBL_CONV_TENO5>{}); break;
-    default: with_avg(std::integral_constant<int, OSBL_CONV_TENO6>{}); break;
   }
 }
 

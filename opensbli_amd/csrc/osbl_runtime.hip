@@ -200,7 +200,7 @@ struct osbl_ctx {
   bool tiled_visc = false;  // 3-D characteristic scheme with viscous terms
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
   bool tiled_central = false;  // 3-D central scheme in one tiled kernel
-  bool plain2d = false;     // 2-D characteristic Euler block: the whole stage in one tiled kernel
+  bool tiled2d = false;     // 2-D characteristic block: the whole stage in one tiled kernel
   bool haloless = false;    // periodic blocks of these two: read in place, no boundary pass in the time loop
   bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
   bool general = false;     // closures, metric or Sutherland viscosity: the general update kernel
@@ -332,6 +332,16 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
   double* Q = Qcur(c);
   double* Qn = c->Qbuf[1 - c->cur];
   const int conv = c->cfg.conv;
+  if (c->tiled2d) {
+    // (the kernel forms the adaptive TENO's sensor; the WENO filter's on another scheme here)
+    if (c->Theta && conv != OSBL_CONV_TENO5 && conv != OSBL_CONV_TENO6)
+      timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
+    timed(c, F_SWEEP_X, [&] {
+      launch_char_tile2d(conv, c->cfg.averaging, mode, c->cfg.viscous != OSBL_VISC_NONE, Q, c->R, c->Qo, Qn, c->g,
+                         c->ph, c->bnd, cA, cB, first, c->Theta, c->suth ? 1 : 0, c->haloless ? 1 : 0, c->stream);
+    });
+    return;
+  }
   if (c->need_prims) {
     // the tiled general schedule forms the constituent relations inside its
     // viscous kernel; only the near-face rows it leaves to k_visc_shell read P
@@ -412,13 +422,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
     });
     return;
   }
-  if (!is_central(conv) && c->nd == 2) {
-    timed(c, F_SWEEP_X, [&] {
-      launch_char_tile2d(conv, c->cfg.averaging, c->plain2d ? mode : 2, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB,
-                         first, c->bnd.dm[0], c->bnd.dm[1], c->Theta, c->haloless ? 1 : 0, c->stream);
-    });
-    if (c->plain2d) return;
-  } else if (!is_central(conv)) {
+  if (!is_central(conv)) {
     for (int d = 0; d < c->nd; ++d) {
       timed(c, F_SWEEP_X + d, [&] {
         launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], c->Theta, d > 0,
@@ -635,12 +639,11 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->vsz = visc3d_segment(c->g);
   c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear;
   central3d_tiles(c->g, &c->ctx, &c->csz);
-  c->plain2d = c->nd == 2 && !is_central(cfg->conv) && !cfg->curvilinear && cfg->viscous == OSBL_VISC_NONE &&
-               !ph.has_force;
-  c->haloless = (c->tiled_central || c->plain2d) && all_periodic(c) && !cfg->filters && !cfg->sensor;
+  c->tiled2d = c->nd == 2 && !is_central(cfg->conv) && !cfg->curvilinear;
+  c->haloless = (c->tiled_central || c->tiled2d) && all_periodic(c) && !cfg->filters;
   c->line = c->nd == 1 && !is_central(cfg->conv) && cfg->viscous == OSBL_VISC_NONE && !stretched && !ph.has_force &&
             cfg->bc[0][0] == OSBL_BC_EXTRAP0 && cfg->bc[0][1] == OSBL_BC_EXTRAP0;
-  c->need_prims = !c->tiled_central && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
+  c->need_prims = !c->tiled_central && !c->tiled2d && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   const size_t bundle = (size_t)fs * c->nv * sizeof(double);
   auto alloc = [&](double** p, size_t bytes) -> int {
@@ -858,8 +861,8 @@ static void filters(osbl_ctx* c) {
     if (ducros) timed(c, F_FILTER, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
     if (c->nd == 2) {
       timed(c, F_FILTER, [&] {
-        launch_char_tile2d(CONV_WFILTER, OSBL_AVG_SIMPLE, 2, Q, c->R, nullptr, nullptr, c->g, c->ph, 0.0, 0.0, 0,
-                           c->bnd.dm[0], c->bnd.dm[1], nullptr, 0, c->stream);
+        launch_char_tile2d(CONV_WFILTER, OSBL_AVG_SIMPLE, 2, false, Q, c->R, nullptr, nullptr, c->g, c->ph, c->bnd,
+                           0.0, 0.0, 0, nullptr, 0, 0, c->stream);
       });
     }
     for (int d = 0; d < c->nd && c->nd == 3; ++d) {
@@ -1269,9 +1272,9 @@ int osbl_kernel_work(osbl_ctx* c, int family, double* bytes, double* flops) {
     case F_BC: b = 16.0 * nv * (double)halo_points(c->g); break;
     case F_PRIMS: b = 8.0 * (nv + c->nd + 2) * n; f = 6.0 * nv * n; break;
     case F_SWEEP_X:
-      // 2-D: both directions, with the RK update on Euler blocks
-      b = (c->plain2d ? 32.0 : 16.0) * nv * n;
-      f = (c->nd == 2 && !c->curv ? 2.0 * interface_flops(c) + (c->plain2d ? 6.0 * nv : 0.0) : interface_flops(c)) * n;
+      // 2-D: the whole stage
+      b = (c->tiled2d ? 32.0 : 16.0) * nv * n;
+      f = (c->tiled2d ? 2.0 * interface_flops(c) + viscous_flops(c) + 6.0 * nv : interface_flops(c)) * n;
       break;
     case F_SWEEP_Y: b = 24.0 * nv * n; f = interface_flops(c) * n; break;
     case F_SWEEP_Z:
