@@ -19,21 +19,26 @@ __device__ __forceinline__ double t_cons(const double* __restrict__ Q, long long
 
 }  // namespace
 
-// One face: type OSBL_BC_* (not periodic, not zeroth-order extrapolation),
-// nh halo points filled, `st` the storage stride pointing inward, `plane` the
-// face's values [nv][n_e2][n_e1] (Dirichlet), Q2 the other state buffer
-// (inlet: its rhoE halos are kept equal to those of Q).
+// What a direction's two faces need: type OSBL_BC_*, halo points filled and
+// the face's values [nv][n_e2][n_e1] (Dirichlet) per side.
+struct BcSides {
+  int type[2], nh[2];
+  const double* plane[2];
+};
+
+// The line normal to face (d, side) through the face point (ia, ib) of the
+// other directions (halos included); `st` below is the storage stride pointing
+// inward, Q2 the other state buffer (inlet: its rhoE halos are kept equal to
+// those of Q).  A line touches its own face's points and halos only and reads
+// at most four points inward, so both faces of a direction (at least 8 points
+// apart) can be done at once.
 template <int ND>
-__global__ void __launch_bounds__(256) k_bc_face(double* __restrict__ Q, double* __restrict__ Q2, Grid g, Phys ph,
-                                                 int d, int side, int type, int nh, double twall,
-                                                 const double* __restrict__ plane) {
+__device__ __forceinline__ void bc_line(double* __restrict__ Q, double* __restrict__ Q2, const Grid& g,
+                                        const Phys& ph, int d, int side, int type, int nh, double twall,
+                                        const double* __restrict__ plane, int ia, int ib) {
   constexpr int NV = ND + 2;
   const int e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
-  const int n1 = g.n[e1] + 2 * g.h[e1], n2 = g.n[e2] + 2 * g.h[e2];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n1 * n2) return;
   int c[3];
-  const int ia = t % n1 - g.h[e1], ib = t / n1 - g.h[e2];
   c[e1] = ia;
   c[e2] = ib;
   c[d] = side == 0 ? 0 : g.n[d] - 1;
@@ -42,6 +47,16 @@ __global__ void __launch_bounds__(256) k_bc_face(double* __restrict__ Q, double*
   const long long fs = g.fs;
   const double gm = ph.gama, M2 = ph.Minf * ph.Minf;
   switch (type) {
+    case OSBL_BC_PERIODIC:  // periodic.py:42-56
+      for (int v = 0; v < NV; ++v)
+        for (int hh = 1; hh <= g.h[d]; ++hh) Q[v * fs + x - hh * st] = Q[v * fs + x + (g.n[d] - hh) * st];
+      break;
+    case OSBL_BC_EXTRAP0:  // boundary point and halos take the first point inside (extrapolation.py:29-58)
+      for (int v = 0; v < NV; ++v) {
+        const double s = Q[v * fs + x + st];
+        for (int hh = 0; hh <= g.h[d]; ++hh) Q[v * fs + x - hh * st] = s;
+      }
+      break;
     case OSBL_BC_EXTRAP1:  // halo i = 2 q[i-1] - q[i-2], outward (extrapolation.py:42-54)
       for (int v = 0; v < NV; ++v)
         for (int hh = 1; hh <= nh; ++hh)
@@ -141,6 +156,38 @@ __global__ void __launch_bounds__(256) k_bc_face(double* __restrict__ Q, double*
   }
 }
 
+// both faces of direction d
+template <int ND>
+__global__ void __launch_bounds__(256) k_bc_sides(double* __restrict__ Q, double* __restrict__ Q2, Grid g, Phys ph,
+                                                  int d, BcSides f, double twall) {
+  const int e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
+  const int n1 = g.n[e1] + 2 * g.h[e1], n2 = g.n[e2] + 2 * g.h[e2];
+  int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 2 * n1 * n2) return;
+  const int side = t >= n1 * n2;
+  t -= side * n1 * n2;
+  bc_line<ND>(Q, Q2, g, ph, d, side, f.type[side], f.nh[side], twall, f.plane[side], t % n1 - g.h[e1],
+              t / n1 - g.h[e2]);
+}
+
+// A 2-D block's four faces by one workgroup, direction 0 before direction 1
+// (block.py:199-210): the kernels per face of a 500x250 block take a launch
+// each for 500 threads of work (four of 4 to 7 us under the profiler; one now).
+__global__ void __launch_bounds__(1024) k_bc_block2d(double* __restrict__ Q, double* __restrict__ Q2, Grid g, Phys ph,
+                                                     BcSides f0, BcSides f1, double twall) {
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const BcSides& f = d == 0 ? f0 : f1;
+    const int n1 = g.n[1 - d] + 2 * g.h[1 - d];
+    for (int t = threadIdx.x; t < 2 * n1; t += 1024) {
+      const int side = t >= n1;
+      bc_line<2>(Q, Q2, g, ph, d, side, f.type[side], f.nh[side], twall, f.plane[side], t - side * n1 - g.h[1 - d],
+                 0);
+    }
+    __syncthreads();
+  }
+}
+
 // Periodic exchange of one direction over the full extents of the others
 // (periodic.py:42-56): halo points [-h, 0) and [N, N+h) take their images.
 __global__ void __launch_bounds__(256) k_periodic_dir(double* __restrict__ Q, int nv, Grid g, int d) {
@@ -185,14 +232,30 @@ __global__ void __launch_bounds__(256) k_fill_face_halo(double* __restrict__ Q, 
   }
 }
 
-void launch_bc_face(int nd, double* Q, double* Q2, const Grid& g, const Phys& ph, int d, int side, int type, int nh,
-                    double twall, const double* plane, hipStream_t s) {
+static BcSides bc_sides(const Grid& g, int d, const int type[2], const int nh[2], double* const plane[2]) {
+  BcSides f;
+  for (int s = 0; s < 2; ++s) {
+    f.type[s] = type[s];
+    f.nh[s] = nh[s] > g.h[d] ? g.h[d] : nh[s];
+    f.plane[s] = plane[s];
+  }
+  return f;
+}
+
+void launch_bc_sides(int nd, double* Q, double* Q2, const Grid& g, const Phys& ph, int d, const int type[2],
+                     const int nh[2], double twall, double* const plane[2], hipStream_t s) {
   const int e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
-  const int n = (g.n[e1] + 2 * g.h[e1]) * (g.n[e2] + 2 * g.h[e2]);
-  if (nh > g.h[d]) nh = g.h[d];
-  if (nd == 3) k_bc_face<3><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, side, type, nh, twall, plane);
-  else if (nd == 2) k_bc_face<2><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, side, type, nh, twall, plane);
-  else k_bc_face<1><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, side, type, nh, twall, plane);
+  const int n = 2 * (g.n[e1] + 2 * g.h[e1]) * (g.n[e2] + 2 * g.h[e2]);
+  const BcSides f = bc_sides(g, d, type, nh, plane);
+  if (nd == 3) k_bc_sides<3><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, f, twall);
+  else if (nd == 2) k_bc_sides<2><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, f, twall);
+  else k_bc_sides<1><<<(n + 255) / 256, 256, 0, s>>>(Q, Q2, g, ph, d, f, twall);
+}
+
+void launch_bc_block2d(double* Q, double* Q2, const Grid& g, const Phys& ph, const int (*type)[2], const int (*nh)[2],
+                       double twall, double* const (*plane)[2], hipStream_t s) {
+  k_bc_block2d<<<1, 1024, 0, s>>>(Q, Q2, g, ph, bc_sides(g, 0, type[0], nh[0], plane[0]),
+                                  bc_sides(g, 1, type[1], nh[1], plane[1]), twall);
 }
 
 void launch_periodic_dir(double* Q, int nv, const Grid& g, int d, hipStream_t s) {

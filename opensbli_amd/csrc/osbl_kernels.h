@@ -6,7 +6,6 @@
 namespace osbl {
 
 void launch_halo_periodic(double* Q, int nv, const Grid& g, hipStream_t s);
-void launch_extrap0(double* Q, int nv, const Grid& g, int d, int side, hipStream_t s);
 void launch_prims(int nd, const double* Q, double* P, const Grid& g, const Phys& ph, hipStream_t s);
 void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
                   const double* met, const double* theta, bool acc, hipStream_t s);
@@ -37,8 +36,11 @@ void launch_visc_gen3d(const double* Q, const double* P, double* R, const Grid& 
 void launch_body_force3d(const double* Q, double* R, const Grid& g, const Phys& ph, hipStream_t s);
 void launch_prims_slab(const double* Q, double* P, const Grid& g, const Phys& ph, int suth, hipStream_t s);
 void launch_prims_mu(int nd, const double* Q, double* P, const Grid& g, const Phys& ph, hipStream_t s);
-void launch_bc_face(int nd, double* Q, double* Q2, const Grid& g, const Phys& ph, int d, int side, int type, int nh,
-                    double twall, const double* plane, hipStream_t s);
+// the two faces of direction d; the four faces of a 2-D block in one workgroup
+void launch_bc_sides(int nd, double* Q, double* Q2, const Grid& g, const Phys& ph, int d, const int type[2],
+                     const int nh[2], double twall, double* const plane[2], hipStream_t s);
+void launch_bc_block2d(double* Q, double* Q2, const Grid& g, const Phys& ph, const int (*type)[2], const int (*nh)[2],
+                       double twall, double* const (*plane)[2], hipStream_t s);
 void launch_periodic_dir(double* Q, int nv, const Grid& g, int d, hipStream_t s);
 void launch_fill_face_halo(double* Q, int nv, const Grid& g, int d, int side, const double* plane, hipStream_t s);
 void launch_pack(const double* F, double* out, const Grid& g, hipStream_t s);

@@ -51,32 +51,6 @@ __global__ void __launch_bounds__(256) k_halo_periodic(double* __restrict__ Q, i
   for (int m = 0; m < nv; ++m) Q[m * g.fs + dst] = Q[m * g.fs + src];
 }
 
-// Zeroth-order extrapolation (extrapolation.py:29-58): on the boundary plane
-// of direction d and side s (the other directions' halos included), the
-// boundary point and its halo points take the value of the first point inside.
-__global__ void __launch_bounds__(256) k_extrap0(double* __restrict__ Q, int nv, Grid g, int d, int side) {
-  const int e1 = (d == 0) ? 1 : 0, e2 = (d == 2) ? 1 : 2;
-  const int n1 = g.n[e1] + 2 * g.h[e1], n2 = g.n[e2] + 2 * g.h[e2];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n1 * n2) return;
-  int c[3];
-  c[e1] = t % n1 - g.h[e1];
-  c[e2] = t / n1 - g.h[e2];
-  const int N = g.n[d];
-  const int b = side == 0 ? 0 : N - 1;
-  const int from = side == 0 ? 1 : N - 2;
-  const int dir = side == 0 ? -1 : 1;
-  c[d] = from;
-  const int src = g.idx(c[0], c[1], c[2]);
-  for (int m = 0; m < nv; ++m) {
-    const double v = Q[m * g.fs + src];
-    for (int hh = 0; hh <= g.h[d]; ++hh) {
-      c[d] = b + dir * hh;
-      Q[m * g.fs + g.idx(c[0], c[1], c[2])] = v;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Constituent relations over the padded domain: u_m, p, T
 // (taylor_green_vortex.py:29-31).  Read by the central and viscous stencils.
@@ -1390,12 +1364,6 @@ void launch_halo_periodic(double* Q, int nv, const Grid& g, hipStream_t s) {
   const long long total = halo_points(g);
   if (total == 0) return;
   k_halo_periodic<<<(unsigned)((total + 255) / 256), 256, 0, s>>>(Q, nv, g, total);
-}
-
-void launch_extrap0(double* Q, int nv, const Grid& g, int d, int side, hipStream_t s) {
-  const int e1 = (d == 0) ? 1 : 0, e2 = (d == 2) ? 1 : 2;
-  const int n = (g.n[e1] + 2 * g.h[e1]) * (g.n[e2] + 2 * g.h[e2]);
-  k_extrap0<<<(n + 255) / 256, 256, 0, s>>>(Q, nv, g, d, side);
 }
 
 void launch_count_nan(const double* F, int v0, int v1, unsigned long long* count, const Grid& g, hipStream_t s) {

@@ -299,24 +299,27 @@ void apply_bcs(osbl_ctx* c, double* Q) {
     timed(c, F_BC, [&] { launch_halo_periodic(Q, c->nv, c->g, c->stream); });
     return;
   }
-  // the reference's order (block.py:199-210): direction by direction, side 0 then side 1
+  // the reference's order (block.py:199-210): direction by direction; the two
+  // faces of a direction do not touch each other's points
   double* Q2 = (Q == c->Qbuf[0]) ? c->Qbuf[1] : c->Qbuf[0];
+  int nh[3][2];
+  for (int d = 0; d < 3; ++d)
+    for (int s = 0; s < 2; ++s) nh[d][s] = bc_halos(c, s);
+  // one workgroup for a 2-D block while a face's lines are at most a round of it
+  if (c->nd == 2 && c->g.n[0] + 8 <= 1024 && c->g.n[1] + 8 <= 1024) {
+    timed(c, F_BC, [&] {
+      launch_bc_block2d(Q, Q2, c->g, c->ph, c->cfg.bc, nh, c->cfg.twall, c->plane_dev, c->stream);
+    });
+    return;
+  }
   for (int d = 0; d < c->nd; ++d) {
     if (c->cfg.bc[d][0] == OSBL_BC_PERIODIC) {
       timed(c, F_BC, [&] { launch_periodic_dir(Q, c->nv, c->g, d, c->stream); });
       continue;
     }
-    for (int s = 0; s < 2; ++s) {
-      const int bc = c->cfg.bc[d][s];
-      if (bc == OSBL_BC_EXTRAP0) {
-        timed(c, F_BC, [&] { launch_extrap0(Q, c->nv, c->g, d, s, c->stream); });
-      } else {
-        timed(c, F_BC, [&] {
-          launch_bc_face(c->nd, Q, Q2, c->g, c->ph, d, s, bc, bc_halos(c, s), c->cfg.twall, c->plane_dev[d][s],
-                         c->stream);
-        });
-      }
-    }
+    timed(c, F_BC, [&] {
+      launch_bc_sides(c->nd, Q, Q2, c->g, c->ph, d, c->cfg.bc[d], nh[d], c->cfg.twall, c->plane_dev[d], c->stream);
+    });
   }
 }
 

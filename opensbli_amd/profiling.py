@@ -27,6 +27,8 @@ FAMILIES = [
     ("k_char_sweep<2, 0,", "char_sweep_x"),
     ("k_char_sweep<2, 1,", "char_sweep_y"),
     ("k_char_sweep<1, 0,", "char_sweep_x"),
+    ("k_char_tile2d", "char_sweep_x"),
+    ("k_line_", "char_sweep_x"),
     ("k_char_vjp", "adjoint"),
     ("k_adj_", "adjoint"),
     ("k_visc_vjp", "adjoint"),
@@ -39,8 +41,7 @@ FAMILIES = [
     ("k_sensor", "constituent_relations"),
     ("k_halo_periodic", "boundary"),
     ("k_periodic_dir", "boundary"),
-    ("k_bc_face", "boundary"),
-    ("k_extrap0", "boundary"),
+    ("k_bc_", "boundary"),
 ]
 
 
