@@ -36,7 +36,7 @@ void launch_visc_gen3d(const double* Q, const double* P, double* R, const Grid& 
 void launch_body_force3d(const double* Q, double* R, const Grid& g, const Phys& ph, hipStream_t s);
 void launch_prims_slab(const double* Q, double* P, const Grid& g, const Phys& ph, int suth, hipStream_t s);
 void launch_prims_mu(int nd, const double* Q, double* P, const Grid& g, const Phys& ph, hipStream_t s);
-// the two faces of direction d; the four faces of a 2-D block in one workgroup
+// the two faces of direction d (1-D, 3-D); the four faces of a 2-D block
 void launch_bc_sides(int nd, double* Q, double* Q2, const Grid& g, const Phys& ph, int d, const int type[2],
                      const int nh[2], double twall, double* const plane[2], hipStream_t s);
 void launch_bc_block2d(double* Q, double* Q2, const Grid& g, const Phys& ph, const int (*type)[2], const int (*nh)[2],

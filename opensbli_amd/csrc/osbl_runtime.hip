@@ -305,8 +305,7 @@ void apply_bcs(osbl_ctx* c, double* Q) {
   int nh[3][2];
   for (int d = 0; d < 3; ++d)
     for (int s = 0; s < 2; ++s) nh[d][s] = bc_halos(c, s);
-  // one workgroup for a 2-D block while a face's lines are at most a round of it
-  if (c->nd == 2 && c->g.n[0] + 8 <= 1024 && c->g.n[1] + 8 <= 1024) {
+  if (c->nd == 2) {
     timed(c, F_BC, [&] {
       launch_bc_block2d(Q, Q2, c->g, c->ph, c->cfg.bc, nh, c->cfg.twall, c->plane_dev, c->stream);
     });

@@ -89,3 +89,13 @@ def test_2d_plate_shapes(n, conv, sensor, bscheme, wall, oracle):
 def test_2d_periodic_viscous_shapes(n, oracle):
     problem, q0 = _block(n, "weno_z", "periodic", viscous="const", rk="ls3")
     _check(problem, q0, oracle, f"2-D viscous {n}")
+
+
+@pytest.mark.parametrize("bc", [["periodic", "zero_gradient"], ["extrap0", "periodic"], ["symmetry", "extrap1"]])
+@pytest.mark.parametrize("n", [(8, 9), (10, 11), (74, 75), (75, 139)])
+def test_2d_faces(n, bc, oracle):
+    """Faces that meet: all of a face's lines, none or some of them away from
+    the corners, which a kernel treats in the directions' order."""
+    problem, q0 = _block(n, "weno_js", "periodic")
+    problem["bc"] = [[b, b] for b in bc]
+    _check(problem, q0, oracle, f"2-D faces {n} {bc}")
