@@ -201,7 +201,7 @@ struct osbl_ctx {
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
   bool tiled_central = false;  // 3-D central scheme in one tiled kernel
   bool tiled2d = false;     // 2-D characteristic block: the whole stage in one tiled kernel
-  bool haloless = false;    // periodic blocks of these two: read in place, no boundary pass in the time loop
+  bool haloless = false;    // periodic blocks of these two, curvilinear blocks: read in place, no boundary pass in the time loop
   bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
   bool general = false;     // closures, metric or Sutherland viscosity: the general update kernel
   bool suth = false;
@@ -211,8 +211,6 @@ struct osbl_ctx {
   double* plane_dev[3][2] = {};             // per-face planes
   bool curv = false;                        // general curvilinear metric
   double* cmet = nullptr;                   // its D_ab (a*nd + b) and detJ, padded fields
-  double* cflux = nullptr;                  // interface fluxes of one direction (nv padded fields)
-  double* cpt = nullptr;                    // per-point detJ F_d, U, a|k| of one direction (nv + 2 fields)
   bool cmet_ready = false;                  // osbl_set_grid_coordinates has run
   int nplane[3][2] = {};
   // profiling
@@ -361,17 +359,11 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
   }
   if (c->Theta) timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
   if (c->curv) {
-    // strong conservation form: per direction the interface fluxes about the
-    // metric normal and their difference, divided by detJ after the last one
+    // strong conservation form: a kernel per direction, the last one with the update
     for (int d = 0; d < c->nd; ++d) {
       timed(c, F_SWEEP_X + d, [&] {
-        launch_curv_direction(c->nd, d, conv, c->cfg.averaging, Q, c->cmet, c->cpt, c->cflux, c->R, c->g, c->ph,
-                              c->cfg.delta[d], c->stream);
-      });
-    }
-    if (mode != 2) {
-      timed(c, F_UPDATE, [&] {
-        launch_update(c->nd, conv, false, mode, Q, c->P, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->stream);
+        launch_curv_sweep(c->nd, d, conv, c->cfg.averaging, mode, Q, c->cmet, c->R, c->Qo, Qn, c->g, c->ph, cA, cB,
+                          first, c->stream);
       });
     }
     return;
@@ -642,7 +634,7 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear;
   central3d_tiles(c->g, &c->ctx, &c->csz);
   c->tiled2d = c->nd == 2 && !is_central(cfg->conv) && !cfg->curvilinear;
-  c->haloless = (c->tiled_central || c->tiled2d) && all_periodic(c) && !cfg->filters;
+  c->haloless = (c->tiled_central || c->tiled2d || cfg->curvilinear) && all_periodic(c) && !cfg->filters;
   c->line = c->nd == 1 && !is_central(cfg->conv) && cfg->viscous == OSBL_VISC_NONE && !stretched && !ph.has_force &&
             cfg->bc[0][0] == OSBL_BC_EXTRAP0 && cfg->bc[0][1] == OSBL_BC_EXTRAP0;
   c->need_prims = !c->tiled_central && !c->tiled2d && (is_central(cfg->conv) || (cfg->viscous != OSBL_VISC_NONE && !c->tiled_visc));
@@ -664,9 +656,7 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
     return rc;
   }
   c->curv = cfg->curvilinear != 0;
-  if (c->curv && ((rc = alloc(&c->cmet, (size_t)fs * (c->nd * c->nd + 1) * sizeof(double))) ||
-                  (rc = alloc(&c->cflux, bundle)) ||
-                  (rc = alloc(&c->cpt, (size_t)fs * (c->nv + 2) * sizeof(double))))) {
+  if (c->curv && (rc = alloc(&c->cmet, (size_t)fs * (c->nd * c->nd + 1) * sizeof(double)))) {
     osbl_destroy(c);
     return rc;
   }
@@ -747,8 +737,6 @@ void osbl_destroy(osbl_ctx* c) {
   (void)hipFree(c->vw);
   (void)hipFree(c->vy);
   (void)hipFree(c->cmet);
-  (void)hipFree(c->cflux);
-  (void)hipFree(c->cpt);
   (void)hipFree(c->cw_dev);
   (void)hipFree(c->Theta);
   (void)hipFree(c->QF);

@@ -136,3 +136,31 @@ def test_run_needs_coordinates():
     with pytest.raises(OsblError, match="osbl_set_grid_coordinates"):
         g.run(1)
     g.close()
+
+
+@pytest.mark.parametrize("conv,avg,rk", [("weno_z", "roe", "rk3"), ("weno_js", "simple", "ls3"), ("teno5", "roe", "ls3")])
+@pytest.mark.parametrize("n", [(8, 9), (15, 17), (31, 8), (32, 16), (63, 31), (94, 46),
+                               (8, 9, 10), (15, 31, 16), (33, 17, 8), (32, 16, 15), (63, 8, 31)])
+def test_shapes(n, conv, avg, rk, oracle):
+    """Blocks of unequal extents around whole tiles of the sweeps (31 cells of
+    8 lines along x, 15 of 16 along the others)."""
+    _say(f"case curvilinear {n} {conv} {avg} {rk}: rhs and 5 steps")
+    nd, h = len(n), 2
+    xi = np.meshgrid(*[(np.arange(-h, m + h) / m) for m in reversed(n)], indexing="ij")[::-1]
+    coords = np.stack([xi[a] + 0.1 * xi[(a + 1) % nd] + 0.02 * np.sin(2 * np.pi * (xi[0] + xi[(a + 1) % nd] + 0.1 * a))
+                       for a in range(nd)])
+    inner = (slice(h, -h),) * nd
+    s = [2 * np.pi * x[inner] for x in xi]
+    rho = 1.0 + 0.1 * np.sin(s[0] + 0.3) * np.cos(s[1])
+    u = [0.4 + 0.1 * np.cos(s[a] - s[(a + 1) % nd]) for a in range(nd)]
+    p = 1.0 + 0.1 * np.sin(s[-1] + 0.7)
+    q0 = np.stack([rho] + [rho * v for v in u] + [p / 0.4 + 0.5 * rho * sum(v * v for v in u)])
+    delta = [1.0 / m for m in n]
+    problem = dict(ndim=nd, n=list(n), delta=delta, conv=conv, averaging=avg, viscous="none", rk=rk,
+                   bc=[["periodic", "periodic"]] * nd, gama=1.4, dt=0.05 * min(delta), curvilinear=1,
+                   grid_coords=coords, grid_halo=h)
+    g, r = _pair(problem, q0, oracle)
+    check_parity(g.rhs(), r.rhs(), "rhs")
+    g.run(5)
+    r.run(5)
+    check_parity(g.get_state(), r.get_state(), "5 steps")
