@@ -16,6 +16,9 @@ void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, 
 void launch_char_tile2d(int conv, int avg, int mode, bool visc, const double* Q, double* R, double* Qo, double* Qn,
                         const Grid& g, const Phys& ph, const Bnd& b, double cA, double cB, int first, double* theta,
                         int suth, int wrap, hipStream_t s);
+// one stage of a 2-D central scheme on a uniform grid without closures
+void launch_central2d(int conv, bool visc, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
+                      const Phys& ph, double cA, double cB, int first, int wrap, hipStream_t s);
 void launch_sweep_z_rk(int conv, int avg, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
                        const Phys& ph, int seg, const double* theta, double cA, double cB, int first, hipStream_t s);
 void launch_sensor(int nd, const double* Q, double* theta, const Grid& g, const Phys& ph, const Bnd& b, hipStream_t s);

@@ -1325,7 +1325,7 @@ static void launch_update_nd(int conv, bool visc, int mode, const double* Q, con
                              hipStream_t s) {
   const bool central = conv == OSBL_CONV_CENTRAL_SKEW || conv == OSBL_CONV_CENTRAL_CONS;
   if (central) {
-    if constexpr (ND < 3) {  // 3-D: k_central3d
+    if constexpr (ND == 1) {  // 2-D: k_central2d, 3-D: k_central3d
     if (conv == OSBL_CONV_CENTRAL_SKEW) {
       if (visc) launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
       else launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
@@ -1334,7 +1334,7 @@ static void launch_update_nd(int conv, bool visc, int mode, const double* Q, con
       else launch_update_m<ND, OSBL_CONV_CENTRAL_CONS, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
     }
     }
-  } else {
+  } else if constexpr (ND != 2) {  // 2-D: k_char_tile2d
     if (visc) launch_update_m<ND, OSBL_CONV_WENO_Z, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
     else launch_update_m<ND, OSBL_CONV_WENO_Z, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
   }
@@ -1343,7 +1343,6 @@ static void launch_update_nd(int conv, bool visc, int mode, const double* Q, con
 void launch_update(int nd, int conv, bool visc, int mode, const double* Q, const double* P, double* R, double* Qo,
                    double* Qn, const Grid& g, const Phys& ph, double cA, double cB, int first, hipStream_t s) {
   if (nd == 3) launch_update_nd<3>(conv, visc, mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
-  else if (nd == 2) launch_update_nd<2>(conv, visc, mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
   else launch_update_nd<1>(conv, visc, mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
 }
 

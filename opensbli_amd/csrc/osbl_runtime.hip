@@ -199,7 +199,7 @@ struct osbl_ctx {
   bool need_prims = false;
   bool tiled_visc = false;  // 3-D characteristic scheme with viscous terms
   bool tiled_gen = false;   // the same on the general path (closures/metric/mu(T) in x and y only)
-  bool tiled_central = false;  // 3-D central scheme in one tiled kernel
+  bool tiled_central = false;  // 2-D or 3-D central scheme: the whole stage in one tiled kernel
   bool tiled2d = false;     // 2-D characteristic block: the whole stage in one tiled kernel
   bool haloless = false;    // periodic blocks of these two, curvilinear blocks: read in place, no boundary pass in the time loop
   bool line = false;        // 1-D Euler block with zeroth-order extrapolation ends: osbl_line.h
@@ -369,10 +369,13 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
     return;
   }
   if (c->tiled_central) {
-    // 3-D central scheme: everything in one kernel (mode 2: the residual, left in R)
+    // central scheme: everything in one kernel (mode 2: the residual, left in R)
+    const bool visc = c->cfg.viscous != OSBL_VISC_NONE;
     timed(c, F_CENTRAL, [&] {
-      launch_central3d(conv, c->cfg.viscous != OSBL_VISC_NONE, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first,
-                       c->ctx, c->csz, all_periodic(c), c->stream);
+      if (c->nd == 2)
+        launch_central2d(conv, visc, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, all_periodic(c), c->stream);
+      else launch_central3d(conv, visc, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->ctx, c->csz,
+                            all_periodic(c), c->stream);
     });
     return;
   }
@@ -631,7 +634,7 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   c->tiled_gen = c->general && c->nd == 3 && !is_central(cfg->conv) && cfg->viscous != OSBL_VISC_NONE &&
                  !c->bnd.mod[2][0] && !c->bnd.mod[2][1] && !cfg->stretch[2];
   c->vsz = visc3d_segment(c->g);
-  c->tiled_central = !c->general && c->nd == 3 && is_central(cfg->conv) && !cfg->curvilinear;
+  c->tiled_central = !c->general && c->nd > 1 && is_central(cfg->conv) && !cfg->curvilinear;
   central3d_tiles(c->g, &c->ctx, &c->csz);
   c->tiled2d = c->nd == 2 && !is_central(cfg->conv) && !cfg->curvilinear;
   c->haloless = (c->tiled_central || c->tiled2d || cfg->curvilinear) && all_periodic(c) && !cfg->filters;

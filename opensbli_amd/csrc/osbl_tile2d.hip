@@ -1,6 +1,7 @@
-// osbl_tile2d.hip -- one stage of a 2-D characteristic block in one kernel:
-// both sweeps, the viscous terms with closures, metric and mu(T), the body
-// force, the adaptive TENO's sensor, and the RK update.
+// osbl_tile2d.hip -- one stage of a 2-D block in one kernel.  Characteristic
+// schemes: both sweeps, the viscous terms with closures, metric and mu(T), the
+// body force, the adaptive TENO's sensor, and the RK update.  Central schemes
+// (uniform grid, no closures): convective and viscous terms and the RK update.
 #include "osbl_kernels.h"
 #include "osbl_visc.h"
 
@@ -228,6 +229,172 @@ __global__ void __launch_bounds__(256, 3) k_char_tile2d(const double* __restrict
       Qn[m * g.fs + x] = __fma_rn(cB, tmp, S[pc][m]);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Central schemes.  A workgroup takes 32 x 8 cells (a wave: two rows of 32, so
+// stores are whole cache lines) and stages the 36 x 12 points around them in
+// LDS with their constituent relations; mode and wrap as above.  The terms are
+// those of central_convective and viscous_terms, the skew-symmetric form
+// summed point by point: sum_y w (q_m(y) (u_j(y) + u_j(x)) + q_m(x) u_j(y)).
+//
+// What bounds it is one tile's latency on small blocks, memory on large ones.
+// 512^2, skew, viscous, under the profiler: halo pass 4.6 + constituent
+// relations 7.0 + update 14.5 us -> 11.5 us in one launch.
+// ---------------------------------------------------------------------------
+constexpr int C2X = 32, C2Y = 8, C2PX = C2X + 4, C2PY = C2Y + 4, C2P = C2PX * C2PY;
+
+template <int CONV, bool VISC>
+__global__ void __launch_bounds__(256, 4) k_central2d(const double* __restrict__ Q, double* __restrict__ R,
+                                                      double* __restrict__ Qo, double* __restrict__ Qn, Grid g,
+                                                      Phys ph, double cA, double cB, int first, int mode, int wrap) {
+  constexpr int ND = 2, NV = 4, E = 3;
+  __shared__ double S[C2P][9];  // q, u, p, T; odd stride: no bank conflicts along x
+  const int t = threadIdx.x, i = t % C2X, j = t / C2X;
+  const int x0 = blockIdx.x * C2X, y0 = blockIdx.y * C2Y;
+  auto image = [&](int a, int n) { return !wrap ? a : (a < 0 ? a + n : (a >= n ? a - n : a)); };
+  double nq[2][NV];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int p = min(t + 256 * k, C2P - 1);
+    const int gx = min(x0 - 2 + p % C2PX, g.n[0] + 1), gy = min(y0 - 2 + p / C2PX, g.n[1] + 1);
+    fetch_q<ND>(nq[k], Q, g.fs, g.idx(image(gx, g.n[0]), image(gy, g.n[1]), 0));
+  }
+  const int cx = x0 + i, cy = y0 + j;
+  const bool own = cx < g.n[0] && cy < g.n[1];
+  const int x = g.idx(cx, cy, 0);
+  double qo[NV] = {0.0, 0.0, 0.0, 0.0};
+  if (own && (mode == 0 ? !first : (mode == 1 && cA != 0.0))) {
+#pragma unroll
+    for (int m = 0; m < NV; ++m) qo[m] = Qo[m * g.fs + x];
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int p = t + 256 * k;
+    const double ir = recip_pos(nq[k][0]);
+    const double u0 = nq[k][1] * ir, u1 = nq[k][2] * ir;
+    const double pr = ph.gm1 * (nq[k][E] - 0.5 * (nq[k][1] * u0 + nq[k][2] * u1));
+    if (p < C2P) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m) S[p][m] = nq[k][m];
+      S[p][4] = u0;
+      S[p][5] = u1;
+      S[p][6] = pr;
+      S[p][7] = pr * ph.gama * ph.Minf * ph.Minf * ir;
+    }
+  }
+  __syncthreads();
+  if (!own) return;
+  const int pc = (j + 2) * C2PX + i + 2;
+  constexpr double WA = 1.0 / 12.0, WB = 2.0 / 3.0;
+  // the loads of a part stay in it, so that few registers hold points
+  auto part = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  double q[NV], r[NV] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int m = 0; m < NV; ++m) q[m] = S[pc][m];
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const int st = d == 0 ? 1 : C2PX;
+    const double uc = S[pc][4 + d], id = ph.inv_delta[d];
+    double a[NV] = {0.0, 0.0, 0.0, 0.0}, su = 0.0, sp = 0.0, spu = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int off[4] = {-2, -1, 1, 2};
+      const double w4[4] = {WA, -WB, WB, -WA};
+      const double* y = S[pc + off[k] * st];
+      const double w = w4[k], u = y[4 + d], p = y[6];
+      if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
+        const double wu = w * (u + uc);
+#pragma unroll
+        for (int m = 0; m < NV; ++m) a[m] = __fma_rn(wu, y[m], a[m]);
+        su = __fma_rn(w, u, su);
+        spu = __fma_rn(w * u, p, spu);
+      } else {
+        const double wu = w * u;
+        a[0] = __fma_rn(w, y[1 + d], a[0]);
+#pragma unroll
+        for (int m = 1; m < E; ++m) a[m] = __fma_rn(wu, y[m], a[m]);
+        a[E] = __fma_rn(wu, y[E] + p, a[E]);
+      }
+      sp = __fma_rn(w, p, sp);
+    }
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      double s = CONV == OSBL_CONV_CENTRAL_SKEW ? 0.5 * __fma_rn(q[m], su, a[m]) : a[m];
+      if (m == 1 + d) s += sp;
+      if (m == E) s += spu;
+      r[m] = __fma_rn(-id, s, r[m]);
+      asm volatile("" : "+v"(r[m]));
+    }
+    part();
+  }
+  if constexpr (VISC) {
+    auto d1 = [&](int st, auto&& f) {
+      return WA * (f(pc - 2 * st) - f(pc + 2 * st)) + WB * (f(pc + st) - f(pc - st));
+    };
+    auto d2 = [&](int st, auto&& f) {
+      return (-1.0 / 12.0) * (f(pc - 2 * st) + f(pc + 2 * st)) + (4.0 / 3.0) * (f(pc - st) + f(pc + st)) - 2.5 * f(pc);
+    };
+    double DU[2][2], DD[2][2][2], D2T[2];
+    const double none[2] = {0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      auto v = [&](int z) { return S[z][4 + m]; };
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const int st = d == 0 ? 1 : C2PX;
+        const double id = ph.inv_delta[d];
+        DU[m][d] = id * d1(st, v);
+        DD[m][d][d] = id * id * d2(st, v);
+        asm volatile("" : "+v"(DU[m][d]), "+v"(DD[m][d][d]));
+      }
+      // D_1(D_0 u_m)
+      auto inner = [&](int z) {
+        return WA * (S[z - 2][4 + m] - S[z + 2][4 + m]) + WB * (S[z + 1][4 + m] - S[z - 1][4 + m]);
+      };
+      double mix = ph.inv_delta[0] * ph.inv_delta[1] * d1(C2PX, inner);
+      asm volatile("" : "+v"(mix));
+      DD[m][0][1] = DD[m][1][0] = mix;
+      part();
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      D2T[d] = ph.inv_delta[d] * ph.inv_delta[d] * d2(d == 0 ? 1 : C2PX, [&](int z) { return S[z][7]; });
+    const double um[3] = {S[pc][4], S[pc][5], 0.0};
+    viscous_assemble<2>(1.0, um, DU, DD, D2T, none, none, ph, false, r);
+  }
+#pragma unroll
+  for (int m = 0; m < NV; ++m) {
+    if (mode == 2) {
+      R[m * g.fs + x] = r[m];
+    } else if (mode == 0) {
+      const double o = first ? q[m] : qo[m];
+      Qn[m * g.fs + x] = __fma_rn(ph.dt * cA, r[m], o);
+      Qo[m * g.fs + x] = __fma_rn(ph.dt * cB, r[m], o);
+    } else {
+      const double tmp = __fma_rn(ph.dt, r[m], cA * qo[m]);
+      Qo[m * g.fs + x] = tmp;
+      Qn[m * g.fs + x] = __fma_rn(cB, tmp, q[m]);
+    }
+  }
+}
+
+void launch_central2d(int conv, bool visc, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
+                      const Phys& ph, double cA, double cB, int first, int wrap, hipStream_t s) {
+  const dim3 grid((g.n[0] + C2X - 1) / C2X, (g.n[1] + C2Y - 1) / C2Y);
+  auto go = [&](auto cc, auto vv) {
+    k_central2d<decltype(cc)::value, decltype(vv)::value>
+        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, mode, wrap);
+  };
+  auto with_visc = [&](auto cc) {
+    if (visc) go(cc, std::true_type{});
+    else go(cc, std::false_type{});
+  };
+  if (conv == OSBL_CONV_CENTRAL_SKEW) with_visc(std::integral_constant<int, OSBL_CONV_CENTRAL_SKEW>{});
+  else with_visc(std::integral_constant<int, OSBL_CONV_CENTRAL_CONS>{});
 }
 
 void launch_char_tile2d(int conv, int avg, int mode, bool visc, const double* Q, double* R, double* Qo, double* Qn,

@@ -33,6 +33,7 @@ FAMILIES = [
     ("k_adj_", "adjoint"),
     ("k_visc_vjp", "adjoint"),
     ("k_central3d", "central_convective"),
+    ("k_central2d", "central_convective"),
     ("k_visc_update3d", "residual_rk_update"),
     ("k_visc_gen3d", "residual_rk_update"),
     ("k_visc_shell", "residual_rk_update"),

@@ -99,3 +99,12 @@ def test_2d_faces(n, bc, oracle):
     problem, q0 = _block(n, "weno_js", "periodic")
     problem["bc"] = [[b, b] for b in bc]
     _check(problem, q0, oracle, f"2-D faces {n} {bc}")
+
+
+@pytest.mark.parametrize("bc", ["periodic", "symmetry"])
+@pytest.mark.parametrize("conv,rk,viscous", [("central_skew", "ls3", "const"), ("central_skew", "rk3", "none"),
+                                             ("central_cons", "rk3", "const"), ("central_cons", "ls3", "none")])
+@pytest.mark.parametrize("n", [(8, 8), (31, 9), (33, 16), (64, 15), (65, 17)])
+def test_2d_central_shapes(n, conv, rk, viscous, bc, oracle):
+    problem, q0 = _block(n, conv, bc, rk=rk, viscous=viscous)
+    _check(problem, q0, oracle, f"2-D {n} {conv} {rk} {viscous} {bc}")
