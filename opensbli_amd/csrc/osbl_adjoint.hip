@@ -213,106 +213,201 @@ __global__ void __launch_bounds__(128) k_adj_stage(const double* __restrict__ Qs
   }
 }
 
-// 2-D variant of k_adj_stage with the stencil inputs staged through LDS: a
-// 64 x 4 block of cells loads the (64+4) x (4+4) tile of q, u and the adjoint
-// weights mu = alpha A + beta B once (periodic wrap), and every cell's four
-// neighbours per direction are then read from LDS.  Same arithmetic as
-// k_adj_stage.
-constexpr int ATX = 64, ATY = 4, APX = ATX + 4, APY = ATY + 4, ANP = APX * APY;
+// ---------------------------------------------------------------------------
+// The same on 2-D blocks in one tiled kernel, with the viscous terms' VJP (the
+// formulas of osbl_adjoint_visc.hip): a workgroup takes 16 x 16 cells and
+// stages rho, u, rhoE and mu = alpha A + beta B of the points around them in
+// LDS (two layers; four with viscous terms), forms w and 2 mu_E tau on the
+// cells and two layers, and finishes every cell.
+//   EULER: out1 = c (A + B) + V and out2 as k_adj_stage, V with the viscous
+//   part when VISC; otherwise out1 += the viscous part alone.
+//
+// What bounds it is one tile's latency at three workgroups a CU, and the points
+// staged more than once (2.25 per cell).  512^2, central, viscous, under the
+// profiler: stage 23.5, padded copies 8.0, w and tau 11.5, viscous part 12.2 us
+// -> 34 us in one launch.
+// ---------------------------------------------------------------------------
+constexpr int A2C = 16;
 
-__global__ void __launch_bounds__(256) k_adj_stage2d(const double* __restrict__ Qs, const double* __restrict__ A,
-                                                     const double* __restrict__ B, double alpha, double beta,
-                                                     double c, double* __restrict__ out1, double* __restrict__ out2,
-                                                     int n0, int n1, Phys ph) {
+template <bool EULER, bool VISC>
+__global__ void __launch_bounds__(256, VISC ? 3 : 4) k_adj_tile2d(const double* __restrict__ Qs,
+                                                                  const double* __restrict__ A,
+                                                                  const double* __restrict__ B, double alpha,
+                                                                  double beta, double c, double* __restrict__ out1,
+                                                                  double* __restrict__ out2, int n0, int n1, Phys ph) {
   constexpr int NV = 4, E = 3;
-  __shared__ double s_mu[NV][ANP];
-  __shared__ double s_q[NV][ANP];
-  __shared__ double s_u[2][ANP];
-  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * ATX + tx;
-  const int x0 = blockIdx.x * ATX, y0 = blockIdx.y * ATY;
+  constexpr int H = VISC ? 4 : 2, PX = A2C + 2 * H, NP = PX * PX;  // staged points
+  constexpr int MX = A2C + 4, NM = VISC ? MX * MX : 1;             // points of w and tau
+  constexpr int U = 0, MU = 1;                                     // fields of S: MU + m is mu_m, m > 0
+  constexpr int TX = A2C + 4;                                      // rho, rhoE, mu_0: the cells and two layers
+  // odd strides: no bank conflicts along x.  49 KB with viscous terms: three
+  // workgroups a CU (two, with eight fields at every point, took as long)
+  __shared__ double S[NP][5];       // u, mu_1, mu_2, mu_E
+  __shared__ double T[TX * TX][3];  // rho, rhoE, mu_0
+  __shared__ double W[NM][5];       // w, 2 mu_E tau_00, _01, _11
+  const int t = threadIdx.x, i = t % A2C, j = t / A2C;
+  const int x0 = blockIdx.x * A2C, y0 = blockIdx.y * A2C;
   const long long cells = (long long)n0 * n1;
-  for (int p = tid; p < ANP; p += ATX * ATY) {
-    const int xx = p % APX, yy = p / APX;
-    int gx = (x0 - 2 + xx) % n0;
-    int gy = (y0 - 2 + yy) % n1;
-    gx = gx < 0 ? gx + n0 : gx;
-    gy = gy < 0 ? gy + n1 : gy;
-    const long long y = gx + (long long)n0 * gy;
-    double q[NV];
+  // a tile's points beyond the block's reach (n + H - 1) feed no cell
+  auto image = [](int a, int n) {
+    a = min(a, n + H - 1);
+    return a < 0 ? a + n : (a >= n ? a - n : a);
+  };
 #pragma unroll
-    for (int m = 0; m < NV; ++m) {
-      q[m] = Qs[m * cells + y];
-      s_q[m][p] = q[m];
-      double v = alpha * A[m * cells + y];
-      if (B) v += beta * B[m * cells + y];
-      s_mu[m][p] = v;
-    }
-    const double ir = 1.0 / q[0];
-    s_u[0][p] = q[1] * ir;
-    s_u[1][p] = q[2] * ir;
-  }
-  __syncthreads();
-  const int i = x0 + tx, j0 = y0 + ty;
-  if (i >= n0 || j0 >= n1) return;
-  const int cc = (ty + 2) * APX + tx + 2;
-  const long long x = i + (long long)n0 * j0;
-  double q[NV], u[2], mu[NV];
-#pragma unroll
-  for (int m = 0; m < NV; ++m) {
-    q[m] = s_q[m][cc];
-    mu[m] = s_mu[m][cc];
-  }
-  u[0] = s_u[0][cc];
-  u[1] = s_u[1][cc];
-  const double p = ph.gm1 * (q[E] - 0.5 * q[0] * (u[0] * u[0] + u[1] * u[1]));
-  double gq[NV], gu[2], gp = 0.0;
-#pragma unroll
-  for (int m = 0; m < NV; ++m) gq[m] = 0.0;
-#pragma unroll
-  for (int jd = 0; jd < 2; ++jd) {
-    const double inv = ph.inv_delta[jd];
-    constexpr double W1A = 1.0 / 12.0, W1B = 2.0 / 3.0;
-    const int st = jd == 0 ? 1 : APX;
-    const int offs[4] = {-2 * st, -st, st, 2 * st};
-    const double wts[4] = {W1A, -W1B, W1B, -W1A};
-    double dmu[NV], dmuu[NV], dq[NV], dmuq = 0.0, duj = 0.0;
-#pragma unroll
-    for (int m = 0; m < NV; ++m) { dmu[m] = 0.0; dmuu[m] = 0.0; dq[m] = 0.0; }
-#pragma unroll
-    for (int sI = 0; sI < 4; ++sI) {
-      const int y = cc + offs[sI];
-      const double w = wts[sI];
-      const double uj = s_u[jd][y];
-      double sq = 0.0;
+  for (int k = 0; k < (NP + 255) / 256; ++k) {
+    const int p = t + 256 * k;
+    if (p < NP) {
+      const long long y = image(x0 - H + p % PX, n0) + (long long)n0 * image(y0 - H + p / PX, n1);
+      double q[NV], mu[NV];
 #pragma unroll
       for (int m = 0; m < NV; ++m) {
-        const double my = s_mu[m][y];
-        const double qy = s_q[m][y];
-        dmu[m] += w * my;
-        dmuu[m] += w * (my * uj);
-        dq[m] += w * qy;
-        sq += my * qy;
+        q[m] = Qs[m * cells + y];
+        mu[m] = alpha * A[m * cells + y];
+        if (B) mu[m] = __fma_rn(beta, B[m * cells + y], mu[m]);
       }
-      dmuq += w * sq;
-      duj += w * uj;
-    }
+      const double ir = recip_pos(q[0]);
+      S[p][U] = q[1] * ir;
+      S[p][U + 1] = q[2] * ir;
 #pragma unroll
-    for (int m = 0; m < NV; ++m) { dmu[m] *= inv; dmuu[m] *= inv; dq[m] *= inv; }
-    dmuq *= inv;
-    duj *= inv;
-    double gu_j = 0.5 * dmuq + p * dmu[E];
-#pragma unroll
-    for (int m = 0; m < NV; ++m) {
-      gq[m] += 0.5 * u[jd] * dmu[m] + 0.5 * dmuu[m] - 0.5 * mu[m] * duj;
-      gu_j += 0.5 * q[m] * dmu[m] - 0.5 * mu[m] * dq[m];
+      for (int m = 1; m < NV; ++m) S[p][MU + m] = mu[m];
+      const int tx = p % PX - (H - 2), ty = p / PX - (H - 2);
+      if (tx >= 0 && ty >= 0 && tx < TX && ty < TX) {
+        T[ty * TX + tx][0] = q[0];
+        T[ty * TX + tx][1] = q[E];
+        T[ty * TX + tx][2] = mu[0];
+      }
     }
-    gu[jd] = gu_j;
-    gp += dmu[1 + jd] + u[jd] * dmu[E];
   }
-  const double ir = 1.0 / q[0];
+  __syncthreads();
+  constexpr double WA = 1.0 / 12.0, WB = 2.0 / 3.0;
+  // first, second and mixed derivative (without 1/Delta) at o of f(point), rows st and PR apart
+  auto d1 = [&](int o, int st, auto&& f) {
+    return WA * (f(o - 2 * st) - f(o + 2 * st)) + WB * (f(o + st) - f(o - st));
+  };
+  auto d2 = [&](int o, int st, auto&& f) {
+    return (-1.0 / 12.0) * (f(o - 2 * st) + f(o + 2 * st)) + (4.0 / 3.0) * (f(o - st) + f(o + st)) - 2.5 * f(o);
+  };
+  auto dmix = [&](int o, int row, auto&& f) { return d1(o, row, [&](int z) { return d1(z, 1, f); }); };
+  // the loads of a part stay in it, so that few registers hold points
+  auto part = [](double& v) {
+    asm volatile("" : "+v"(v) : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const double id0 = ph.inv_delta[0], id1 = ph.inv_delta[1];
+  if constexpr (VISC) {
+#pragma unroll
+    for (int k = 0; k < (NM + 255) / 256; ++k) {
+      const int p = t + 256 * k;
+      if (p < NM) {
+        const int o = (p / MX + 2) * PX + p % MX + 2;
+        auto u0 = [&](int z) { return S[z][U]; };
+        auto u1 = [&](int z) { return S[z][U + 1]; };
+        const double d00 = id0 * d1(o, 1, u0), d01 = id1 * d1(o, PX, u0);
+        const double d10 = id0 * d1(o, 1, u1), d11 = id1 * d1(o, PX, u1);
+        const double muE = S[o][MU + E], f = 2.0 * muE * ph.inv_re, div = (2.0 / 3.0) * (d00 + d11);
+        W[p][0] = __fma_rn(muE, S[o][U], S[o][MU + 1]);
+        W[p][1] = __fma_rn(muE, S[o][U + 1], S[o][MU + 2]);
+        W[p][2] = f * (2.0 * d00 - div);
+        W[p][3] = f * (d01 + d10);
+        W[p][4] = f * (2.0 * d11 - div);
+      }
+    }
+    __syncthreads();
+  }
+  const int cx = x0 + i, cy = y0 + j;
+  if (cx >= n0 || cy >= n1) return;
+  const long long x = cx + (long long)n0 * cy;
+  const int o = (j + H) * PX + i + H, to = (j + 2) * TX + i + 2;
+  const double rho = T[to][0], ir = recip_pos(rho);
+  const double u[2] = {S[o][U], S[o][U + 1]};
   const double uu = u[0] * u[0] + u[1] * u[1];
+  const double p = ph.gm1 * (T[to][1] - 0.5 * rho * uu);
+  double gq[NV] = {0.0, 0.0, 0.0, 0.0}, gu[2] = {0.0, 0.0}, gp = 0.0;
+  if constexpr (EULER) {
+    double q[NV], mu[NV];
+    q[0] = rho;
+    q[1] = rho * u[0];
+    q[2] = rho * u[1];
+    q[E] = T[to][1];
+    mu[0] = T[to][2];
+#pragma unroll
+    for (int m = 1; m < NV; ++m) mu[m] = S[o][MU + m];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int st = d == 0 ? 1 : PX;
+      double dmu[NV] = {0.0, 0.0, 0.0, 0.0}, dmuu[NV] = {0.0, 0.0, 0.0, 0.0};
+      double duj = 0.0, dmuq = 0.0, mdq = 0.0;  // D u_j, D(mu.q), mu.D q
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int off[4] = {-2, -1, 1, 2};
+        const double w4[4] = {WA, -WB, WB, -WA};
+        const double* y = S[o + off[k] * st];
+        const double* z = T[to + off[k] * (d == 0 ? 1 : TX)];
+        const double w = w4[k], wu = w * y[U + d], r = z[0];
+        const double qy[NV] = {r, r * y[U], r * y[U + 1], z[1]};
+        double sq = 0.0, sm = 0.0;
+#pragma unroll
+        for (int m = 0; m < NV; ++m) {
+          const double my = m == 0 ? z[2] : y[MU + m];
+          dmu[m] = __fma_rn(w, my, dmu[m]);
+          dmuu[m] = __fma_rn(wu, my, dmuu[m]);
+          sq = __fma_rn(my, qy[m], sq);
+          sm = __fma_rn(mu[m], qy[m], sm);
+        }
+        dmuq = __fma_rn(w, sq, dmuq);
+        mdq = __fma_rn(w, sm, mdq);
+        duj += wu;
+      }
+      const double inv = ph.inv_delta[d];
+      double qdm = 0.0;
+#pragma unroll
+      for (int m = 0; m < NV; ++m) {
+        gq[m] = __fma_rn(0.5 * inv, u[d] * dmu[m] + dmuu[m] - mu[m] * duj, gq[m]);
+        qdm = __fma_rn(q[m], dmu[m], qdm);
+        asm volatile("" : "+v"(gq[m]));
+      }
+      gu[d] = inv * (0.5 * (dmuq - mdq + qdm) + p * dmu[E]);
+      gp = __fma_rn(inv, __fma_rn(u[d], dmu[E], dmu[1 + d]), gp);
+      asm volatile("" : "+v"(gu[d]));
+      part(gp);
+    }
+  }
+  double gT = 0.0;
+  if constexpr (VISC) {
+    const int mo = (j + 2) * MX + i + 2;
+    const double muE = S[o][MU + E], id[2] = {id0, id1};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      // (sum_j M_jj w_k + 1/3 sum_m M_mk w_m) / Re - sum_b D_b(2 mu_E tau_kb), and mu_E times the same of u
+      auto wk = [&](int z) { return W[z][k]; };
+      auto wo = [&](int z) { return W[z][1 - k]; };
+      auto uk = [&](int z) { return S[z][U + k]; };
+      auto uo = [&](int z) { return S[z][U + 1 - k]; };
+      double c0 = id0 * id0, c1 = id1 * id1;
+      (k == 0 ? c0 : c1) *= 4.0 / 3.0;
+      const double cm = (1.0 / 3.0) * id0 * id1;
+      double vw = c0 * d2(mo, 1, wk) + c1 * d2(mo, MX, wk) + cm * dmix(mo, MX, wo);
+      part(vw);
+      double vu = c0 * d2(o, 1, uk) + c1 * d2(o, PX, uk) + cm * dmix(o, PX, uo);
+      part(vu);
+      double s = ph.inv_re * __fma_rn(muE, vu, vw);
+      s -= id[0] * d1(mo, 1, [&](int z) { return W[z][2 + k]; });
+      s -= id[1] * d1(mo, MX, [&](int z) { return W[z][3 + k]; });
+      gu[k] += s;
+      part(gu[k]);
+    }
+    auto me = [&](int z) { return S[z][MU + E]; };
+    gT = ph.cq * (id0 * id0 * d2(o, 1, me) + id1 * id1 * d2(o, PX, me));
+  }
+  // chain rule through u = rhou / rho, p and T = gama Minf^2 p / rho
   double v[NV];
-  v[0] = gq[0] + gp * ph.gm1 * 0.5 * uu;
+  v[0] = gq[0];
+  if constexpr (VISC) {
+    const double gM = ph.gama * ph.Minf * ph.Minf * ir;
+    gp = __fma_rn(gT, gM, gp);
+    v[0] -= gT * (p * gM) * ir;
+  }
+  v[0] += gp * ph.gm1 * 0.5 * uu;
 #pragma unroll
   for (int d = 0; d < 2; ++d) {
     v[0] -= gu[d] * u[d] * ir;
@@ -321,19 +416,31 @@ __global__ void __launch_bounds__(256) k_adj_stage2d(const double* __restrict__ 
   v[E] = gq[E] + gp * ph.gm1;
 #pragma unroll
   for (int m = 0; m < NV; ++m) {
-    const double ab = A[m * cells + x] + (B ? B[m * cells + x] : 0.0);
-    out1[m * cells + x] = c * ab + v[m];
-    if (out2) out2[m * cells + x] = ab;
+    if constexpr (EULER) {
+      const double ab = A[m * cells + x] + (B ? B[m * cells + x] : 0.0);
+      out1[m * cells + x] = c * ab + v[m];
+      if (out2) out2[m * cells + x] = ab;
+    } else {
+      out1[m * cells + x] += v[m];
+    }
   }
+}
+
+void launch_adj_tile2d(bool euler, bool visc, const double* Qs, const double* A, const double* B, double alpha,
+                       double beta, double c, double* out1, double* out2, const Grid& g, const Phys& ph,
+                       hipStream_t s) {
+  const dim3 grid((g.n[0] + A2C - 1) / A2C, (g.n[1] + A2C - 1) / A2C);
+  auto go = [&](auto ee, auto vv) {
+    k_adj_tile2d<decltype(ee)::value, decltype(vv)::value>
+        <<<grid, 256, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0], g.n[1], ph);
+  };
+  if (!euler) go(std::false_type{}, std::true_type{});
+  else if (visc) go(std::true_type{}, std::true_type{});
+  else go(std::true_type{}, std::false_type{});
 }
 
 void launch_adj_stage(int nd, const double* Qs, const double* A, const double* B, double alpha, double beta, double c,
                       double* out1, double* out2, const Grid& g, const Phys& ph, hipStream_t s) {
-  if (nd == 2) {
-    dim3 grid((g.n[0] + ATX - 1) / ATX, (g.n[1] + ATY - 1) / ATY);
-    k_adj_stage2d<<<grid, dim3(ATX, ATY), 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0], g.n[1], ph);
-    return;
-  }
   dim3 grid((g.n[0] + 127) / 128, g.n[1], g.n[2]);
   if (nd == 3) k_adj_stage<3><<<grid, 128, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0], g.n[1], g.n[2], ph);
   else k_adj_stage<1><<<grid, 128, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0], g.n[1], g.n[2], ph);

@@ -229,22 +229,19 @@ void launch_unpack_prims(int nd, const double* q, double* Qpad, double* P, const
 
 // out (packed) += (dV/dQ at q)^T (alpha A + beta B) for the viscous terms V,
 // q the packed state.  P (nd + 2 padded fields), Mpad (nv) and W
-// (visc_vjp_fields(nd)) are scratch; the grid's halo is >= 4 (the first pass
+// (visc_vjp_fields(nd)) are scratch (2-D: launch_adj_tile2d); the grid's halo is >= 4 (the first pass
 // reads P and M two layers beyond the two halo layers of W it forms).
 void launch_visc_vjp(int nd, const double* q, const double* A, const double* B, double alpha, double beta, double* P,
                      double* Mpad, double* W, double* out, const Grid& g, const Phys& ph, hipStream_t s) {
   dim3 gu((g.n[0] + 2 * g.h[0] + 255) / 256, g.n[1] + 2 * g.h[1], g.n[2] + 2 * g.h[2]);
   if (nd == 3) k_adj_unpack<3><<<gu, 256, 0, s>>>(q, A, B, alpha, beta, P, Mpad, g, ph);
-  else if (nd == 2) k_adj_unpack<2><<<gu, 256, 0, s>>>(q, A, B, alpha, beta, P, Mpad, g, ph);
   else k_adj_unpack<1><<<gu, 256, 0, s>>>(q, A, B, alpha, beta, P, Mpad, g, ph);
   // w and 2 mu_E tau over the interior and two halo layers
-  dim3 gp((g.n[0] + 4 + 127) / 128, g.n[1] + (nd >= 2 ? 4 : 0), g.n[2] + (nd >= 3 ? 4 : 0));
+  dim3 gp((g.n[0] + 4 + 127) / 128, g.n[1] + (nd == 3 ? 4 : 0), g.n[2] + (nd == 3 ? 4 : 0));
   if (nd == 3) k_visc_vjp_pre<3><<<gp, 128, 0, s>>>(P, Mpad, W, g, ph);
-  else if (nd == 2) k_visc_vjp_pre<2><<<gp, 128, 0, s>>>(P, Mpad, W, g, ph);
   else k_visc_vjp_pre<1><<<gp, 128, 0, s>>>(P, Mpad, W, g, ph);
   dim3 grid((g.n[0] + 127) / 128, g.n[1], g.n[2]);
   if (nd == 3) k_visc_vjp<3><<<grid, 128, 0, s>>>(q, P, Mpad, W, out, g, ph);
-  else if (nd == 2) k_visc_vjp<2><<<grid, 128, 0, s>>>(q, P, Mpad, W, out, g, ph);
   else k_visc_vjp<1><<<grid, 128, 0, s>>>(q, P, Mpad, W, out, g, ph);
 }
 

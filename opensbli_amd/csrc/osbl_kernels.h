@@ -12,13 +12,13 @@ void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, 
 // one stage of a 2-D characteristic block (osbl_tile2d.hip); theta: the
 // adaptive TENO's sensor is formed and left there; wrap: periodic in both
 // directions, halos not read.  conv CONV_WFILTER, mode 2: the WENO filter's
-// flux differences into R
+// flux differences into R.  PK, when given: Q's interior, packed
 void launch_char_tile2d(int conv, int avg, int mode, bool visc, const double* Q, double* R, double* Qo, double* Qn,
                         const Grid& g, const Phys& ph, const Bnd& b, double cA, double cB, int first, double* theta,
-                        int suth, int wrap, hipStream_t s);
-// one stage of a 2-D central scheme on a uniform grid without closures
+                        int suth, int wrap, double* PK, hipStream_t s);
+// one stage of a 2-D central scheme on a uniform grid without closures; PK as above
 void launch_central2d(int conv, bool visc, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
-                      const Phys& ph, double cA, double cB, int first, int wrap, hipStream_t s);
+                      const Phys& ph, double cA, double cB, int first, int wrap, double* PK, hipStream_t s);
 void launch_sweep_z_rk(int conv, int avg, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
                        const Phys& ph, int seg, const double* theta, double cA, double cB, int first, hipStream_t s);
 void launch_sensor(int nd, const double* Q, double* theta, const Grid& g, const Phys& ph, const Bnd& b, hipStream_t s);
@@ -52,6 +52,11 @@ void launch_unpack(const double* in, double* F, const Grid& g, hipStream_t s);
 long long halo_points(const Grid& g);
 void launch_rhs_vjp(int nd, const double* Q, const double* P, const double* M, double* out, const Grid& g,
                     const Phys& ph, hipStream_t s);
+// a 2-D reverse stage of the central scheme (euler) and/or of the viscous terms
+// (alone: added to out1), on packed arrays
+void launch_adj_tile2d(bool euler, bool visc, const double* Qs, const double* A, const double* B, double alpha,
+                       double beta, double c, double* out1, double* out2, const Grid& g, const Phys& ph,
+                       hipStream_t s);
 void launch_adj_stage(int nd, const double* Qs, const double* A, const double* B, double alpha, double beta, double c,
                       double* out1, double* out2, const Grid& g, const Phys& ph, hipStream_t s);
 void launch_pack_all(const double* F, double* out, const Grid& g, int nv, hipStream_t s);

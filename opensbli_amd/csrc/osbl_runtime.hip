@@ -328,17 +328,20 @@ void loop_bcs(osbl_ctx* c) {
 
 // spatial residual of the current state into R (characteristic part only),
 // followed by the fused central/viscous + update kernel with the given mode
-void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
+// pk (optional): takes the packed input state
+void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = nullptr) {
   double* Q = Qcur(c);
   double* Qn = c->Qbuf[1 - c->cur];
   const int conv = c->cfg.conv;
+  const bool tile = c->tiled2d || (c->tiled_central && c->nd == 2);  // these write pk themselves
+  if (pk && !tile) launch_pack_all(Q, pk, c->g, c->nv, c->stream);
   if (c->tiled2d) {
     // (the kernel forms the adaptive TENO's sensor; the WENO filter's on another scheme here)
     if (c->Theta && conv != OSBL_CONV_TENO5 && conv != OSBL_CONV_TENO6)
       timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
     timed(c, F_SWEEP_X, [&] {
       launch_char_tile2d(conv, c->cfg.averaging, mode, c->cfg.viscous != OSBL_VISC_NONE, Q, c->R, c->Qo, Qn, c->g,
-                         c->ph, c->bnd, cA, cB, first, c->Theta, c->suth ? 1 : 0, c->haloless ? 1 : 0, c->stream);
+                         c->ph, c->bnd, cA, cB, first, c->Theta, c->suth ? 1 : 0, c->haloless ? 1 : 0, pk, c->stream);
     });
     return;
   }
@@ -373,7 +376,8 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first) {
     const bool visc = c->cfg.viscous != OSBL_VISC_NONE;
     timed(c, F_CENTRAL, [&] {
       if (c->nd == 2)
-        launch_central2d(conv, visc, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, all_periodic(c), c->stream);
+        launch_central2d(conv, visc, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, all_periodic(c), pk,
+                         c->stream);
       else launch_central3d(conv, visc, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, cA, cB, first, c->ctx, c->csz,
                             all_periodic(c), c->stream);
     });
@@ -855,7 +859,7 @@ static void filters(osbl_ctx* c) {
     if (c->nd == 2) {
       timed(c, F_FILTER, [&] {
         launch_char_tile2d(CONV_WFILTER, OSBL_AVG_SIMPLE, 2, false, Q, c->R, nullptr, nullptr, c->g, c->ph, c->bnd,
-                           0.0, 0.0, 0, nullptr, 0, 0, c->stream);
+                           0.0, 0.0, 0, nullptr, 0, 0, nullptr, c->stream);
       });
     }
     for (int d = 0; d < c->nd && c->nd == 3; ++d) {
@@ -1361,7 +1365,7 @@ static int adjoint_ready(osbl_ctx* c, bool need_rk3, AdjBufs* b) {
     HIPCHK(hipMemsetAsync(c->Abuf, 0, bundle, c->stream));
     HIPCHK(hipMemsetAsync(c->Mbuf, 0, bundle, c->stream));
   }
-  if (c->cfg.viscous == OSBL_VISC_CONST && !c->vw) {
+  if (c->cfg.viscous == OSBL_VISC_CONST && c->nd != 2 && !c->vw) {
     const size_t bytes = (size_t)c->g.fs * visc_vjp_fields(c->nd) * sizeof(double);
     if (hipMalloc((void**)&c->vw, bytes) != hipSuccess) return fail(OSBL_E_NOMEM, "adjoint viscous scratch");
     HIPCHK(hipMemsetAsync(c->vw, 0, bytes, c->stream));
@@ -1393,18 +1397,24 @@ static void vjp(osbl_ctx* c, const AdjBufs& b, const double* q, const double* mu
 // out (packed) += (dV/dQ at q)^T (alpha A + beta B) for the viscous terms V
 static void visc_vjp(osbl_ctx* c, const AdjBufs& b, const double* q, const double* A, const double* B, double alpha,
                      double beta, double* out) {
-  launch_visc_vjp(c->nd, q, A, B, alpha, beta, b.P, b.Mbuf, b.vw, out, c->g, c->ph, c->stream);
+  if (c->nd == 2) launch_adj_tile2d(false, true, q, A, B, alpha, beta, 0.0, out, nullptr, c->g, c->ph, c->stream);
+  else launch_visc_vjp(c->nd, q, A, B, alpha, beta, b.P, b.Mbuf, b.vw, out, c->g, c->ph, c->stream);
 }
 
 // out1 = c (A + B) + (dR/dQ at Qs)^T (alpha A + beta B), out2 = A + B (optional)
 static void adj_stage(osbl_ctx* c, const AdjBufs& b, const double* Qs, const double* A, const double* B, double alpha,
                       double beta, double cc, double* out1, double* out2) {
-  if (c->cfg.conv == OSBL_CONV_WENO_Z)
+  const bool visc = c->cfg.viscous == OSBL_VISC_CONST;
+  if (c->cfg.conv == OSBL_CONV_WENO_Z) {
     launch_adj_stage_char(c->nd, c->cfg.averaging, Qs, A, B, alpha, beta, cc, out1, out2, c->g, c->ph, false,
                           c->stream, b.vy);
-  else
+  } else if (c->nd == 2) {
+    launch_adj_tile2d(true, visc, Qs, A, B, alpha, beta, cc, out1, out2, c->g, c->ph, c->stream);
+    return;
+  } else {
     launch_adj_stage(c->nd, Qs, A, B, alpha, beta, cc, out1, out2, c->g, c->ph, c->stream);
-  if (c->cfg.viscous == OSBL_VISC_CONST) visc_vjp(c, b, Qs, A, B, alpha, beta, out1);
+  }
+  if (visc) visc_vjp(c, b, Qs, A, B, alpha, beta, out1);
 }
 
 // one RK3 step backwards: lam <- (dQ_{n+1}/dQ_n)^T lam
@@ -1487,8 +1497,8 @@ static int scratch_bufs(osbl_ctx* c, AdjBufs* b) {
   auto at = [&](long long o) { return o < 0 ? nullptr : base + o; };
   *b = AdjBufs{at(o_A), at(o_M), at(o_pk), at(o_vw), at(o_P), nullptr};
   // zero everything from the first halo buffer on (A, M, the viscous
-  // fields, P): the allocating path's buffers start zeroed
-  if (halo || visc) {
+  // fields, P): the allocating path's buffers start zeroed (2-D: not read)
+  if ((halo || visc) && c->nd != 2) {
     const long long from = halo ? o_A : o_vw;
     const long long n = off - from;
     const unsigned blocks = (unsigned)std::min<long long>((n + 255) / 256, 8192);
@@ -1522,8 +1532,7 @@ int osbl_step_stages_dev(osbl_ctx* c, double* stages_dev) {
   const int mode = c->cfg.rk == OSBL_RK3 ? 0 : 1;
   loop_bcs(c);
   for (int s = 0; s < c->nstages; ++s) {
-    launch_pack_all(Qcur(c), stages_dev + (long long)s * c->nv * n, c->g, c->nv, c->stream);
-    stage(c, mode, c->A[s], c->B[s], s == 0);
+    stage(c, mode, c->A[s], c->B[s], s == 0, stages_dev + (long long)s * c->nv * n);
     c->cur ^= 1;
     loop_bcs(c);
   }

@@ -32,13 +32,15 @@ constexpr int T2C = 15, T2P = T2C + 6;  // cells and staged points per side
 //
 // mode as k_update (2: residual into R).  wrap: periodic in both directions,
 // points are read at their periodic images and the halos need not be filled.
-// SENSOR: theta is formed here and left in TH (interior).
+// SENSOR: theta is formed here and left in TH (interior).  PK, when given,
+// takes the packed stage input (the adjoint's; a pass of 5.5 us at 512^2).
 // ---------------------------------------------------------------------------
 template <int CONV, int AVG, bool VISC, bool SENSOR>
 __global__ void __launch_bounds__(256, 3) k_char_tile2d(const double* __restrict__ Q, double* __restrict__ R,
                                                         double* __restrict__ Qo, double* __restrict__ Qn, Grid g,
                                                         Phys ph, Bnd b, double cA, double cB, int first, int mode,
-                                                        double* __restrict__ TH, int suth, int wrap) {
+                                                        double* __restrict__ TH, int suth, int wrap,
+                                                        double* __restrict__ PK) {
   constexpr int ND = 2, NV = 4;
   constexpr bool ROE = AVG == OSBL_AVG_ROE;
   constexpr int NF = NV + ND + 2 + ((ROE || VISC) ? 2 : 0);  // q, u, p, a (, sqrt(rho), sqrt(rho) H; then T, mu)
@@ -215,6 +217,10 @@ __global__ void __launch_bounds__(256, 3) k_char_tile2d(const double* __restrict
     r[2] -= ph.force[1];
     r[3] -= ph.force[0] * S[pc][4] + ph.force[1] * S[pc][5];
   }
+  if (PK) {
+#pragma unroll
+    for (int m = 0; m < NV; ++m) PK[((long long)m * g.n[1] + cy) * g.n[0] + cx] = S[pc][m];
+  }
 #pragma unroll
   for (int m = 0; m < NV; ++m) {
     if (mode == 2) {
@@ -247,7 +253,8 @@ constexpr int C2X = 32, C2Y = 8, C2PX = C2X + 4, C2PY = C2Y + 4, C2P = C2PX * C2
 template <int CONV, bool VISC>
 __global__ void __launch_bounds__(256, 4) k_central2d(const double* __restrict__ Q, double* __restrict__ R,
                                                       double* __restrict__ Qo, double* __restrict__ Qn, Grid g,
-                                                      Phys ph, double cA, double cB, int first, int mode, int wrap) {
+                                                      Phys ph, double cA, double cB, int first, int mode, int wrap,
+                                                      double* __restrict__ PK) {
   constexpr int ND = 2, NV = 4, E = 3;
   __shared__ double S[C2P][9];  // q, u, p, T; odd stride: no bank conflicts along x
   const int t = threadIdx.x, i = t % C2X, j = t / C2X;
@@ -366,6 +373,10 @@ __global__ void __launch_bounds__(256, 4) k_central2d(const double* __restrict__
     const double um[3] = {S[pc][4], S[pc][5], 0.0};
     viscous_assemble<2>(1.0, um, DU, DD, D2T, none, none, ph, false, r);
   }
+  if (PK) {
+#pragma unroll
+    for (int m = 0; m < NV; ++m) PK[((long long)m * g.n[1] + cy) * g.n[0] + cx] = q[m];
+  }
 #pragma unroll
   for (int m = 0; m < NV; ++m) {
     if (mode == 2) {
@@ -383,11 +394,11 @@ __global__ void __launch_bounds__(256, 4) k_central2d(const double* __restrict__
 }
 
 void launch_central2d(int conv, bool visc, int mode, const double* Q, double* R, double* Qo, double* Qn, const Grid& g,
-                      const Phys& ph, double cA, double cB, int first, int wrap, hipStream_t s) {
+                      const Phys& ph, double cA, double cB, int first, int wrap, double* PK, hipStream_t s) {
   const dim3 grid((g.n[0] + C2X - 1) / C2X, (g.n[1] + C2Y - 1) / C2Y);
   auto go = [&](auto cc, auto vv) {
     k_central2d<decltype(cc)::value, decltype(vv)::value>
-        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, mode, wrap);
+        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, cA, cB, first, mode, wrap, PK);
   };
   auto with_visc = [&](auto cc) {
     if (visc) go(cc, std::true_type{});
@@ -399,11 +410,11 @@ void launch_central2d(int conv, bool visc, int mode, const double* Q, double* R,
 
 void launch_char_tile2d(int conv, int avg, int mode, bool visc, const double* Q, double* R, double* Qo, double* Qn,
                         const Grid& g, const Phys& ph, const Bnd& b, double cA, double cB, int first, double* theta,
-                        int suth, int wrap, hipStream_t s) {
+                        int suth, int wrap, double* PK, hipStream_t s) {
   const dim3 grid((g.n[0] + T2C - 1) / T2C, (g.n[1] + T2C - 1) / T2C);
   auto go = [&](auto cc, auto aa, auto vv, auto ss) {
     k_char_tile2d<decltype(cc)::value, decltype(aa)::value, decltype(vv)::value, decltype(ss)::value>
-        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, b, cA, cB, first, mode, theta, suth, wrap);
+        <<<grid, 256, 0, s>>>(Q, R, Qo, Qn, g, ph, b, cA, cB, first, mode, theta, suth, wrap, PK);
   };
   if (conv == CONV_WFILTER) {  // SimpleAverage (WENO_filter.py:324)
     go(std::integral_constant<int, CONV_WFILTER>{}, std::integral_constant<int, OSBL_AVG_SIMPLE>{}, std::false_type{},

@@ -147,3 +147,62 @@ def test_sutherland_adjoint_refused():
     b = Block(problem)
     with pytest.raises(OsblError, match="Sutherland"):
         _gpu_vjp(b, q0, np.ones_like(q0))
+
+
+def _shape_case(shape, conv, viscous):
+    problem, _, _ = _kh_visc(32, conv)
+    n0, n1 = shape
+    problem.update(n=[n0, n1], delta=[1.0 / n0, 1.0 / n1], viscous=viscous, dt=0.1 / max(shape))
+    y, x = np.meshgrid(np.arange(n1) / n1, np.arange(n0) / n0, indexing="ij")
+    rho = 1.5 + 0.3 * np.sin(2 * np.pi * (x + y))
+    u, v = 0.3 * np.cos(2 * np.pi * (x - y)), 0.2 * np.sin(2 * np.pi * (x + 0.3)) * np.cos(2 * np.pi * y)
+    p = 2.5 + 0.2 * np.cos(2 * np.pi * (y + 0.1))
+    q0 = np.stack([rho, rho * u, rho * v, p / 0.4 + 0.5 * rho * (u * u + v * v)])
+    return problem, q0, np.random.RandomState(3).normal(size=q0.shape)
+
+
+@pytest.mark.parametrize("shape", [(8, 9), (15, 17), (33, 16), (48, 31)])
+def test_viscous_part_shapes(shape):
+    """The viscous part of a WENO5-Z block's product (with it less without
+    it) on blocks around whole 16 x 16 tiles, against autograd."""
+    import torch
+    import torch_reference as tr
+    from opensbli_amd.native import Block
+    _say(f"case viscous part of the product {shape}")
+    problem, q0, mu = _shape_case(shape, "weno_z", "const")
+    gk = _gpu_vjp(Block(problem), q0, mu) - _gpu_vjp(Block(dict(problem, viscous="none")), q0, mu)
+    qt = torch.tensor(q0, requires_grad=True)
+    r = tr.viscous(qt, problem["delta"], problem["gama"], VISC["Minf"], VISC["Re"], VISC["Pr"])
+    (gt,) = torch.autograd.grad((r * torch.tensor(mu)).sum(), qt)
+    err = np.abs(gk - gt.numpy()).max() / np.abs(gt.numpy()).max()
+    _say("max rel diff", err)
+    assert err < 1e-10
+
+
+@pytest.mark.parametrize("viscous", ["const", "none"])
+@pytest.mark.parametrize("shape", [(8, 9), (15, 17), (33, 16), (48, 31)])
+def test_gradient_shapes(shape, viscous):
+    """Two RK3 steps backwards of the central scheme on such blocks, for a
+    random linear functional of the state, against autograd.  (Not WENO5-Z:
+    at odd sizes this state's largest wave speed belongs to two points at
+    once, where the local Lax-Friedrichs flux has no derivative.)"""
+    import torch
+    import torch_reference as tr
+    from opensbli_amd.adjoint import integrate
+    from opensbli_amd.native import Block
+    _say(f"case adjoint shapes {shape} {viscous}")
+    problem, q0, mu = _shape_case(shape, "central_skew", viscous)
+    mu = torch.tensor(mu)
+    qd = torch.tensor(q0, device="cuda", requires_grad=True)
+    (integrate(qd, Block(problem), 2, 1) * mu.cuda()).sum().backward()
+    qt = torch.tensor(q0, requires_grad=True)
+    if viscous == "none":
+        qn = tr.integrate(qt, 2, problem["dt"], problem["delta"], problem["gama"])
+    else:
+        qn = tr.integrate_ns(qt, 2, problem["dt"], problem["delta"], problem["gama"], VISC["Minf"], VISC["Re"],
+                             VISC["Pr"])
+    (qn * mu).sum().backward()
+    gk, gt = qd.grad.cpu().numpy(), qt.grad.numpy()
+    err = np.abs(gk - gt).max() / np.abs(gt).max()
+    _say("max rel diff", err)
+    assert err < 1e-10
