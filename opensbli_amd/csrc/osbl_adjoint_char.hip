@@ -150,59 +150,52 @@ __device__ __forceinline__ Dual<N> dsqrt(const Dual<N>& a) {
   return r;
 }
 
-__device__ __forceinline__ double sgn(double x) { return (double)((x > 0.0) - (x < 0.0)); }
-
-// Gradient of weno5z(x0..x4) (the one-division WENO-Z of osbl_device.h) with
-// respect to its five arguments, scaled by gbar; returns the reconstruction
-// itself (the same weights, the candidates' 1/6 applied to each candidate).
+// WENO5-Z of the values x0..x4 (weno5_gap<true> of osbl_device.h: from their
+// differences A, B, C, Dd) and its gradient with respect to them, scaled by
+// gbar; returns the reconstruction.  With Q_r the product of the other two
+// q_i = e_i^2, q = q_0 q_1 q_2 and w_r = 3, 6, 1 the weights are
+// a_r = w_r (tau^2 Q_r + q), the value x2 + sum(a_r c_r) / (6 sum(a_r)).
 __device__ __forceinline__ double weno5z_grad(const double x[5], double gbar, double g[5]) {
-  const double fm2 = x[0], fm1 = x[1], f0 = x[2], f1 = x[3], f2 = x[4];
-  const double t0 = f0 - 2.0 * f1 + f2, s0 = 3.0 * f0 - 4.0 * f1 + f2;
-  const double t1 = fm1 - 2.0 * f0 + f1, s1 = fm1 - f1;
-  const double t2 = fm2 - 2.0 * fm1 + f0, s2 = fm2 - 4.0 * fm1 + 3.0 * f0;
-  constexpr double C13 = 13.0 / 12.0;
-  const double b0 = C13 * t0 * t0 + 0.25 * s0 * s0;
-  const double b1 = C13 * t1 * t1 + 0.25 * s1 * s1;
-  const double b2 = C13 * t2 * t2 + 0.25 * s2 * s2;
-  const double dtau = b0 - b2;  // tau^2 = (b0 - b2)^2
-  const double tt = dtau * dtau;
-  const double e0 = 1.0e-14 + b0, e1 = 1.0e-14 + b1, e2 = 1.0e-14 + b2;
+  constexpr double K = 3.0 / 13.0, EPS = 12.0 / 13.0 * 1.0e-14, S6 = 1.0 / 6.0;
+  const double A = x[1] - x[0], B = x[2] - x[1], C = x[3] - x[2], Dd = x[4] - x[3];
+  const double t0 = Dd - C, t1 = C - B, t2 = B - A;
+  const double s0 = __fma_rn(-2.0, C, t0), s1 = B + C, s2 = __fma_rn(2.0, B, t2);
+  const double k0 = K * s0, k1 = K * s1, k2 = K * s2;
+  const double e0 = __fma_rn(t0, t0, __fma_rn(k0, s0, EPS));
+  const double e1 = __fma_rn(t1, t1, __fma_rn(k1, s1, EPS));
+  const double e2 = __fma_rn(t2, t2, __fma_rn(k2, s2, EPS));
   const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
-  const double A0 = 0.3 * (q0 + tt) * (q1 * q2);
-  const double A1 = 0.6 * (q1 + tt) * (q0 * q2);
-  const double A2 = 0.1 * (q2 + tt) * (q0 * q1);
-  constexpr double S6 = 1.0 / 6.0;
-  const double r0 = (2.0 * f0 + 5.0 * f1 - f2) * S6;
-  const double r1 = (-fm1 + 5.0 * f0 + 2.0 * f1) * S6;
-  const double r2 = (2.0 * fm2 - 7.0 * fm1 + 11.0 * f0) * S6;
-  const double iS = recip_pos(A0 + A1 + A2);
-  const double W = (A0 * r0 + A1 * r1 + A2 * r2) * iS;
+  const double q12 = q1 * q2, q02 = q0 * q2, q01 = q0 * q1, q = q01 * q2;
+  const double tau = e0 - e2, tt = tau * tau;
+  const double a0 = 3.0 * __fma_rn(tt, q12, q), a1 = 6.0 * __fma_rn(tt, q02, q), a2 = __fma_rn(tt, q01, q);
+  const double c0 = __fma_rn(4.0, C, -Dd), c1 = __fma_rn(2.0, C, B), c2 = __fma_rn(5.0, B, -2.0 * A);
+  const double iS = recip_pos(a0 + a1 + a2);
+  const double W = (a0 * c0 + a1 * c1 + a2 * c2) * iS;
   // reverse
-  const double rb0 = A0 * iS * gbar, rb1 = A1 * iS * gbar, rb2 = A2 * iS * gbar;
-  const double Ab0 = (r0 - W) * iS * gbar, Ab1 = (r1 - W) * iS * gbar, Ab2 = (r2 - W) * iS * gbar;
-  const double q12 = q1 * q2, q02 = q0 * q2, q01 = q0 * q1;
-  const double qb0 = Ab0 * 0.3 * q12 + Ab1 * 0.6 * (q1 + tt) * q2 + Ab2 * 0.1 * (q2 + tt) * q1;
-  const double qb1 = Ab0 * 0.3 * (q0 + tt) * q2 + Ab1 * 0.6 * q02 + Ab2 * 0.1 * (q2 + tt) * q0;
-  const double qb2 = Ab0 * 0.3 * (q0 + tt) * q1 + Ab1 * 0.6 * (q1 + tt) * q0 + Ab2 * 0.1 * q01;
-  const double ttb = Ab0 * 0.3 * q12 + Ab1 * 0.6 * q02 + Ab2 * 0.1 * q01;
-  double bb0 = 2.0 * e0 * qb0, bb1 = 2.0 * e1 * qb1, bb2 = 2.0 * e2 * qb2;
-  const double db = 2.0 * dtau * ttb;
-  bb0 += db;
-  bb2 -= db;
-  const double tb0 = 2.0 * C13 * t0 * bb0, sb0 = 0.5 * s0 * bb0;
-  const double tb1 = 2.0 * C13 * t1 * bb1, sb1 = 0.5 * s1 * bb1;
-  const double tb2 = 2.0 * C13 * t2 * bb2, sb2 = 0.5 * s2 * bb2;
-  // fm2
-  g[0] = tb2 + sb2 + rb2 * (2.0 * S6);
-  // fm1
-  g[1] = tb1 + sb1 - 2.0 * tb2 - 4.0 * sb2 - rb1 * S6 - rb2 * (7.0 * S6);
-  // f0
-  g[2] = tb0 + 3.0 * sb0 - 2.0 * tb1 + tb2 + 3.0 * sb2 + rb0 * (2.0 * S6) + rb1 * (5.0 * S6) + rb2 * (11.0 * S6);
-  // f1
-  g[3] = -2.0 * tb0 - 4.0 * sb0 + tb1 - sb1 + rb0 * (5.0 * S6) + rb1 * (2.0 * S6);
-  // f2
-  g[4] = tb0 + sb0 - rb0 * S6;
-  return W;
+  const double gi = gbar * S6 * iS;
+  const double cb0 = a0 * gi, cb1 = a1 * gi, cb2 = a2 * gi;
+  const double b0 = 3.0 * gi * (c0 - W), b1 = 6.0 * gi * (c1 - W), b2 = gi * (c2 - W);  // of a_r / w_r, times w_r
+  const double qb = b0 + b1 + b2;
+  const double ttb = b0 * q12 + b1 * q02 + b2 * q01;
+  const double u0 = b0 * tt, u1 = b1 * tt, u2 = b2 * tt;  // of Q_r
+  const double db = tau * ttb;                            // half of tau's, as the d_i are of e_i's
+  const double d0 = __fma_rn(e0, u1 * q2 + u2 * q1 + qb * q12, db);
+  const double d1 = e1 * (u0 * q2 + u2 * q0 + qb * q02);
+  const double d2 = __fma_rn(e2, u0 * q1 + u1 * q0 + qb * q01, -db);
+  const double f0 = 4.0 * d0, f1 = 4.0 * d1, f2 = 4.0 * d2;
+  const double tb0 = f0 * t0, tb1 = f1 * t1, tb2 = f2 * t2;
+  const double sb0 = f0 * k0, sb1 = f1 * k1, sb2 = f2 * k2;
+  // t0 = D - C, s0 = D - 3 C; t1 = C - B, s1 = B + C; t2 = B - A, s2 = 3 B - A
+  const double gA = -(tb2 + sb2) - 2.0 * cb2;
+  const double gB = (tb2 - tb1) + __fma_rn(3.0, sb2, sb1) + __fma_rn(5.0, cb2, cb1);
+  const double gC = (tb1 - tb0) + __fma_rn(-3.0, sb0, sb1) + __fma_rn(4.0, cb0, 2.0 * cb1);
+  const double gD = tb0 + sb0 - cb0;
+  g[0] = -gA;
+  g[1] = gA - gB;
+  g[2] = gB - gC + gbar;
+  g[3] = gC - gD;
+  g[4] = gD;
+  return __fma_rn(S6, W, x[2]);
 }
 
 // Adjoints of the averaged state's symbols (AvgT's members).
@@ -385,38 +378,27 @@ __device__ __forceinline__ void average_rev(const Pt<ND>& L, const Pt<ND>& R, co
   gR[0] += rRb;
 }
 
-// |lambda_K| at a point and its derivative with respect to (u_D, a)
+// lambda_K = u_D + lam_sign<ND, K>() a
 template <int ND, int K>
-__device__ __forceinline__ double lam_point(double ud, double a, double& dud, double& da) {
-  double l;
-  if constexpr (ND == 1) {
-    if constexpr (K == 0) { l = ud - a; dud = 1.0; da = -1.0; }
-    else if constexpr (K == 1) { l = ud; dud = 1.0; da = 0.0; }
-    else { l = ud + a; dud = 1.0; da = 1.0; }
-  } else {
-    constexpr int NV = ND + 2;
-    if constexpr (K == NV - 2) { l = ud + a; dud = 1.0; da = 1.0; }
-    else if constexpr (K == NV - 1) { l = ud - a; dud = 1.0; da = -1.0; }
-    else { l = ud; dud = 1.0; da = 0.0; }
-  }
-  const double s = sgn(l);
-  dud *= s;
-  da *= s;
-  return fabs(l);
+__device__ constexpr double lam_sign() {
+  if constexpr (ND == 1) return (double)(K - 1);
+  else return K == ND ? 1.0 : (K == ND + 1 ? -1.0 : 0.0);
 }
 
-// Accumulator of the VJP's contributions g[p][m] (window point p, variable m)
-// in a lane's own LDS column: an atomic add that returns nothing, so no
-// register waits for the old value (every lane owns its column: no contention)
+// A lane's own LDS column of 6 x NV values: for every window point p first
+// its characteristic fields' adjoints, then its contributions g[p][m]
 template <int ND>
-struct LdsAcc {
-  double* s;   // slot (0, 0) of this lane
-  int stride;  // doubles between slots
-  __device__ __forceinline__ void add(int p, int m, double v) const { atomicAdd(&s[(p * (ND + 2) + m) * stride], v); }
+struct LdsCol {
+  double* s;   // value (0, 0) of this lane
+  int stride;  // doubles between values
+  __device__ __forceinline__ double& at(int p, int r) const { return s[(p * (ND + 2) + r) * stride]; }
 };
 
-// g[p][m] += (d F_{i+1/2} / d Q_p)^T nu for the window w = Q_{i-2..i+3}
-// (points 0..5, read through the LdsWindow accessors)
+// g[p][m] = (d F_{i+1/2} / d Q_p)^T nu for the window w = Q_{i-2..i+3}
+// (points 0..5, read through the LdsWindow accessors).  The state's part is
+// L^T times the adjoints of the characteristic states: those are stored per
+// field and point and multiplied by L once at the end, not added to g field by
+// field (84 LDS additions per 2-D interface).
 template <int ND, int D, int AVG, class W, class G>
 __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2], const Phys& ph, const G& g) {
   constexpr int NV = ND + 2, NS = ND + 2;  // averaged symbols: rho, a, u_0..u_{ND-1}
@@ -445,10 +427,22 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
 #pragma unroll
   for (int p = 0; p < 6; ++p) { nud[p] = 0.0; npp[p] = 0.0; na[p] = 0.0; }
 
+  // ends a part of the work: what follows re-reads its points, and no part is
+  // scheduled into another's registers
+  auto step = [](double& x) {
+    asm volatile("" : "+v"(x) : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
   auto field = [&](auto kc) {
     constexpr int K = decltype(kc)::value;
     constexpr unsigned LM = lmask<ND, D, K>();
     constexpr unsigned RM = rmask<ND, D, K>();
+    auto lp_of = [](double ud, const double* l) {  // cf = u_D cs + p lp, lp = l_{1+D} + u_D l_E
+      double v = 0.0;
+      if constexpr ((LM >> (1 + D)) & 1u) v = l[1 + D];
+      if constexpr ((LM >> (NV - 1)) & 1u) v += ud * l[NV - 1];
+      return v;
+    };
     double l[NV], r[NV];
 #pragma unroll
     for (int m = 0; m < NV; ++m) { l[m] = 0.0; r[m] = 0.0; }
@@ -465,44 +459,50 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
       rcol<ND, D, K>(v, ph, r);
     }
     // lambda_max and its first maximising point
-    double lam = 0.0, dlu = 0.0, dla = 0.0;
+    constexpr double LS = lam_sign<ND, K>();
+    double lsel = 0.0;
     int pst = -1;
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
-      double du_, da_;
-      const double lp = lam_point<ND, K>(w.u(p, D), w.a(p), du_, da_);
-      if (lp > lam) {
-        lam = lp;
+      const double lp = LS == 0.0 ? w.u(p, D) : __fma_rn(LS, w.a(p), w.u(p, D));
+      if (fabs(lp) > fabs(lsel)) {
+        lsel = lp;
         pst = p;
-        dlu = du_;
-        dla = da_;
       }
     }
-    double cs[6], lpv[6], fp[6], fm[6];
+    double lam = fabs(lsel);
+    const double dlu = lsel < 0.0 ? -1.0 : 1.0, dla = LS * dlu;
+    step(lam);
+    double cs[6], cf[6];
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
       double c = 0.0;
 #pragma unroll
       for (int m = 0; m < NV; ++m)
         if ((LM >> m) & 1u) c += l[m] * w.q(p, m);
-      double lpp = 0.0;
-      if constexpr ((LM >> (1 + D)) & 1u) lpp = l[1 + D];
-      if constexpr ((LM >> (NV - 1)) & 1u) lpp += w.u(p, D) * l[NV - 1];
-      const double cf = w.u(p, D) * c + w.pr(p) * lpp;
       cs[p] = c;
-      lpv[p] = lpp;
-      fp[p] = 0.5 * (cf + lam * c);
-      fm[p] = 0.5 * (cf - lam * c);
+      cf[p] = w.u(p, D) * c + w.pr(p) * lp_of(w.u(p, D), l);
     }
+    step(cf[5]);
     // F += r rc: rc's adjoint, then the two reconstructions (values and
     // gradients from one evaluation of their weights each)
     double nrc = 0.0;
 #pragma unroll
     for (int m = 0; m < NV; ++m)
       if ((RM >> m) & 1u) nrc += r[m] * nu[m];
-    double gp[5], gm[5];
-    const double fmr[5] = {fm[5], fm[4], fm[3], fm[2], fm[1]};
-    const double rc = weno5z_grad(fp, nrc, gp) + weno5z_grad(fmr, nrc, gm);
+    double gp[5], gm[5], x[5];
+#pragma unroll
+    for (int p = 0; p < 5; ++p) x[p] = 0.5 * __fma_rn(lam, cs[p], cf[p]);
+    double rc = weno5z_grad(x, nrc, gp);
+#pragma unroll
+    for (int p = 0; p < 5; ++p) asm volatile("" : "+v"(gp[p]));
+    step(rc);
+#pragma unroll
+    for (int p = 0; p < 5; ++p) x[p] = 0.5 * __fma_rn(-lam, cs[5 - p], cf[5 - p]);
+    rc += weno5z_grad(x, nrc, gm);
+#pragma unroll
+    for (int p = 0; p < 5; ++p) asm volatile("" : "+v"(gm[p]));
+    step(rc);
     double nr[NV];
 #pragma unroll
     for (int m = 0; m < NV; ++m) nr[m] = ((RM >> m) & 1u) ? rc * nu[m] : 0.0;
@@ -527,10 +527,9 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
       const double ncf = 0.5 * (a_ + b_);
       double ncs = 0.5 * lam * (a_ - b_);
       nlam += 0.5 * cs[p] * (a_ - b_);
-      // cf = u_D cs + p lp, lp = l_{1+D} + u_D l_E
       ncs += w.u(p, D) * ncf;
       nud[p] += cs[p] * ncf;
-      npp[p] += lpv[p] * ncf;
+      npp[p] += lp_of(w.u(p, D), l) * ncf;
       if constexpr ((LM >> (1 + D)) & 1u) nl[1 + D] += w.pr(p) * ncf;
       if constexpr ((LM >> (NV - 1)) & 1u) {
         nl[NV - 1] += w.pr(p) * w.u(p, D) * ncf;
@@ -539,17 +538,17 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
       // cs = sum_m l_m q_m
 #pragma unroll
       for (int m = 0; m < NV; ++m)
-        if ((LM >> m) & 1u) {
-          g.add(p, m, l[m] * ncs);
-          nl[m] += w.q(p, m) * ncs;
-        }
+        if ((LM >> m) & 1u) nl[m] += w.q(p, m) * ncs;
+      g.at(p, K) = ncs;
+      asm volatile("" : "+v"(nud[p]), "+v"(npp[p]));
+      step(nlam);
     }
     // lambda_max
 #pragma unroll
     for (int p = 0; p < 6; ++p)
       if (p == pst) {
         nud[p] += dlu * nlam;
-        na[p] += dla * nlam;
+        if constexpr (LS != 0.0) na[p] += dla * nlam;
       }
     if constexpr (ND == 1) {
 #pragma unroll
@@ -582,6 +581,7 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
     }
   }
 
+  step(nud[0]);
   // averaged state -> the two states
   if constexpr (ND == 1) {
     b.rho = nvs[0];
@@ -590,21 +590,26 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
   } else {
     finish_avg_rev<ND>(v, ph, b);
   }
+  double gl[NV], gr[NV];
+#pragma unroll
+  for (int m = 0; m < NV; ++m) { gl[m] = 0.0; gr[m] = 0.0; }
   {
     Pt<ND> L, R;
     w.point(2, L);
     w.point(3, R);
-    double gl[NV], gr[NV];
-#pragma unroll
-    for (int m = 0; m < NV; ++m) { gl[m] = 0.0; gr[m] = 0.0; }
     average_rev<ND, AVG>(L, R, ph, b, gl, gr);
-#pragma unroll
-    for (int m = 0; m < NV; ++m) {
-      g.add(2, m, gl[m]);
-      g.add(3, m, gr[m]);
-    }
   }
-  // u_D, p, a of every point -> its conservative variables
+#pragma unroll
+  for (int m = 0; m < NV; ++m) asm volatile("" : "+v"(gl[m]), "+v"(gr[m]));
+  step(nud[0]);
+  double l[NV][NV];
+  sfor<0, NV>([&](auto kc) {
+    constexpr int K = decltype(kc)::value;
+#pragma unroll
+    for (int m = 0; m < NV; ++m) l[K][m] = 0.0;
+    lrow<ND, D, K>(v, ph, l[K]);
+  });
+  // characteristic states, u_D, p, a of every point -> its conservative variables
 #pragma unroll
   for (int p = 0; p < 6; ++p) {
     const double rho = w.q(p, 0), ir = recip_pos(rho);
@@ -617,13 +622,25 @@ __device__ __forceinline__ void char_flux_vjp(const W& w, const double nu[ND + 2
     double g0 = -na[p] * 0.5 * a * ir;
     // p = (gama-1)(E - |rho u|^2 / (2 rho))
     g0 += np_ * ph.gm1 * 0.5 * uu;
-#pragma unroll
-    for (int m = 0; m < ND; ++m) g.add(p, 1 + m, -np_ * ph.gm1 * w.u(p, m));
-    g.add(p, NV - 1, np_ * ph.gm1);
     // u_D = rhou_D / rho
     g0 += -nud[p] * w.u(p, D) * ir;
-    g.add(p, 1 + D, nud[p] * ir);
-    g.add(p, 0, g0);
+    double o[NV];
+    o[0] = g0;
+#pragma unroll
+    for (int m = 0; m < ND; ++m) o[1 + m] = -np_ * ph.gm1 * w.u(p, m);
+    o[1 + D] += nud[p] * ir;
+    o[NV - 1] = np_ * ph.gm1;
+    sfor<0, NV>([&](auto kc) {
+      constexpr int K = decltype(kc)::value;
+      constexpr unsigned LM = lmask<ND, D, K>();
+      const double n = g.at(p, K);
+#pragma unroll
+      for (int m = 0; m < NV; ++m)
+        if ((LM >> m) & 1u) o[m] = __fma_rn(l[K][m], n, o[m]);
+    });
+#pragma unroll
+    for (int m = 0; m < NV; ++m) g.at(p, m) = o[m] + (p == 2 ? gl[m] : (p == 3 ? gr[m] : 0.0));
+    if (p < 5) step(nud[p + 1]);
   }
 }
 
@@ -658,6 +675,12 @@ __device__ __forceinline__ void vjp_line(long long line, int n0, int n1, long lo
 // twice) and no partial sums leave the wave.
 //   ACC = false: out1 = c (A + B) + V (and out2 = A + B when given);
 //   ACC = true:  out1 += V.
+// What bounds it is FP64 issue at two waves per SIMD: ~2900 VALU instructions
+// per 64 interfaces, 256 registers with ~30 values spilled across the fields
+// (330 and one wave per SIMD without the bound).  512^2, ten steps' gradient:
+// 11.0 ms with reconstructions and their gradients from values and 84 LDS
+// additions per interface, 10.4 from differences at two waves, 10.3 with L
+// applied once, 9.9 with the largest wave speed's sign taken once.
 constexpr int VJW = 2;         // waves per block
 constexpr int VJP = 64 + 5;    // points staged per chunk
 constexpr int VJSTEP = 59;     // cells completed per chunk
@@ -720,9 +743,7 @@ __device__ __forceinline__ void vjp_chunk(long long wid, int lane, double (*S)[V
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (int r = 0; r < 6 * NV; ++r) G[r][lane] = 0.0;
-  char_flux_vjp<ND, D, AVG>(LdsWindow<ND>{&S[0][lane], VJP}, nu, ph, LdsAcc<ND>{&G[0][lane], 64});
+  char_flux_vjp<ND, D, AVG>(LdsWindow<ND>{&S[0][lane], VJP}, nu, ph, LdsCol<ND>{&G[0][lane], 64});
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -752,7 +773,7 @@ __device__ __forceinline__ void vjp_chunk(long long wid, int lane, double (*S)[V
 }
 
 template <int ND, int D, int AVG, bool ACC>
-__global__ void __launch_bounds__(64 * VJW) k_char_vjp_lanes(const double* __restrict__ Qs,
+__global__ void __launch_bounds__(64 * VJW, 2) k_char_vjp_lanes(const double* __restrict__ Qs,
                                                              const double* __restrict__ A,
                                                              const double* __restrict__ B, double alpha, double beta,
                                                              double c, double* __restrict__ out1,
@@ -780,13 +801,13 @@ __global__ void __launch_bounds__(64 * VJW) k_char_vjp_lanes(const double* __res
 }
 
 // Both directions of a 2-D VJP in one launch, so that the y waves fill the
-// SIMDs the x waves leave idle in their last round (one wave per SIMD):
+// SIMDs the x waves leave idle in their last round (two waves per SIMD):
 // x waves as k_char_vjp_lanes<2, 0, AVG, false> (out1, out2), y waves write
 // their V to vy, which k_add_packed then adds to out1.  With both block
 // counts multiples of 8, each XCD takes an eighth of the x blocks and then an
 // eighth of the y blocks, in order; otherwise blocks run in launch order.
 template <int AVG>
-__global__ void __launch_bounds__(64 * VJW) k_char_vjp_xy(const double* __restrict__ Qs, const double* __restrict__ A,
+__global__ void __launch_bounds__(64 * VJW, 2) k_char_vjp_xy(const double* __restrict__ Qs, const double* __restrict__ A,
                                                           const double* __restrict__ B, double alpha, double beta,
                                                           double c, double* __restrict__ out1,
                                                           double* __restrict__ out2, double* __restrict__ vy, int n0,
