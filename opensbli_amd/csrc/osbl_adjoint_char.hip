@@ -8,8 +8,8 @@
 // slides the forward 6-point window along a grid line; per interface it
 // re-evaluates the forward flux of every characteristic field and runs it
 // backwards:
-//   * the reconstructions through a hand-written reverse of the one-division
-//     WENO-Z weights (tau^2 is smooth; no branch),
+//   * the reconstructions through a hand-written reverse of the WENO-Z
+//     weights in difference form (tau^2 is smooth; no branch),
 //   * lambda_max = max_p |lambda(p)| to its first maximising point (the
 //     subgradient the forward's max picks),
 //   * the characteristic projections CS = L.Q, CF = u_D CS + p (L_{1+D} + u_D L_E),
@@ -18,8 +18,8 @@
 //     1-D eigensystem),
 //   * the constituent relations u_D, p, a of every stencil point.
 // The lanes of a wave take 64 consecutive interfaces of a grid line: the
-// chunk's points sit in LDS with their constituent relations, every lane adds
-// its interface's contributions to its own LDS column, and each cell gathers
+// chunk's points sit in LDS with their constituent relations, every lane leaves
+// its interface's contributions in its own LDS column, and each cell gathers
 // the six contributions that reach it from its neighbours' columns; no
 // partial sums leave the wave.
 #include <algorithm>

@@ -466,96 +466,8 @@ __device__ __forceinline__ void rcol(const AvgT<ND, T>& v, const Phys& ph, T r[N
   }
 }
 
-// |lambda_K| at a stencil point from its own u_D and a (shock_capturing.py:512-536)
-template <int ND, int D, int K>
-__device__ __forceinline__ double abs_lambda_ua(double ud, double a) {
-  if constexpr (ND == 1) {
-    if constexpr (K == 0) return fabs(ud - a);
-    else if constexpr (K == 1) return fabs(ud);
-    else return fabs(ud + a);
-  } else {
-    constexpr int NV = ND + 2;
-    if constexpr (K == NV - 2) return fabs(ud + a);
-    else if constexpr (K == NV - 1) return fabs(ud - a);
-    else return fabs(ud);
-  }
-}
-template <int ND, int D, int K>
-__device__ __forceinline__ double abs_lambda(const Pt<ND>& s) {
-  return abs_lambda_ua<ND, D, K>(s.u[D], s.a);
-}
-
-// ---------------------------------------------------------------------------
-// Reconstructions at i+1/2.  Arguments are the 6 points f[-2..3] in the
-// orientation of the "right" reconstruction (weno.py side +1, applied to
-// f+).  The left reconstruction (side -1, applied to f-) is the right one
-// applied to the mirrored points f[3-p] -- except for TENO6, whose
-// right-side fourth indicator has the unsquared 781/720 term
-// (teno.py:166-167), hence the QUIRK flag.
-// ---------------------------------------------------------------------------
-
-// WENO5-Z (weno.py:283-338) with eps = 1e-14, p = 2.  The weights are
-// alpha_r = d_r (1 + tau^2/b_r^2), b_r = eps + beta_r; multiplying every
-// alpha_r by b0^2 b1^2 b2^2 leaves omega_r = alpha_r / sum(alpha) unchanged
-// and needs one division instead of four.
-// numerator and denominator of the WENO5-Z value (value = num/den)
-__device__ __forceinline__ void weno5z_nd(double fm2, double fm1, double f0, double f1, double f2, double& num,
-                                          double& den) {
-  const double t0 = f0 - 2.0 * f1 + f2, s0 = 3.0 * f0 - 4.0 * f1 + f2;
-  const double t1 = fm1 - 2.0 * f0 + f1, s1 = fm1 - f1;
-  const double t2 = fm2 - 2.0 * fm1 + f0, s2 = fm2 - 4.0 * fm1 + 3.0 * f0;
-  constexpr double C13 = 13.0 / 12.0;
-  const double b0 = C13 * t0 * t0 + 0.25 * s0 * s0;
-  const double b1 = C13 * t1 * t1 + 0.25 * s1 * s1;
-  const double b2 = C13 * t2 * t2 + 0.25 * s2 * s2;
-  const double tau = fabs(b0 - b2);
-  const double tt = tau * tau;
-  const double e0 = 1.0e-14 + b0, e1 = 1.0e-14 + b1, e2 = 1.0e-14 + b2;
-  const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
-  const double A0 = 0.3 * (q0 + tt) * (q1 * q2);
-  const double A1 = 0.6 * (q1 + tt) * (q0 * q2);
-  const double A2 = 0.1 * (q2 + tt) * (q0 * q1);
-  // the candidates' common factor 1/6 moves into the denominator
-  const double r0 = 2.0 * f0 + 5.0 * f1 - f2;
-  const double r1 = -fm1 + 5.0 * f0 + 2.0 * f1;
-  const double r2 = 2.0 * fm2 - 7.0 * fm1 + 11.0 * f0;
-  num = A0 * r0 + A1 * r1 + A2 * r2;
-  den = 6.0 * (A0 + A1 + A2);
-}
-
-// n1/d1 + n2/d2 with one division: (n1 d2 + n2 d1)/(d1 d2).  The weights'
-// denominators grow like beta^6 (at least ~1e-85 from eps), so d1 d2 is a
-// normal number unless |f| exceeds ~1e12; then the two quotients are formed
-// separately.
-__device__ __forceinline__ double sum_quotients(double n1, double d1, double n2, double d2) {
-  const double dd = d1 * d2;
-  if (dd < 1.0e300) return quot_pos(n1 * d2 + n2 * d1, dd);
-  return n1 / d1 + n2 / d2;
-}
-
-// WENO5-JS (weno.py:341-369) with eps = 1e-6: alpha_r = d_r/(eps+beta_r)^2,
-// rewritten as d_r * prod_{s!=r} (eps+beta_s)^2 with one division.
-__device__ __forceinline__ void weno5js_nd(double fm2, double fm1, double f0, double f1, double f2, double& num,
-                                           double& den) {
-  const double t0 = f0 - 2.0 * f1 + f2, s0 = 3.0 * f0 - 4.0 * f1 + f2;
-  const double t1 = fm1 - 2.0 * f0 + f1, s1 = fm1 - f1;
-  const double t2 = fm2 - 2.0 * fm1 + f0, s2 = fm2 - 4.0 * fm1 + 3.0 * f0;
-  constexpr double C13 = 13.0 / 12.0;
-  const double e0 = 1.0e-6 + (C13 * t0 * t0 + 0.25 * s0 * s0);
-  const double e1 = 1.0e-6 + (C13 * t1 * t1 + 0.25 * s1 * s1);
-  const double e2 = 1.0e-6 + (C13 * t2 * t2 + 0.25 * s2 * s2);
-  const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
-  const double A0 = 0.3 * (q1 * q2), A1 = 0.6 * (q0 * q2), A2 = 0.1 * (q0 * q1);
-  // the candidates' common factor 1/6 moves into the denominator
-  const double r0 = 2.0 * f0 + 5.0 * f1 - f2;
-  const double r1 = -fm1 + 5.0 * f0 + 2.0 * f1;
-  const double r2 = 2.0 * fm2 - 7.0 * fm1 + 11.0 * f0;
-  num = A0 * r0 + A1 * r1 + A2 * r2;
-  den = 6.0 * (A0 + A1 + A2);
-}
-
-// WENO5-JS as above, also returning the shock sensor of its non-linear
-// weights (weno.py:415-431, normalised, sensor_theta = 4):
+// WENO5-JS (weno.py:341-369, eps = 1e-6) of values f[-2..2], also returning the
+// shock sensor of its non-linear weights (weno.py:415-431, normalised, sensor_theta = 4):
 // rj = sum_r |omega_r/d_r - 1|^4 / (|1/min d - 1|^4 + 2) = (...)/6563.
 __device__ __forceinline__ double weno5js_sensor(double fm2, double fm1, double f0, double f1, double f2, double& rj) {
   const double t0 = f0 - 2.0 * f1 + f2, s0 = 3.0 * f0 - 4.0 * f1 + f2;
@@ -598,124 +510,6 @@ constexpr int CONV_WFILTER = 16;
 __device__ __forceinline__ double pow6(double x) {
   const double x2 = x * x;
   return x2 * x2 * x2;
-}
-
-// TENO5 / TENO6 (teno.py:57-234, 407-465):
-// alpha_r = (1 + tau/(eps + beta_r))^6, delta_r = 0 if alpha_r*(1/sum alpha) < C_T,
-// omega_r = d_r delta_r / sum(d delta).
-// Numerator and denominator of the value (value = num/den).  The four (three)
-// quotients tau/(eps + beta_r) share one division: with e_r = eps + beta_r,
-// 1/e_0 = e_1 e_2 e_3 / (e_0 e_1 e_2 e_3) and so on, unless that product
-// leaves the normal range (then each quotient is formed on its own).  The
-// cut-off compares alpha_r * (1/sum alpha) with C_T as written.
-template <bool SIX, bool QUIRK>
-__device__ __forceinline__ void teno_nd(double fm2, double fm1, double f0, double f1, double f2, double f3,
-                                        double eps, double ct, double& num, double& den) {
-  constexpr double C13 = 13.0 / 12.0;
-  double q;
-  q = fm1 - f1;
-  double b0 = 0.25 * q * q;
-  q = fm1 - 2.0 * f0 + f1;
-  b0 += C13 * q * q;
-  q = 3.0 * f0 - 4.0 * f1 + f2;
-  double b1 = 0.25 * q * q;
-  q = f0 - 2.0 * f1 + f2;
-  b1 += C13 * q * q;
-  q = fm2 - 4.0 * fm1 + 3.0 * f0;
-  double b2 = 0.25 * q * q;
-  q = fm2 - 2.0 * fm1 + f0;
-  b2 += C13 * q * q;
-  constexpr double S6 = 1.0 / 6.0;
-  const double r0 = (-fm1 + 5.0 * f0 + 2.0 * f1) * S6;
-  const double r1 = (2.0 * f0 + 5.0 * f1 - f2) * S6;
-  const double r2 = (2.0 * fm2 - 7.0 * fm1 + 11.0 * f0) * S6;
-  const double e0 = eps + b0, e1 = eps + b1, e2 = eps + b2;
-  if constexpr (SIX) {
-    q = -11.0 * f0 + 18.0 * f1 - 9.0 * f2 + 2.0 * f3;
-    double b3 = (1.0 / 36.0) * q * q;
-    q = 2.0 * f0 - 5.0 * f1 + 4.0 * f2 - f3;
-    b3 += C13 * q * q;
-    q = -f0 + 3.0 * f1 - 3.0 * f2 + f3;
-    if constexpr (QUIRK) b3 += (781.0 / 720.0) * q;
-    else b3 += (781.0 / 720.0) * q * q;
-    const double r3 = (3.0 * f0 + 13.0 * f1 - 5.0 * f2 + f3) * (1.0 / 12.0);
-    const double tau = fabs(b3 - (b0 + b2 - 4.0 * b1) * S6);
-    const double e3 = eps + b3;
-    const double p01 = e0 * e1, p23 = e2 * e3;
-    const double pr = p01 * p23;
-    double a0, a1, a2, a3;
-    if (fabs(pr) > 1.0e-300 && fabs(pr) < 1.0e300) {
-      const double tp = quot_pos(tau, pr);
-      a0 = pow6(1.0 + (e1 * p23) * tp);
-      a1 = pow6(1.0 + (e0 * p23) * tp);
-      a2 = pow6(1.0 + (e3 * p01) * tp);
-      a3 = pow6(1.0 + (e2 * p01) * tp);
-    } else {
-      a0 = pow6(1.0 + tau / e0);
-      a1 = pow6(1.0 + tau / e1);
-      a2 = pow6(1.0 + tau / e2);
-      a3 = pow6(1.0 + tau / e3);
-    }
-    const double ias = recip_pos(a0 + a1 + a2 + a3);
-    const double d0 = (a0 * ias < ct) ? 0.0 : 1.0;
-    const double d1 = (a1 * ias < ct) ? 0.0 : 1.0;
-    const double d2 = (a2 * ias < ct) ? 0.0 : 1.0;
-    const double d3 = (a3 * ias < ct) ? 0.0 : 1.0;
-    constexpr double D0 = 231.0 / 500.0, D1 = 3.0 / 10.0, D2 = 27.0 / 500.0, D3 = 23.0 / 125.0;
-    const double w0 = D0 * d0, w1 = D1 * d1, w2 = D2 * d2, w3 = D3 * d3;
-    num = w0 * r0 + w1 * r1 + w2 * r2 + w3 * r3;
-    den = w0 + w1 + w2 + w3;
-  } else {
-    const double tau = fabs(b0 - b2);
-    const double p01 = e0 * e1;
-    const double pr = p01 * e2;
-    double a0, a1, a2;
-    if (fabs(pr) > 1.0e-300 && fabs(pr) < 1.0e300) {
-      const double tp = quot_pos(tau, pr);
-      a0 = pow6(1.0 + (e1 * e2) * tp);
-      a1 = pow6(1.0 + (e0 * e2) * tp);
-      a2 = pow6(1.0 + p01 * tp);
-    } else {
-      a0 = pow6(1.0 + tau / e0);
-      a1 = pow6(1.0 + tau / e1);
-      a2 = pow6(1.0 + tau / e2);
-    }
-    const double ias = recip_pos(a0 + a1 + a2);
-    const double d0 = (a0 * ias < ct) ? 0.0 : 1.0;
-    const double d1 = (a1 * ias < ct) ? 0.0 : 1.0;
-    const double d2 = (a2 * ias < ct) ? 0.0 : 1.0;
-    constexpr double D0 = 11.0 / 20.0, D1 = 4.0 / 10.0, D2 = 1.0 / 20.0;
-    const double w0 = D0 * d0, w1 = D1 * d1, w2 = D2 * d2;
-    num = w0 * r0 + w1 * r1 + w2 * r2;
-    den = w0 + w1 + w2;
-  }
-}
-
-// Sum of the right reconstruction of f+ and the left reconstruction of f-
-// (shock_capturing.py:257-265) for one characteristic field.
-template <int CONV>
-__device__ __forceinline__ double recon_pair(const double fp[6], const double fm[6], double eps, double ct) {
-  if constexpr (CONV == OSBL_CONV_WENO_Z) {
-    double n1, d1, n2, d2;
-    weno5z_nd(fp[0], fp[1], fp[2], fp[3], fp[4], n1, d1);
-    weno5z_nd(fm[5], fm[4], fm[3], fm[2], fm[1], n2, d2);
-    return sum_quotients(n1, d1, n2, d2);
-  } else if constexpr (CONV == OSBL_CONV_WENO_JS) {
-    double n1, d1, n2, d2;
-    weno5js_nd(fp[0], fp[1], fp[2], fp[3], fp[4], n1, d1);
-    weno5js_nd(fm[5], fm[4], fm[3], fm[2], fm[1], n2, d2);
-    return sum_quotients(n1, d1, n2, d2);
-  } else if constexpr (CONV == OSBL_CONV_TENO6) {
-    double n1, d1, n2, d2;
-    teno_nd<true, true>(fp[0], fp[1], fp[2], fp[3], fp[4], fp[5], eps, ct, n1, d1);
-    teno_nd<true, false>(fm[5], fm[4], fm[3], fm[2], fm[1], fm[0], eps, ct, n2, d2);
-    return sum_quotients(n1, d1, n2, d2);
-  } else {
-    double n1, d1, n2, d2;
-    teno_nd<false, false>(fp[0], fp[1], fp[2], fp[3], fp[4], fp[5], eps, ct, n1, d1);
-    teno_nd<false, false>(fm[5], fm[4], fm[3], fm[2], fm[1], fm[0], eps, ct, n2, d2);
-    return sum_quotients(n1, d1, n2, d2);
-  }
 }
 
 // ---------------------------------------------------------------------------
