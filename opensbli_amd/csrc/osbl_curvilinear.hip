@@ -209,6 +209,8 @@ __device__ __forceinline__ void curv_flux(const double* __restrict__ s, const Ph
 // update and the halo exchange.  3-D keeps 50 differences in 172 to 200
 // registers: two waves per SIMD (96^3: 70 + 63 + 75 us), as three spill (79 +
 // 79 + 94; TENO6 116 + 115 + 131 against 89 + 80 + 89).
+// Tiles of 63 x 4 along x gained 5 % at 1024^2 and 1 % at 96^3 and waste more on
+// other extents; 31 x 8 along y and z, half cache lines, took 72 and 91 us there.
 // ---------------------------------------------------------------------------
 template <int ND, int D, int CONV, int AVG>
 __global__ void __launch_bounds__(256, ND == 3 ? 2 : 3) k_curv_sweep(const double* __restrict__ Q, const double* __restrict__ M,
