@@ -212,10 +212,12 @@ __global__ void __launch_bounds__(256, 3) k_char_tile2d(const double* __restrict
     const double um[3] = {S[pc][4], S[pc][5], 0.0};
     viscous_assemble<2>(S[pc][9], um, DU, DD, D2T, DT, DMU, ph, suth != 0, r);
   }
-  if (ph.has_force) {
-    r[1] -= ph.force[0];
-    r[2] -= ph.force[1];
-    r[3] -= ph.force[0] * S[pc][4] + ph.force[1] * S[pc][5];
+  if constexpr (CONV != CONV_WFILTER) {  // the filter's R holds flux differences alone
+    if (ph.has_force) {
+      r[1] -= ph.force[0];
+      r[2] -= ph.force[1];
+      r[3] -= ph.force[0] * S[pc][4] + ph.force[1] * S[pc][5];
+    }
   }
   if (PK) {
 #pragma unroll

@@ -112,6 +112,23 @@ def test_weno_filter_with_characteristic_scheme_and_walls(oracle):
     _compare(p, q0, oracle)
 
 
+@pytest.mark.parametrize("sensor", ["constant", "ducros"])
+@pytest.mark.parametrize("conv", ["weno_z", "central_skew"])
+def test_weno_filter_on_a_channel_with_body_force(conv, sensor, oracle):
+    """The filter's flux differences hold no body force: a 2-D channel driven
+    by one, with a control that the interior outside the wall zones shows."""
+    from opensbli_amd.problems import channel
+    _say(f"case weno filter on the channel 32x33 with body force, {conv}, sensor={sensor}")
+    p, q0 = channel(n=(32, 33), conv=conv)
+    p.update(filters={"weno": {"sensor": sensor, "control": 1.0}}, sensor_eps=1e-12)
+    a, b = _compare(p, q0, oracle)
+    r = oracle.RefSolver(dict(p, filters={}))
+    r.set_state(q0)
+    r.run(100)
+    d = np.abs(r.get_state() - b)[:, 8:-8]
+    assert d.max() > 1e-7, d.max()
+
+
 @pytest.mark.parametrize("restart", [False, True])
 def test_sfd(restart, oracle):
     n = (48, 32)
