@@ -100,6 +100,7 @@ __device__ __forceinline__ void line_segment(double (*S)[LINE_NF], int lane, int
 #pragma unroll
       for (int e = 0; e < 8; ++e) S[lane][e] = S[64 + lane][e];
     }
+    line_wave_sync();  // the next points go into slots 64..68
     base += 64;
   }
 }
