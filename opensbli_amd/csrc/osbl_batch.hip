@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -303,6 +304,7 @@ struct osbl_batch {
   double* Qo = nullptr;
   double* stage_buf = nullptr;
   double* host_buf = nullptr;  // pinned: the state of the longest line
+  std::mutex host_mu;          // one line at a time goes through host_buf
   hipStream_t stream = nullptr;
   // staged mode
   int* d_seg_inst = nullptr;
@@ -604,6 +606,7 @@ int osbl_batch_get_state(osbl_batch* b, int inst, double* host) {
   const Inst& in = b->h_inst[inst];
   // one kernel that writes to pinned memory and one wait: 512 instances one
   // by one took 21 ms with a blocking copy per variable
+  std::lock_guard<std::mutex> lock(b->host_mu);
   k_batch_gather<<<(in.n + 255) / 256, 256, 0, b->stream>>>(b->QA + in.off, b->fs, in.n, b->host_buf);
   BCHK(hipGetLastError());
   BCHK(hipStreamSynchronize(b->stream));

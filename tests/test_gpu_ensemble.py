@@ -72,6 +72,20 @@ def test_ensemble_thread_tables_agree():
             assert np.array_equal(a, b)
 
 
+def test_ensemble_states_read_from_several_threads():
+    """Lines read back by eight host threads at once: each gets its own."""
+    from concurrent.futures import ThreadPoolExecutor
+    from opensbli_amd.ensemble import Ensemble
+    _say("case ensemble states read from eight threads")
+    par = _small(ninst=64, seed=13, steps=3)
+    e = Ensemble(par)
+    e.run("persistent")
+    alone = [e.get_state(i) for i in range(64)]
+    with ThreadPoolExecutor(8) as ex:
+        for i, got in enumerate(ex.map(e.get_state, list(range(64)) * 8)):
+            assert np.array_equal(got, alone[i % 64]), i % 64
+
+
 def test_ensemble_vs_oracle(oracle):
     from opensbli_amd.ensemble import Ensemble, instance_problem
     _say("case ensemble vs oracle")
