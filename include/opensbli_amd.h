@@ -98,6 +98,10 @@ typedef struct osbl_config {
   int32_t viscous;     /* OSBL_VISC_* */
   int32_t rk;          /* OSBL_RK* */
   int32_t bc[3][2];    /* OSBL_BC_* per direction and side */
+  /* The nonlinear weights are formed from products of their smoothness
+     indicators: differences of the characteristic fluxes between neighbouring
+     points up to 1e22 (WENO) or 1e75 (TENO), and TENO's eps from 1e-150 on,
+     keep those in the range of a double. */
   double gama, Minf, Re, Pr, dt, eps, teno_ct;
   int32_t bscheme[3][2]; /* OSBL_BS_* per face (faces that modify the central stencils) */
   int32_t stretch[3];    /* 1: direction d is stretched along itself; coordinates via osbl_set_coordinates

@@ -618,9 +618,10 @@ __device__ __forceinline__ void weno5_gap(double A, double B, double C, double D
 
 // TENO5 / TENO6 (teno.py:57-234, 407-465): alpha_r = (1 + tau/e_r)^6,
 // e_r = eps + beta_r; delta_r = 0 where alpha_r < C_T sum(alpha), and
-// omega_r = d_r delta_r / sum(d delta).  The quotients tau/e_r share one
-// division by the product of the e_r.  eps comes at least 1e-70 (osbl_create),
-// so the product stays normal for differences up to ~1e37.
+// omega_r = d_r delta_r / sum(d delta).  The quotients tau/e_r share a
+// division by the product of two e_r (one by the product of all took as many
+// instructions, but leaves the range of a double for differences beyond 1e37
+// or eps below 1e-75; these products hold to 1e75 and 1e-150).
 template <bool SIX, bool QUIRK>
 __device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd, double E, double eps, double ct,
                                          double& num, double& den) {
@@ -644,10 +645,9 @@ __device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd
     const double c3 = 4.5 * C - 2.0 * Dd + 0.5 * E;
     const double tau = fabs(b3 - (b0 + b2 - 4.0 * b1) * (1.0 / 6.0));
     const double e3 = eps + b3;
-    const double p01 = e0 * e1, p23 = e2 * e3;
-    const double tp = quot_near(tau, p01 * p23);
-    const double a0 = pow6(__fma_rn(e1 * p23, tp, 1.0)), a1 = pow6(__fma_rn(e0 * p23, tp, 1.0));
-    const double a2 = pow6(__fma_rn(e3 * p01, tp, 1.0)), a3 = pow6(__fma_rn(e2 * p01, tp, 1.0));
+    const double x01 = quot_near(tau, e0 * e1), x23 = quot_near(tau, e2 * e3);
+    const double a0 = pow6(__fma_rn(e1, x01, 1.0)), a1 = pow6(__fma_rn(e0, x01, 1.0));
+    const double a2 = pow6(__fma_rn(e3, x23, 1.0)), a3 = pow6(__fma_rn(e2, x23, 1.0));
     const double cut = ct * (a0 + a1 + a2 + a3);
     const double w0 = a0 < cut ? 0.0 : 231.0 / 500.0, w1 = a1 < cut ? 0.0 : 3.0 / 10.0;
     const double w2 = a2 < cut ? 0.0 : 27.0 / 500.0, w3 = a3 < cut ? 0.0 : 23.0 / 125.0;
@@ -655,10 +655,9 @@ __device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd
     den = w0 + w1 + w2 + w3;
   } else {
     const double tau = fabs(b0 - b2);
-    const double p01 = e0 * e1;
-    const double tp = quot_near(tau, p01 * e2);
-    const double a0 = pow6(__fma_rn(e1 * e2, tp, 1.0)), a1 = pow6(__fma_rn(e0 * e2, tp, 1.0));
-    const double a2 = pow6(__fma_rn(p01, tp, 1.0));
+    const double x01 = quot_near(tau, e0 * e1);
+    const double a0 = pow6(__fma_rn(e1, x01, 1.0)), a1 = pow6(__fma_rn(e0, x01, 1.0));
+    const double a2 = pow6(1.0 + quot_near(tau, e2));
     const double cut = ct * (a0 + a1 + a2);
     const double w0 = a0 < cut ? 0.0 : 11.0 / 20.0, w1 = a1 < cut ? 0.0 : 4.0 / 10.0, w2 = a2 < cut ? 0.0 : 1.0 / 20.0;
     num = w0 * c0 + w1 * c1 + w2 * c2;

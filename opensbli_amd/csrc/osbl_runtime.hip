@@ -602,7 +602,7 @@ int osbl_create(const osbl_config* cfg, osbl_ctx** out) {
   ph.Re = cfg->Re;
   ph.Pr = cfg->Pr;
   ph.dt = cfg->dt;
-  ph.eps = std::max(cfg->eps, 1.0e-70);  // teno_gap multiplies four of these
+  ph.eps = cfg->eps;
   ph.teno_ct = cfg->teno_ct;
   for (int d = 0; d < 3; ++d) ph.inv_delta[d] = d < c->nd ? 1.0 / cfg->delta[d] : 0.0;
   ph.inv_re = cfg->viscous != OSBL_VISC_NONE ? 1.0 / cfg->Re : 0.0;

@@ -108,3 +108,18 @@ def test_2d_faces(n, bc, oracle):
 def test_2d_central_shapes(n, conv, rk, viscous, bc, oracle):
     problem, q0 = _block(n, conv, bc, rk=rk, viscous=viscous)
     _check(problem, q0, oracle, f"2-D {n} {conv} {rk} {viscous} {bc}")
+
+
+@pytest.mark.parametrize("conv,averaging", [("teno5", "roe"), ("teno6", "simple")])
+@pytest.mark.parametrize("s,eps", [(1.0, 1e-16), (1.0, 1e-100), (1e25, 1e-16), (1e30, 1e-16)])
+def test_2d_rough_state_in_other_units(s, eps, conv, averaging, oracle):
+    """Velocities times s, pressures times s^2 on a rough state, where TENO's
+    cut-off decides: the weights' quotients stay in range with the oracle's."""
+    n = (24, 20)
+    problem, _ = _block(n, conv, "periodic", averaging)
+    problem.update(dt=0.1 * problem["dt"] / s, eps=eps)
+    rs = np.random.RandomState(2)
+    rho, p = (rs.uniform(0.8, 1.2, n[::-1]) for _ in range(2))
+    u = [s * rs.uniform(-0.3, 0.3, n[::-1]) for _ in range(2)]
+    q0 = np.stack([rho] + [rho * v for v in u] + [s * s * p / 0.4 + 0.5 * rho * (u[0] ** 2 + u[1] ** 2)])
+    _check(problem, q0, oracle, f"2-D in units of {s:g}, eps={eps:g} {conv} {averaging}")

@@ -1,5 +1,5 @@
-"""Device code on the CPU (tests/host): osbl_line.h compiled for the host with
-a stand-in for the HIP header, the lanes of a wave as fibers."""
+"""Device code on the CPU (tests/host): osbl_device.h and osbl_line.h compiled
+for the host with a stand-in for the HIP header, the lanes of a wave as fibers."""
 import ctypes
 import os
 import subprocess
@@ -24,6 +24,11 @@ def _compile(tmp, name):
 @pytest.fixture(scope="module")
 def lanes(tmp_path_factory):
     return _compile(tmp_path_factory.mktemp("host"), "line_lanes")
+
+
+@pytest.fixture(scope="module")
+def recon(tmp_path_factory):
+    return _compile(tmp_path_factory.mktemp("host"), "recon")
 
 
 def _segment(lib, q, qo, s0, s1, conv, mode, first, down, dt=1e-3):
@@ -59,3 +64,55 @@ def test_a_line_does_not_depend_on_the_order_of_the_lanes(lanes, n, conv, mode):
             a[:, s0:s1] = b[:, s0:s1]
     for a, b in zip(up, parts):
         assert np.array_equal(a, b)
+
+
+def _dp(a):
+    return a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+
+
+def _teno_reference(d, six, quirk, eps, ct):
+    """The weights from one quotient each (teno.py:57-234, 407-465): value and
+    how near to the cut-off the nearest weight is (relative)."""
+    A, B, C, D, E = (np.ascontiguousarray(d[:, k]) for k in range(5))
+    b = [13 / 12 * (C - B) ** 2 + 0.25 * (B + C) ** 2,
+         13 / 12 * (D - C) ** 2 + 0.25 * (D - 3 * C) ** 2,
+         13 / 12 * (B - A) ** 2 + 0.25 * (3 * B - A) ** 2]
+    c = [B + 2 * C, 4 * C - D, 5 * B - 2 * A]
+    w = [0.55, 0.4, 0.05]
+    tau = np.abs(b[0] - b[2])
+    if six:
+        q3 = C - 2 * D + E
+        b.append((11 * C - 7 * D + 2 * E) ** 2 / 36 + 13 / 12 * (3 * D - 2 * C - E) ** 2 +
+                 781 / 720 * (2 * q3 if quirk else q3 * q3))
+        c.append(4.5 * C - 2 * D + 0.5 * E)
+        w = [0.462, 0.3, 0.054, 0.184]
+        tau = np.abs(b[3] - (b[0] + b[2] - 4 * b[1]) / 6)
+    with np.errstate(all="ignore"):
+        a = [(1 + tau / (eps + x)) ** 6 for x in b]
+        cut = ct * sum(a)
+        near = np.min([np.abs(x / cut - 1) for x in a], axis=0)
+        keep = [np.where(x < cut, 0.0, wr) for x, wr in zip(a, w)]
+        return sum(k * x for k, x in zip(keep, c)) / sum(keep), near
+
+
+@pytest.mark.parametrize("six,quirk", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("eps", [1e-140, 1e-100, 4e-16])
+@pytest.mark.parametrize("scale", [1e-60, 1e-30, 1.0, 1e30, 1e39, 1e52, 1e70])
+def test_teno_weights_over_the_range_of_the_quotients(recon, scale, eps, six, quirk):
+    """Differences and eps for which the product of all indicators leaves the
+    range of a double: the weights are those of the quotients taken one by one
+    (the indicators' rounding, 1e-12, apart; a weight that near to the cut-off
+    may fall on either side)."""
+    rs = np.random.RandomState(5)
+    n = 4000
+    d = scale * rs.standard_normal((n, 5)) * 10.0 ** rs.uniform(-3, 0, (n, 5))
+    d[::7] = 0.0           # a uniform stretch
+    d[1::7] = scale * 0.1  # a linear one
+    num, den = np.empty(n), np.empty(n)
+    f = ctypes.c_double
+    recon.teno(int(six), int(quirk), ctypes.c_long(n), _dp(d), f(eps), f(1e-6), _dp(num), _dp(den))
+    want, near = _teno_reference(d, six, quirk, eps, 1e-6)
+    ok = np.isfinite(want) & ~(near < 1e-9)
+    assert ok.mean() > 0.8
+    err = np.abs(num / den - want)[ok] / scale
+    assert np.all(err <= 1e-12), (err.max(), int((~(err <= 1e-12)).sum()))
