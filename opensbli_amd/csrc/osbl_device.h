@@ -148,23 +148,16 @@ __device__ __forceinline__ void st_once(double v, double* p, int nt) {
 // within 2^-24.2), in about half the instructions of the IEEE sequences, which
 // must also handle scaling and special operands.
 //
-// a/b: one Newton-Raphson step for the reciprocal, the quotient then corrected
-// once by its residual (Markstein's method); within an ulp of the correctly
-// rounded result.
+// a/b and sqrt(x): one Newton-Raphson step, the result then corrected once by
+// its residual (Markstein's method; for the root the residual times the
+// estimate itself is enough): 0.50 ulp.  1/b: the first two terms of the series
+// in the estimate's error e (2^-24, so e^3 is below rounding) in one step,
+// 1/(1-e) = 1 + e + e^2, also 0.50 ulp.
 __device__ __forceinline__ double quot_pos(double a, double b) {
   double r = __builtin_amdgcn_rcp(b);
   r = __fma_rn(__fma_rn(-b, r, 1.0), r, r);
   const double q = a * r;
   return __fma_rn(__fma_rn(-b, q, a), r, q);
-}
-// The following add the first two terms of the series in the estimate's error
-// e (2^-24, so e^3 is below rounding) in one step: 1/(1-e) = 1 + e + e^2 and
-// 1/sqrt(1-2e) = 1 + e + 3/2 e^2; within an ulp or so, one or two
-// instructions shorter than two refinements.
-__device__ __forceinline__ double quot_near(double a, double b) {
-  const double r = __builtin_amdgcn_rcp(b);
-  const double e = __fma_rn(-b, r, 1.0), q = a * r;
-  return __fma_rn(q, __fma_rn(e, e, e), q);
 }
 __device__ __forceinline__ double recip_pos(double b) {
   const double r = __builtin_amdgcn_rcp(b);
@@ -173,9 +166,9 @@ __device__ __forceinline__ double recip_pos(double b) {
 }
 __device__ __forceinline__ double sqrt_pos(double x) {
   const double r = __builtin_amdgcn_rsq(x);
-  const double y = x * r;
-  const double e = __fma_rn(-0.5 * r, y, 0.5);
-  return __fma_rn(y, __fma_rn(1.5 * e, e, e), y);
+  const double h = 0.5 * r, y = x * r;
+  const double z = __fma_rn(y, __fma_rn(-h, y, 0.5), y);
+  return __fma_rn(h, __fma_rn(-z, z, x), z);
 }
 // max(m, |x|) in one instruction (fmax first quiets its operands)
 __device__ __forceinline__ double max_abs(double m, double x) {
@@ -262,7 +255,7 @@ struct RoeF {
 template <int ND>
 __device__ __forceinline__ void roe_factors(const Pt<ND>& P, double& sq, double& h) {
   sq = sqrt_pos(P.q[0]);
-  h = (P.q[ND + 1] + P.p) * quot_near(sq, P.q[0]);
+  h = (P.q[ND + 1] + P.p) * quot_pos(sq, P.q[0]);
 }
 
 template <int ND>
@@ -645,7 +638,7 @@ __device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd
     const double c3 = 4.5 * C - 2.0 * Dd + 0.5 * E;
     const double tau = fabs(b3 - (b0 + b2 - 4.0 * b1) * (1.0 / 6.0));
     const double e3 = eps + b3;
-    const double x01 = quot_near(tau, e0 * e1), x23 = quot_near(tau, e2 * e3);
+    const double x01 = quot_pos(tau, e0 * e1), x23 = quot_pos(tau, e2 * e3);
     const double a0 = pow6(__fma_rn(e1, x01, 1.0)), a1 = pow6(__fma_rn(e0, x01, 1.0));
     const double a2 = pow6(__fma_rn(e3, x23, 1.0)), a3 = pow6(__fma_rn(e2, x23, 1.0));
     const double cut = ct * (a0 + a1 + a2 + a3);
@@ -655,9 +648,9 @@ __device__ __forceinline__ void teno_gap(double A, double B, double C, double Dd
     den = w0 + w1 + w2 + w3;
   } else {
     const double tau = fabs(b0 - b2);
-    const double x01 = quot_near(tau, e0 * e1);
+    const double x01 = quot_pos(tau, e0 * e1);
     const double a0 = pow6(__fma_rn(e1, x01, 1.0)), a1 = pow6(__fma_rn(e0, x01, 1.0));
-    const double a2 = pow6(1.0 + quot_near(tau, e2));
+    const double a2 = pow6(1.0 + quot_pos(tau, e2));
     const double cut = ct * (a0 + a1 + a2);
     const double w0 = a0 < cut ? 0.0 : 11.0 / 20.0, w1 = a1 < cut ? 0.0 : 4.0 / 10.0, w2 = a2 < cut ? 0.0 : 1.0 / 20.0;
     num = w0 * c0 + w1 * c1 + w2 * c2;
@@ -701,7 +694,7 @@ __device__ __forceinline__ double recon_gap(const double dcs[5], const double dc
       teno_gap<SIX, true>(p[0], p[1], p[2], p[3], p[4], eps, ct, n1, d1);
       teno_gap<SIX, false>(m[4], m[3], m[2], m[1], m[0], eps, ct, n2, d2);
     }
-    return __fma_rn(1.0 / 6.0, quot_near(n1, d1) - quot_near(n2, d2), -lam * dcs[2]);
+    return __fma_rn(1.0 / 6.0, quot_pos(n1, d1) - quot_pos(n2, d2), -lam * dcs[2]);
   }
 }
 

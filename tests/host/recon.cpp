@@ -19,3 +19,18 @@ extern "C" void teno(int six, int quirk, long n, const double* d, double eps, do
     else teno_gap<false, false>(x[0], x[1], x[2], x[3], x[4], eps, ct, num[i], den[i]);
   }
 }
+
+// the largest errors of a/b, 1/b and sqrt(b) over n operands, in units in the last place
+extern "C" void ulps(long n, const double* a, const double* b, double* worst) {
+  auto err = [](double got, long double want) {
+    int e;
+    std::frexp((double)want, &e);
+    return (double)(std::fabs((long double)got - want) / std::ldexp(1.0L, e - 53));
+  };
+  worst[0] = worst[1] = worst[2] = 0.0;
+  for (long i = 0; i < n; ++i) {
+    worst[0] = std::max(worst[0], err(quot_pos(a[i], b[i]), (long double)a[i] / b[i]));
+    worst[1] = std::max(worst[1], err(recip_pos(b[i]), 1.0L / b[i]));
+    worst[2] = std::max(worst[2], err(sqrt_pos(b[i]), std::sqrt((long double)b[i])));
+  }
+}

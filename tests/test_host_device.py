@@ -116,3 +116,14 @@ def test_teno_weights_over_the_range_of_the_quotients(recon, scale, eps, six, qu
     assert ok.mean() > 0.8
     err = np.abs(num / den - want)[ok] / scale
     assert np.all(err <= 1e-12), (err.max(), int((~(err <= 1e-12)).sum()))
+
+
+def test_quotients_and_roots_are_rounded_correctly_or_nearly(recon):
+    """a/b, 1/b and sqrt(b) from estimates as coarse as the hardware's: within
+    0.501 units in the last place (an IEEE result is within 0.5)."""
+    rs = np.random.RandomState(1)
+    n = 400000
+    a, b = (rs.uniform(1, 2, n) * 2.0 ** rs.randint(-40, 40, n) for _ in range(2))
+    worst = np.empty(3)
+    recon.ulps(ctypes.c_long(n), _dp(a), _dp(b), _dp(worst))
+    assert np.all(worst <= 0.501), worst
