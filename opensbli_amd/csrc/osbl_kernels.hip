@@ -756,7 +756,7 @@ void launch_visc_update3d(const double* Q, double* R, const Grid& g, const Phys&
 // (scheme.py:299-387) and the RK update, with the formulas of
 // central_convective and viscous_terms.
 //
-// A 64 x TY block of (x, y) columns marches along z.  When plane z+2 is in
+// A TX x TY block of (x, y) columns (64 or 32 by 8) marches along z.  When plane z+2 is in
 // LDS (conservative and primitive variables with a 2-point x/y halo), each
 // thread evaluates everything that needs only that plane for its column --
 // the x and y terms, added up in r -- and keeps in a register queue over
@@ -774,9 +774,10 @@ void launch_visc_update3d(const double* Q, double* R, const Grid& g, const Phys&
 // The stage moves Q, the register and the new state once: 160 B per cell
 // against 280 for a convective kernel that leaves R to a viscous kernel.  What
 // bounds it now is a block's chain per plane (LDS reads, two waves per SIMD,
-// a barrier) and, at 256^3, HBM: 0.75 ms a stage, 3.6 TB/s of those 160 B;
+// a barrier) and, at 256^3, HBM: 0.73 ms a stage, 3.7 TB/s of those 160 B;
 // the two kernels and the halo pass took 1.36 ms.  Reading a point's fields
-// two at a time (ds_read_b128) and adding up point by point took it from 0.88.
+// two at a time (ds_read_b128) took it from 0.88 to 0.75, adding up the pairs'
+// differences with Q and p in one sum (fewer operations and registers) to 0.73.
 //   MODE 0/1: RK update; MODE 2: the residual alone, into R.
 // ---------------------------------------------------------------------------
 template <int CONV, bool VISC, int MODE, int TX, int TY>
@@ -851,61 +852,63 @@ __global__ void __launch_bounds__(TX * TY, 2)
   };
   // fields 2 i and 2 i + 1 of the point o of a slot
   auto two = [](const double (*S)[NF], int o, int i) { return *reinterpret_cast<const Two*>(&S[o][2 * i]); };
-  // sums over the points -2, -1, 1, 2 of a direction: first differences of
-  // Q u_j, Q, p, p u_j, u_0..u_2 and second ones of u_0..u_2, T
+  // sums over the points -2, -1, 1, 2 of a direction: q is the convective term
+  // of the conservative variables over `hi` below -- skew: first difference of
+  // Q (u_j + u0) + 2 p e, conservative: of Q u_j + p e, with p e = (0, p e_j,
+  // p u_j); u, uu and TT first and second differences of u_0..u_2 and T.  The
+  // outer and the inner pair are each taken as a difference (a sum) before
+  // they are weighted: a field uniform along the direction gives exactly zero.
   struct Sums {
-    double qu[NV], q[NV], p, pu, u[3], uu[3], TT;
+    double q[NV], u[3], uu[3], TT;
   };
-  auto gather = [&](const double (*S)[NF], int j, int st) {
+  constexpr bool SKEW = CONV == OSBL_CONV_CENTRAL_SKEW;
+  auto gather = [&](const double (*S)[NF], int j, int st, double u0) {
     Sums a{};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int o = c + (s < 2 ? s - 2 : s - 1) * st;
-      const double w = s == 0 ? 1.0 / 12.0 : (s == 1 ? -2.0 / 3.0 : (s == 2 ? 2.0 / 3.0 : -1.0 / 12.0));
-      const double w2 = (s == 0 || s == 3) ? -1.0 / 12.0 : 4.0 / 3.0;
-      const Two f0 = two(S, o, 0), f1 = two(S, o, 1), f2 = two(S, o, 2), f3 = two(S, o, 3);
-      const double q[NV] = {f0.a, f0.b, f1.a, f1.b, f2.a}, p = f2.b;
-      const double uj = j == 0 ? f3.a : f3.b, wu = w * uj;
-      if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
-#pragma unroll
-        for (int m = 0; m < NV; ++m) {
-          a.qu[m] = __fma_rn(wu, q[m], a.qu[m]);
-          a.q[m] = __fma_rn(w, q[m], a.q[m]);
-        }
-      } else {
-        a.q[0] = __fma_rn(w, q[1 + j], a.q[0]);
-#pragma unroll
-        for (int m = 1; m < NV; ++m) a.qu[m] = __fma_rn(wu, q[m], a.qu[m]);
-      }
-      a.p = __fma_rn(w, p, a.p);
-      a.pu = __fma_rn(wu, p, a.pu);
+    for (int s = 0; s < 2; ++s) {
+      // D = 1/12 (f[-2] - f[2]) + 2/3 (f[1] - f[-1]): l minus r, weighted w
+      const int l = c + (s == 0 ? -2 : 1) * st, r = c + (s == 0 ? 2 : -1) * st;
+      const double w = s == 0 ? 1.0 / 12.0 : 2.0 / 3.0, w2 = s == 0 ? -1.0 / 12.0 : 4.0 / 3.0;
+      const Two l3 = two(S, l, 3), r3 = two(S, r, 3);
+      const double ul = j == 0 ? l3.a : l3.b, ur = j == 0 ? r3.a : r3.b;
       if constexpr (VISC) {
-        const Two f4 = two(S, o, 4);
-        a.u[0] = __fma_rn(w, f3.a, a.u[0]);
-        a.u[1] = __fma_rn(w, f3.b, a.u[1]);
-        a.u[2] = __fma_rn(w, f4.a, a.u[2]);
-        a.uu[0] = __fma_rn(w2, f3.a, a.uu[0]);
-        a.uu[1] = __fma_rn(w2, f3.b, a.uu[1]);
-        a.uu[2] = __fma_rn(w2, f4.a, a.uu[2]);
-        a.TT = __fma_rn(w2, f4.b, a.TT);
+        const Two l4 = two(S, l, 4), r4 = two(S, r, 4);
+        a.u[0] = __fma_rn(w, l3.a - r3.a, a.u[0]);
+        a.u[1] = __fma_rn(w, l3.b - r3.b, a.u[1]);
+        a.u[2] = __fma_rn(w, l4.a - r4.a, a.u[2]);
+        a.uu[0] = __fma_rn(w2, l3.a + r3.a, a.uu[0]);
+        a.uu[1] = __fma_rn(w2, l3.b + r3.b, a.uu[1]);
+        a.uu[2] = __fma_rn(w2, l4.a + r4.a, a.uu[2]);
+        a.TT = __fma_rn(w2, l4.b + r4.b, a.TT);
       } else {
-        a.u[j] = __fma_rn(w, uj, a.u[j]);
+        a.u[j] = __fma_rn(w, ul - ur, a.u[j]);
       }
+      __builtin_amdgcn_sched_barrier(0);  // (the pair's fields in two parts: registers)
+      const Two l0 = two(S, l, 0), l1 = two(S, l, 1), l2 = two(S, l, 2);
+      const Two r0 = two(S, r, 0), r1 = two(S, r, 1), r2 = two(S, r, 2);
+      const double ql[NV] = {l0.a, l0.b, l1.a, l1.b, l2.a}, qr[NV] = {r0.a, r0.b, r1.a, r1.b, r2.a};
+      if constexpr (SKEW) {
+        const double vl = ul + u0, vr = ur + u0;
+#pragma unroll
+        for (int m = 0; m < NV; ++m) a.q[m] = __fma_rn(w, __fma_rn(ql[m], vl, -(qr[m] * vr)), a.q[m]);
+        a.q[1 + j] = __fma_rn(2.0 * w, l2.b - r2.b, a.q[1 + j]);
+        a.q[4] = __fma_rn(2.0 * w, __fma_rn(l2.b, ul, -(r2.b * ur)), a.q[4]);
+      } else {
+        a.q[0] = __fma_rn(w, ql[1 + j] - qr[1 + j], a.q[0]);
+#pragma unroll
+        for (int m = 1; m < 4; ++m) a.q[m] = __fma_rn(w, __fma_rn(ql[m], ul, -(qr[m] * ur)), a.q[m]);
+        a.q[1 + j] = __fma_rn(w, l2.b - r2.b, a.q[1 + j]);
+        a.q[4] = __fma_rn(w, __fma_rn(ql[4] + l2.b, ul, -((qr[4] + r2.b) * ur)), a.q[4]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     return a;
   };
-  auto add_convect = [](const Sums& a, int j, double inv, const double (&q0)[NV], double u0, double* r) {
-    if constexpr (CONV == OSBL_CONV_CENTRAL_SKEW) {
-      const double hi = -0.5 * inv, hu = hi * u0, du = hi * a.u[j];
+  auto add_convect = [](const Sums& a, int j, double inv, const double (&q0)[NV], double* r) {
+    const double hi = SKEW ? -0.5 * inv : -inv;
+    const double du = hi * a.u[j];
 #pragma unroll
-      for (int m = 0; m < NV; ++m) r[m] += hi * a.qu[m] + hu * a.q[m] + q0[m] * du;
-    } else {
-      r[0] -= inv * a.q[0];
-#pragma unroll
-      for (int m = 1; m < NV; ++m) r[m] -= inv * a.qu[m];
-    }
-    r[1 + j] -= inv * a.p;
-    r[4] -= inv * a.pu;
+    for (int m = 0; m < NV; ++m) r[m] += SKEW ? hi * a.q[m] + q0[m] * du : hi * a.q[m];
   };
   // convective terms along z: values of Q_m, u_j, p at the
   // offsets -2, -1, 1, 2 through fq, fu, fp; the cell's own Q and u_j
@@ -983,8 +986,8 @@ __global__ void __launch_bounds__(TX * TY, 2)
 #pragma unroll
         for (int m = 0; m < NV; ++m) r[m] = 0.0;
         const double q0[NV] = {e[0], e[1], e[2], e[3], e[4]};
-        const Sums ax = gather(S, 0, 1);
-        add_convect(ax, 0, ix, q0, f3.a, r);
+        const Sums ax = gather(S, 0, 1, f3.a);
+        add_convect(ax, 0, ix, q0, r);
         if constexpr (VISC) {
           const double xx = ix * ix, yy = iy * iy;
           const Two f4 = two(S, c, 4);
@@ -995,8 +998,8 @@ __global__ void __launch_bounds__(TX * TY, 2)
           e[7] = ix * ax.u[2];
           asm volatile("" : "+v"(p0), "+v"(p1), "+v"(p2), "+v"(TT), "+v"(ux), "+v"(sh), "+v"(e[7]));
           settle(r);
-          const Sums ay = gather(S, 1, PX);
-          add_convect(ay, 1, iy, q0, f3.b, r);
+          const Sums ay = gather(S, 1, PX, f3.b);
+          add_convect(ay, 1, iy, q0, r);
           p0 += yy * (ay.uu[0] - 2.5 * f3.a);
           p1 += (4.0 / 3.0) * yy * (ay.uu[1] - 2.5 * f3.b);
           p2 += yy * (ay.uu[2] - 2.5 * f4.a);
@@ -1028,7 +1031,7 @@ __global__ void __launch_bounds__(TX * TY, 2)
           settle(r);
         } else {
           settle(r);
-          add_convect(gather(S, 1, PX), 1, iy, q0, f3.b, r);
+          add_convect(gather(S, 1, PX, f3.b), 1, iy, q0, r);
           settle(r);
         }
       } else if constexpr (VISC) {
@@ -1046,17 +1049,22 @@ __global__ void __launch_bounds__(TX * TY, 2)
         for (int m = 0; m < NV; ++m) r[m] = rr[0][m];
         const double* k0 = zq[2];
         const double q0[NV] = {k0[0], k0[1], k0[2], k0[3], k0[4]};
-        // velocities and pressure of the column
+        // velocities and pressure of the column, each rounded (no product is
+        // contracted into a difference): equal values have zero derivatives
+        auto rounded = [](double v) {
+          asm("" : "+v"(v));
+          return v;
+        };
         double u[5][3], p[5];
 #pragma unroll
         for (int s = 0; s < 5; ++s) {
           double ke = 0.0;
 #pragma unroll
           for (int m = 0; m < 3; ++m) {
-            u[s][m] = zq[s][1 + m] * zq[s][5];
+            u[s][m] = rounded(zq[s][1 + m] * zq[s][5]);
             ke += u[s][m] * zq[s][1 + m];
           }
-          p[s] = ph.gm1 * (zq[s][4] - 0.5 * ke);
+          p[s] = rounded(ph.gm1 * (zq[s][4] - 0.5 * ke));
         }
         auto pl = [](int s) { return s < 2 ? s : s + 1; };
         convect(
@@ -1066,7 +1074,7 @@ __global__ void __launch_bounds__(TX * TY, 2)
         if constexpr (VISC) {
           double T[5], du[3], ddu[3];
 #pragma unroll
-          for (int s = 0; s < 5; ++s) T[s] = cT * p[s] * zq[s][5];
+          for (int s = 0; s < 5; ++s) T[s] = rounded(cT * p[s] * zq[s][5]);
           const double zz = iz * iz;
 #pragma unroll
           for (int m = 0; m < 3; ++m) {

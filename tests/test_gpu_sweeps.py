@@ -123,3 +123,23 @@ def test_2d_rough_state_in_other_units(s, eps, conv, averaging, oracle):
     u = [s * rs.uniform(-0.3, 0.3, n[::-1]) for _ in range(2)]
     q0 = np.stack([rho] + [rho * v for v in u] + [s * s * p / 0.4 + 0.5 * rho * (u[0] ** 2 + u[1] ** 2)])
     _check(problem, q0, oracle, f"2-D in units of {s:g}, eps={eps:g} {conv} {averaging}")
+
+
+@pytest.mark.parametrize("conv", ["central_skew", "central_cons"])
+@pytest.mark.parametrize("viscous", ["const", "none"])
+def test_3d_central_residual_of_a_uniform_state_is_zero(viscous, conv):
+    """Every first derivative is a sum of differences between points, so it
+    vanishes exactly on a uniform state whose products are exact (u a power of
+    two, whose second derivatives vanish as well).  T's second derivative is
+    rounded: Pr = 1e300 leaves nothing of it."""
+    from opensbli_amd.native import Block
+    n = (70, 9, 11)
+    problem, q0 = _block(n, conv, "periodic", viscous=viscous)
+    u = [0.5, -0.25, 0.125]
+    for k, v in enumerate([1.0] + u + [1.0 / 3.0 + 2.0]):
+        q0[k] = v
+    problem["Pr"] = 1e300
+    print("case uniform 3-D state", conv, viscous, flush=True)
+    g = Block(problem)
+    g.set_state(q0)
+    assert np.abs(g.rhs()).max() < 1e-280
