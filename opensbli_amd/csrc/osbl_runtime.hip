@@ -333,15 +333,14 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
   double* Q = Qcur(c);
   double* Qn = c->Qbuf[1 - c->cur];
   const int conv = c->cfg.conv;
+  // the adaptive TENO's sensor (Theta may be the WENO filter's, formed in filters())
+  double* theta = c->cfg.sensor ? c->Theta : nullptr;
   const bool tile = c->tiled2d || (c->tiled_central && c->nd == 2);  // these write pk themselves
   if (pk && !tile) launch_pack_all(Q, pk, c->g, c->nv, c->stream);
   if (c->tiled2d) {
-    // (the kernel forms the adaptive TENO's sensor; the WENO filter's on another scheme here)
-    if (c->Theta && conv != OSBL_CONV_TENO5 && conv != OSBL_CONV_TENO6)
-      timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
     timed(c, F_SWEEP_X, [&] {
       launch_char_tile2d(conv, c->cfg.averaging, mode, c->cfg.viscous != OSBL_VISC_NONE, Q, c->R, c->Qo, Qn, c->g,
-                         c->ph, c->bnd, cA, cB, first, c->Theta, c->suth ? 1 : 0, c->haloless ? 1 : 0, pk, c->stream);
+                         c->ph, c->bnd, cA, cB, first, theta, c->suth ? 1 : 0, c->haloless ? 1 : 0, pk, c->stream);
     });
     return;
   }
@@ -360,7 +359,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
       });
     }
   }
-  if (c->Theta) timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, c->Theta, c->g, c->ph, c->bnd, c->stream); });
+  if (theta) timed(c, F_PRIMS, [&] { launch_sensor(c->nd, Q, theta, c->g, c->ph, c->bnd, c->stream); });
   if (c->curv) {
     // strong conservation form: a kernel per direction, the last one with the update
     for (int d = 0; d < c->nd; ++d) {
@@ -388,16 +387,16 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
     // viscous kernel and the y sweep accumulate, and the z sweep adds the last
     // difference and applies the RK update, so the update needs no pass of its own
     timed(c, F_SWEEP_X, [&] {
-      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, c->Theta, false,
+      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, false,
                    c->stream);
     });
     timed(c, F_UPDATE, [&] { launch_visc_update3d(Q, c->R, c->g, c->ph, c->vsz, c->stream); });
     timed(c, F_SWEEP_Y, [&] {
-      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, c->Theta, true,
+      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, true,
                    c->stream);
     });
     timed(c, F_SWEEP_Z, [&] {
-      launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, c->Theta, cA, cB,
+      launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, theta, cA, cB,
                         first, c->stream);
     });
     return;
@@ -406,7 +405,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
     // the same schedule on the general path: tiled viscous terms with closures,
     // metric and mu(T) (z free of both), sweeps with the metric, RK in the z sweep
     timed(c, F_SWEEP_X, [&] {
-      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[0], c->Theta, false,
+      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[0], theta, false,
                    c->stream);
     });
     timed(c, F_UPDATE, [&] {
@@ -414,11 +413,11 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
       if (c->ph.has_force) launch_body_force3d(Q, c->R, c->g, c->ph, c->stream);
     });
     timed(c, F_SWEEP_Y, [&] {
-      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[1], c->Theta, true,
+      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[1], theta, true,
                    c->stream);
     });
     timed(c, F_SWEEP_Z, [&] {
-      launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, c->Theta, cA, cB,
+      launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, theta, cA, cB,
                         first, c->stream);
     });
     return;
@@ -426,7 +425,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
   if (!is_central(conv)) {
     for (int d = 0; d < c->nd; ++d) {
       timed(c, F_SWEEP_X + d, [&] {
-        launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], c->Theta, d > 0,
+        launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], theta, d > 0,
                      c->stream);
       });
     }
@@ -1174,6 +1173,8 @@ int osbl_rhs(osbl_ctx* c, double* residual_host) {
   if (!c || !residual_host) return fail(OSBL_E_ARG, "null argument");
   if (int rc = check_ready(c)) return rc;
   loop_bcs(c);
+  // (the WENO filter's sensor of this state, for osbl_get_sensor)
+  if (c->Theta && !c->cfg.sensor) launch_sensor(c->nd, Qcur(c), c->Theta, c->g, c->ph, c->bnd, c->stream);
   stage(c, 2, 0.0, 0.0, 0);
   HIPCHK(hipGetLastError());
   const long long n = cells(c);

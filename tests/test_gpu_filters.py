@@ -129,6 +129,20 @@ def test_weno_filter_on_a_channel_with_body_force(conv, sensor, oracle):
     assert d.max() > 1e-7, d.max()
 
 
+@pytest.mark.parametrize("n", [(48, 40), (24, 20, 16)])
+def test_weno_filter_with_teno_and_its_fixed_cutoff(n, oracle):
+    """The filter's Ducros sensor is not the scheme's: TENO without `sensor`
+    keeps teno_ct."""
+    _say(f"case weno filter (ducros) on TENO5 with a fixed cut-off {n}")
+    p = _problem(n, "teno5", {"weno": {"sensor": "ducros"}}, teno_ct=1e-3)
+    q0 = _state(n, seed=8)
+    a, b = _compare(p, q0, oracle, steps=10)
+    r = oracle.RefSolver(dict(p, sensor=True))
+    r.set_state(q0)
+    r.run(10)
+    assert np.abs(r.get_state() - b).max() > 1e-6
+
+
 @pytest.mark.parametrize("restart", [False, True])
 def test_sfd(restart, oracle):
     n = (48, 32)
