@@ -347,7 +347,8 @@ int osbl_batch_get_state(osbl_batch* b, int inst, double* host);
    mode 1 = one launch per RK stage over all running instances, replayed from
    hipGraphs; returns the device time in *elapsed_ms */
 int osbl_batch_run(osbl_batch* b, int mode, double* elapsed_ms);
-/* persistent mode: threads per workgroup (64..512, multiple of 64) for instances with n <= max_n[k] */
+/* persistent mode: threads per workgroup (64..1024, multiple of 64) for instances with n <= max_n[k];
+   without a table, 64 per 63 points, at most 1024 */
 int osbl_batch_set_threads(osbl_batch* b, int nbuckets, const int32_t* max_n, const int32_t* threads);
 /* staged mode: iterations captured per hipGraph */
 int osbl_batch_set_graph_steps(osbl_batch* b, int steps);

@@ -648,7 +648,8 @@ int osbl_batch_run(osbl_batch* b, int mode, double* elapsed_ms) {
 int osbl_batch_set_threads(osbl_batch* b, int nbuckets, const int32_t* max_n, const int32_t* threads) {
   if (!b || nbuckets <= 0 || !max_n || !threads) return bfail(OSBL_E_ARG, "invalid argument");
   for (int k = 0; k < nbuckets; ++k)
-    if (threads[k] < 64 || threads[k] > 512 || threads[k] % 64) return bfail(OSBL_E_ARG, "threads must be 64..512, multiple of 64");
+    if (threads[k] < 64 || threads[k] > 1024 || threads[k] % 64)
+      return bfail(OSBL_E_ARG, "threads must be 64..1024, multiple of 64");
   b->bucket_n.assign(max_n, max_n + nbuckets);
   b->bucket_t.assign(threads, threads + nbuckets);
   b->bucket_n.back() = 1 << 30;

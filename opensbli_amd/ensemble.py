@@ -116,7 +116,7 @@ class Ensemble:
 
 
 BUCKETS = [256, 512, 1024, 2048, 4096]
-CANDIDATES = [64, 128, 256, 512]
+CANDIDATES = [64, 128, 256, 512, 1024]
 
 
 def autotune(par, conv="weno_z", rk="rk3", probe_steps=40, buckets=BUCKETS, candidates=CANDIDATES, cache=None):

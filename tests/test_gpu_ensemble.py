@@ -72,6 +72,30 @@ def test_ensemble_thread_tables_agree():
             assert np.array_equal(a, b)
 
 
+def test_ensemble_thread_tables_up_to_the_default():
+    """Lines on both sides of 63 points per wave for 512 and for 1024 threads
+    (what a line takes without a table): on the chip and through memory, the
+    same bits."""
+    from opensbli_amd.ensemble import CANDIDATES, Ensemble
+    _say("case ensemble thread tables up to 1024")
+    par = _small(ninst=6, seed=17, steps=7)
+    par["n"] = np.array([62, 504, 505, 1008, 1009, 1700], dtype=np.int32)
+    par["dx"] = 1.0 / (par["n"] - 1)
+    par["dt"] = 0.2 * par["dx"]
+    outs = []
+    for t in [None, 64, 512, 1024]:
+        e = Ensemble(par)
+        if t:
+            e.set_threads([1 << 30], [t])
+        e.run("persistent")
+        outs.append([e.get_state(i) for i in range(6)])
+        e.close()
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            assert np.array_equal(a, b)
+    assert CANDIDATES[-1] == 1024
+
+
 def test_ensemble_states_read_from_several_threads():
     """Lines read back by eight host threads at once: each gets its own."""
     from concurrent.futures import ThreadPoolExecutor
