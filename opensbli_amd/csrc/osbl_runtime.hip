@@ -1347,41 +1347,42 @@ static int adjoint_check(const osbl_ctx* c, bool need_rk3) {
   return OSBL_OK;
 }
 
-// which buffers the context's scheme uses
-static bool adj_needs_halo_bufs(const osbl_ctx* c) {
+// whether a call reads padded copies of the state and the weights and the
+// constituent relations: osbl_rhs_vjp_dev (`vjp`) of a central scheme, viscous
+// terms; a 2-D block's reverse stages work on the packed arrays
+static bool adj_needs_halo_bufs(const osbl_ctx* c, bool vjp) {
+  if (c->nd == 2) return vjp && c->cfg.conv == OSBL_CONV_CENTRAL_SKEW;
   return c->cfg.conv == OSBL_CONV_CENTRAL_SKEW || c->cfg.viscous == OSBL_VISC_CONST;
 }
-static bool adj_needs_prims(const osbl_ctx* c) { return adj_needs_halo_bufs(c); }
+static bool adj_needs_visc_fields(const osbl_ctx* c) { return c->cfg.viscous == OSBL_VISC_CONST && c->nd != 2; }
 
 // allocating set-up: the context's own buffers, made on first use
 static int adjoint_ready(osbl_ctx* c, bool need_rk3, AdjBufs* b) {
   int rc = adjoint_check(c, need_rk3);
   if (rc) return rc;
-  if (!c->Abuf) {
-    const size_t bundle = (size_t)c->g.fs * c->nv * sizeof(double);
-    const size_t packed = (size_t)cells(c) * c->nv * sizeof(double);
-    if (hipMalloc((void**)&c->Abuf, bundle) != hipSuccess || hipMalloc((void**)&c->Mbuf, bundle) != hipSuccess ||
-        hipMalloc((void**)&c->pk, 3 * packed) != hipSuccess)
-      return fail(OSBL_E_NOMEM, "adjoint buffers");
-    HIPCHK(hipMemsetAsync(c->Abuf, 0, bundle, c->stream));
-    HIPCHK(hipMemsetAsync(c->Mbuf, 0, bundle, c->stream));
+  auto need = [&](double** p, size_t doubles, bool zero, const char* what) -> int {
+    if (*p) return OSBL_OK;
+    if (hipMalloc((void**)p, doubles * sizeof(double)) != hipSuccess) {
+      *p = nullptr;
+      return fail(OSBL_E_NOMEM, "%s", what);
+    }
+    if (zero) HIPCHK(hipMemsetAsync(*p, 0, doubles * sizeof(double), c->stream));
+    return OSBL_OK;
+  };
+  const size_t bundle = (size_t)c->g.fs * c->nv, packed = (size_t)cells(c) * c->nv;
+  if ((rc = need(&c->pk, 3 * packed, false, "adjoint buffers"))) return rc;
+  if (adj_needs_halo_bufs(c, !need_rk3)) {
+    // (blocks of one tiled kernel per stage keep no constituent-relation array)
+    if ((rc = need(&c->Abuf, bundle, true, "adjoint buffers")) ||
+        (rc = need(&c->Mbuf, bundle, true, "adjoint buffers")) ||
+        (rc = need(&c->P, (size_t)c->g.fs * (c->nd + 3), true, "adjoint constituent relations")))
+      return rc;
   }
-  if (c->cfg.viscous == OSBL_VISC_CONST && c->nd != 2 && !c->vw) {
-    const size_t bytes = (size_t)c->g.fs * visc_vjp_fields(c->nd) * sizeof(double);
-    if (hipMalloc((void**)&c->vw, bytes) != hipSuccess) return fail(OSBL_E_NOMEM, "adjoint viscous scratch");
-    HIPCHK(hipMemsetAsync(c->vw, 0, bytes, c->stream));
-  }
-  if (adj_needs_prims(c) && !c->P) {
-    // 3-D characteristic blocks evaluate their viscous terms without a
-    // constituent-relation array; the viscous VJP needs one
-    const size_t bytes = (size_t)c->g.fs * (c->nd + 3) * sizeof(double);
-    if (hipMalloc((void**)&c->P, bytes) != hipSuccess) return fail(OSBL_E_NOMEM, "adjoint constituent relations");
-    HIPCHK(hipMemsetAsync(c->P, 0, bytes, c->stream));
-  }
-  if (c->cfg.conv == OSBL_CONV_WENO_Z && c->nd == 2 && !c->vy) {
-    if (hipMalloc((void**)&c->vy, (size_t)cells(c) * c->nv * sizeof(double)) != hipSuccess)
-      return fail(OSBL_E_NOMEM, "adjoint VJP staging");
-  }
+  if (adj_needs_visc_fields(c) &&
+      (rc = need(&c->vw, (size_t)c->g.fs * visc_vjp_fields(c->nd), true, "adjoint viscous scratch")))
+    return rc;
+  if (c->cfg.conv == OSBL_CONV_WENO_Z && c->nd == 2 && (rc = need(&c->vy, packed, false, "adjoint VJP staging")))
+    return rc;
   *b = AdjBufs{c->Abuf, c->Mbuf, c->pk, c->vw, c->P, c->vy};
   return OSBL_OK;
 }
@@ -1485,12 +1486,11 @@ static int scratch_bufs(osbl_ctx* c, AdjBufs* b) {
     return at;
   };
   const long long o_pk = take(3 * packed);
-  const bool halo = adj_needs_halo_bufs(c);
+  const bool halo = adj_needs_halo_bufs(c, false), visc = adj_needs_visc_fields(c);
   const long long o_A = halo ? take(fs * c->nv) : -1;
   const long long o_M = halo ? take(fs * c->nv) : -1;
-  const bool visc = c->cfg.viscous == OSBL_VISC_CONST;
   const long long o_vw = visc ? take(fs * visc_vjp_fields(c->nd)) : -1;
-  const long long o_P = adj_needs_prims(c) ? take(fs * (c->nd + 3)) : -1;
+  const long long o_P = halo ? take(fs * (c->nd + 3)) : -1;
   const size_t need = (size_t)off * sizeof(double);
   if (need > kScratchBytes)
     return fail(OSBL_E_ARG, "osbl_adjoint_step_dev_noalloc: this block needs %zu bytes of scratch, more than the "
@@ -1498,9 +1498,9 @@ static int scratch_bufs(osbl_ctx* c, AdjBufs* b) {
   auto at = [&](long long o) { return o < 0 ? nullptr : base + o; };
   *b = AdjBufs{at(o_A), at(o_M), at(o_pk), at(o_vw), at(o_P), nullptr};
   // zero everything from the first halo buffer on (A, M, the viscous
-  // fields, P): the allocating path's buffers start zeroed (2-D: not read)
-  if ((halo || visc) && c->nd != 2) {
-    const long long from = halo ? o_A : o_vw;
+  // fields, P): the allocating path's buffers start zeroed
+  if (halo) {
+    const long long from = o_A;
     const long long n = off - from;
     const unsigned blocks = (unsigned)std::min<long long>((n + 255) / 256, 8192);
     k_zero<<<blocks, 256, 0, c->stream>>>(base + from, n);

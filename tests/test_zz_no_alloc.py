@@ -83,6 +83,15 @@ def test_noalloc_adjoint_step_3d_viscous(conv):
     _check(f"TGV 16^3 {conv} viscous", *_both(p, q, 4))
 
 
+@pytest.mark.parametrize("conv", ["weno_z", "central_skew"])
+def test_noalloc_adjoint_step_2d_viscous_near_the_scratch_size(conv):
+    """A 2-D step works on packed arrays: 12 doubles a cell of scratch, 92 of
+    the 128 MiB for 1000^2."""
+    _say(f"case noalloc adjoint step: KH 1000^2 {conv} viscous")
+    p, q = _kh(1000, conv, viscous=True)
+    _check(f"KH 1000^2 {conv} viscous", *_both(p, q, 5))
+
+
 def test_noalloc_adjoint_step_refuses_oversized_block():
     import torch
     from opensbli_amd.native import Block, OsblError
