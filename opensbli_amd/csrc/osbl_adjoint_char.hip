@@ -669,18 +669,23 @@ __device__ __forceinline__ void vjp_line(long long line, int n0, int n1, long lo
 // I = a .. a+63 of one line.  The chunk's 69 points (a-2 .. a+66, periodic
 // images) are staged in LDS with their constituent relations, lane l
 // evaluates the VJP of interface a+l from LDS, and the contributions of the
-// six interfaces j-3 .. j+2 that reach cell j = a+l are gathered by
-// cross-lane shuffles; lanes 3..61 hold complete cells, so consecutive
+// six interfaces j-3 .. j+2 that reach cell j = a+l are gathered from
+// the lanes' LDS columns; lanes 3..61 hold complete cells, so consecutive
 // chunks of a line start 59 cells apart (five interfaces are evaluated
 // twice) and no partial sums leave the wave.
 //   ACC = false: out1 = c (A + B) + V (and out2 = A + B when given);
 //   ACC = true:  out1 += V.
-// What bounds it is FP64 issue at two waves per SIMD: ~2900 VALU instructions
-// per 64 interfaces, 256 registers with ~30 values spilled across the fields
-// (330 and one wave per SIMD without the bound).  512^2, ten steps' gradient:
-// 11.0 ms with reconstructions and their gradients from values and 84 LDS
-// additions per interface, 10.4 from differences at two waves, 10.3 with L
-// applied once, 9.9 with the largest wave speed's sign taken once.
+// What bounds it is FP64 issue at EU waves per SIMD: ~2900 VALU instructions
+// per 64 interfaces.  The work of an interface wants 330 registers; with two
+// waves per SIMD (256) 2-D spills ~30 values, 3-D ~50, across the fields.  Two
+// waves pay in 2-D from more than 1024 waves on, a round of the 1024 SIMDs
+// (vjp_eu; one step's reverse, one and two waves: 128^2 50 and 70 us, 200^2
+// 88 and 86, 256^2 128 and 131, 400^2 243 and 228, 512^2 358 and 347); 1-D and
+// 3-D always take one (32^3 156 and 238 us, 64^3 1200 and 1514, 96^3 2696 and
+// 3281).  512^2, ten steps' gradient: 11.0 ms with reconstructions and their
+// gradients from values and 84 LDS additions per interface, 10.4 from
+// differences at two waves, 10.3 with L applied once, 9.9 with the largest wave
+// speed's sign taken once.
 constexpr int VJW = 2;         // waves per block
 constexpr int VJP = 64 + 5;    // points staged per chunk
 constexpr int VJSTEP = 59;     // cells completed per chunk
@@ -772,13 +777,19 @@ __device__ __forceinline__ void vjp_chunk(long long wid, int lane, double (*S)[V
   }
 }
 
-template <int ND, int D, int AVG, bool ACC>
-__global__ void __launch_bounds__(64 * VJW, 2) k_char_vjp_lanes(const double* __restrict__ Qs,
-                                                             const double* __restrict__ A,
-                                                             const double* __restrict__ B, double alpha, double beta,
-                                                             double c, double* __restrict__ out1,
-                                                             double* __restrict__ out2, int n0, int n1, int n2,
-                                                             Phys ph) {
+// waves per SIMD to compile a VJP of `waves` waves for
+template <int ND>
+static int vjp_eu(long long waves) {
+  return ND == 2 && waves > 1024 ? 2 : 1;
+}
+
+template <int ND, int D, int AVG, bool ACC, int EU>
+__global__ void __launch_bounds__(64 * VJW, EU) k_char_vjp_lanes(const double* __restrict__ Qs,
+                                                              const double* __restrict__ A,
+                                                              const double* __restrict__ B, double alpha, double beta,
+                                                              double c, double* __restrict__ out1,
+                                                              double* __restrict__ out2, int n0, int n1, int n2,
+                                                              Phys ph) {
   constexpr int NV = ND + 2;
   constexpr int NF = NV + ND + 2;  // q, u, p, a
   __shared__ double sh[VJW][NF][VJP];
@@ -801,17 +812,18 @@ __global__ void __launch_bounds__(64 * VJW, 2) k_char_vjp_lanes(const double* __
 }
 
 // Both directions of a 2-D VJP in one launch, so that the y waves fill the
-// SIMDs the x waves leave idle in their last round (two waves per SIMD):
+// SIMDs the x waves leave idle in their last round:
 // x waves as k_char_vjp_lanes<2, 0, AVG, false> (out1, out2), y waves write
 // their V to vy, which k_add_packed then adds to out1.  With both block
 // counts multiples of 8, each XCD takes an eighth of the x blocks and then an
 // eighth of the y blocks, in order; otherwise blocks run in launch order.
-template <int AVG>
-__global__ void __launch_bounds__(64 * VJW, 2) k_char_vjp_xy(const double* __restrict__ Qs, const double* __restrict__ A,
-                                                          const double* __restrict__ B, double alpha, double beta,
-                                                          double c, double* __restrict__ out1,
-                                                          double* __restrict__ out2, double* __restrict__ vy, int n0,
-                                                          int n1, int bx, int by, Phys ph) {
+template <int AVG, int EU>
+__global__ void __launch_bounds__(64 * VJW, EU) k_char_vjp_xy(const double* __restrict__ Qs,
+                                                           const double* __restrict__ A, const double* __restrict__ B,
+                                                           double alpha, double beta, double c,
+                                                           double* __restrict__ out1, double* __restrict__ out2,
+                                                           double* __restrict__ vy, int n0, int n1, int bx, int by,
+                                                           Phys ph) {
   constexpr int NV = 4, NF = 8;
   __shared__ double sh[VJW][NF][VJP];
   __shared__ double ga[VJW][6 * NV][64];
@@ -850,12 +862,21 @@ static void launch_cv_d(const double* Qs, const double* A, const double* B, doub
     if (e != D) lines *= g.n[e];
   const long long waves = lines * ((g.n[D] + VJSTEP - 1) / VJSTEP);
   const unsigned blocks = (unsigned)((waves + VJW - 1) / VJW);
-  if (acc)
-    k_char_vjp_lanes<ND, D, AVG, true><<<blocks, 64 * VJW, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0],
-                                                                     g.n[1], g.n[2], ph);
-  else
-    k_char_vjp_lanes<ND, D, AVG, false><<<blocks, 64 * VJW, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0],
-                                                                      g.n[1], g.n[2], ph);
+  auto go = [&](auto ac, auto eu) {
+    k_char_vjp_lanes<ND, D, AVG, decltype(ac)::value, decltype(eu)::value>
+        <<<blocks, 64 * VJW, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, g.n[0], g.n[1], g.n[2], ph);
+  };
+  auto with_eu = [&](auto ac) {
+    if constexpr (ND == 2) {
+      if (vjp_eu<ND>(waves) == 2) {
+        go(ac, std::integral_constant<int, 2>{});
+        return;
+      }
+    }
+    go(ac, std::integral_constant<int, 1>{});
+  };
+  if (acc) with_eu(std::true_type{});
+  else with_eu(std::false_type{});
 }
 
 template <int ND, int AVG>
@@ -867,8 +888,12 @@ static void launch_cv_nd(const double* Qs, const double* A, const double* B, dou
       const long long wx = (long long)g.n[1] * ((g.n[0] + VJSTEP - 1) / VJSTEP);
       const long long wy = (long long)g.n[0] * ((g.n[1] + VJSTEP - 1) / VJSTEP);
       const int bx = (int)((wx + VJW - 1) / VJW), by = (int)((wy + VJW - 1) / VJW);
-      k_char_vjp_xy<AVG><<<bx + by, 64 * VJW, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, vy, g.n[0], g.n[1], bx,
-                                                       by, ph);
+      auto go = [&](auto eu) {
+        k_char_vjp_xy<AVG, decltype(eu)::value><<<bx + by, 64 * VJW, 0, s>>>(Qs, A, B, alpha, beta, c, out1, out2, vy,
+                                                                            g.n[0], g.n[1], bx, by, ph);
+      };
+      if (vjp_eu<2>(wx + wy) == 2) go(std::integral_constant<int, 2>{});
+      else go(std::integral_constant<int, 1>{});
       const long long n = (long long)g.n[0] * g.n[1] * 4;
       k_add_packed<<<(unsigned)std::min<long long>((n + 255) / 256, 4096), 256, 0, s>>>(out1, vy, n);
       return;

@@ -92,6 +92,16 @@ def test_noalloc_adjoint_step_2d_viscous_near_the_scratch_size(conv):
     _check(f"KH 1000^2 {conv} viscous", *_both(p, q, 5))
 
 
+@pytest.mark.parametrize("n", [59, 128, 176, 350])
+def test_noalloc_adjoint_step_waves(n):
+    """WENO5-Z blocks around the number of waves from which the VJPs are
+    compiled for two waves per SIMD (1024): 176^2 has 1056 in the paired launch
+    and 528 in each of the two, 350^2 more in all."""
+    _say(f"case noalloc adjoint step: KH {n}^2 weno_z")
+    p, q = _kh(n, "weno_z")
+    _check(f"KH {n}^2 weno_z", *_both(p, q, 6))
+
+
 def test_noalloc_adjoint_step_refuses_oversized_block():
     import torch
     from opensbli_amd.native import Block, OsblError
