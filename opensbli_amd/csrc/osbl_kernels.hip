@@ -1145,13 +1145,14 @@ int visc3d_segment(const Grid& g) { return tile_segment(g, VTX, VTY, 512, 64); }
 // viscous): 64 x 8 tiles, one block per CU (131 KB of LDS), 4.0 per plane + 10
 // per segment; 32 x 8 tiles, two per CU, 4.2 and 9, or 3.05 and 8 while there
 // are no more blocks than CUs.  The cheapest of all is taken: 256^3 64 x 8 x
-// 128 (0.75 ms; 0.78 with 32 planes), 128^3 about 91 us (101 with 64 x 8 x 8),
-// 24x30x40 32 x 8 x 2 (14 us; 18 with 64-wide tiles).
+// 128 (0.73 ms; 4 % more with 32 planes), 128^3 about 91 us (101 with 64 x 8 x 8),
+// 24x30x40 and smaller blocks 32 x 8 x 1 (8^3 to 32^3 11 us; 13.5 with two
+// planes, 18 with 64-wide tiles).
 void central3d_tiles(const Grid& g, int* tx, int* sz) {
   double best = 1.0e300;
   for (int w = 64; w >= 32; w -= 32) {
     const long long tiles = (long long)((g.n[0] + w - 1) / w) * ((g.n[1] + 7) / 8);
-    for (int p = 2; p <= 256; ++p) {
+    for (int p = 1; p <= 256; ++p) {
       const long long blocks = tiles * ((g.n[2] + p - 1) / p);
       double t;
       if (w == 64) t = (double)((blocks + 255) / 256) * (4.0 * p + 10.0);
