@@ -7,8 +7,9 @@ namespace osbl {
 
 void launch_halo_periodic(double* Q, int nv, const Grid& g, hipStream_t s);
 void launch_prims(int nd, const double* Q, double* P, const Grid& g, const Phys& ph, hipStream_t s);
+// the characteristic sweep of direction d (1-D, 3-D): d = 0 assigns R, the others add to it
 void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
-                  const double* met, const double* theta, bool acc, hipStream_t s);
+                  const double* met, const double* theta, hipStream_t s);
 // one stage of a 2-D characteristic block (osbl_tile2d.hip); theta: the
 // adaptive TENO's sensor is formed and left there; wrap: periodic in both
 // directions, halos not read.  conv CONV_WFILTER, mode 2: the WENO filter's

@@ -235,7 +235,7 @@ static int sweep_xl_cells(const Grid& g) {
 }
 
 // (at least three waves per SIMD)
-template <int ND, int CONV, int AVG, bool ACC>
+template <int ND, int CONV, int AVG>
 __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __restrict__ Q, double* __restrict__ R,
                                                           Grid g, Phys ph, int nwaves, int cells, int periodic,
                                                           const double* __restrict__ met,
@@ -280,9 +280,7 @@ __global__ void __launch_bounds__(64 * XW, 3) k_char_sweep_xl(const double* __re
     const double gi = met ? -met[x] * inv : -inv;
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
-      const double v = r[m] * gi;
-      if constexpr (ACC) st_once(ld_once(&R[m * g.fs + line + x], ph.nt) + v, &R[m * g.fs + line + x], ph.nt);
-      else st_once(v, &R[m * g.fs + line + x], ph.nt);
+      st_once(r[m] * gi, &R[m * g.fs + line + x], ph.nt);
     }
   };
   int base = wrap ? s0 : s0 - 1;
@@ -1227,30 +1225,26 @@ __global__ void k_clear_count(unsigned long long* count) { *count = 0; }
 // launch helpers (instantiation tables)
 // ---------------------------------------------------------------------------
 template <int ND, int D, int CONV, int AVG>
-static void launch_sweep_t(const double* Q, double* R, const Grid& g, const Phys& ph, int seg, bool acc,
-                           const double* met, const double* theta, hipStream_t s) {
+static void launch_sweep_t(const double* Q, double* R, const Grid& g, const Phys& ph, int seg, const double* met,
+                           const double* theta, hipStream_t s) {
   if constexpr (D == 0 && ND == 3) {
     const int cells = sweep_xl_cells(g);
     const int nwaves = g.n[1] * g.n[2] * ((g.n[0] + cells - 1) / cells);
     const unsigned blocks = (unsigned)((nwaves + XW - 1) / XW);
-    if (acc)
-      k_char_sweep_xl<ND, CONV, AVG, true>
-          <<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nwaves, cells, g.periodic_x, met, theta);
-    else
-      k_char_sweep_xl<ND, CONV, AVG, false>
-          <<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nwaves, cells, g.periodic_x, met, theta);
-    return;
+    k_char_sweep_xl<ND, CONV, AVG>
+        <<<blocks, 64 * XW, 0, s>>>(Q, R, g, ph, nwaves, cells, g.periodic_x, met, theta);
+  } else {
+    long long lines = 1;
+    for (int e = 0; e < 3; ++e)
+      if (e != D) lines *= g.n[e];
+    seg = fit_segment(lines, g.n[D], seg, 4);
+    const long long nseg = (g.n[D] + seg - 1) / seg;
+    const long long total = lines * nseg;
+    const unsigned blocks = (unsigned)((total + 255) / 256);
+    const RkArgs none{nullptr, nullptr, 0.0, 0.0, 0};
+    // (y and z add to the directions before them, x on a line is the only one)
+    k_char_sweep<ND, D, CONV, AVG, (D > 0)><<<blocks, 256, 0, s>>>(Q, R, g, ph, seg, total, met, theta, none);
   }
-  long long lines = 1;
-  for (int e = 0; e < 3; ++e)
-    if (e != D) lines *= g.n[e];
-  seg = fit_segment(lines, g.n[D], seg, 4);
-  const long long nseg = (g.n[D] + seg - 1) / seg;
-  const long long total = lines * nseg;
-  const unsigned blocks = (unsigned)((total + 255) / 256);
-  const RkArgs none{nullptr, nullptr, 0.0, 0.0, 0};
-  if (acc) k_char_sweep<ND, D, CONV, AVG, true><<<blocks, 256, 0, s>>>(Q, R, g, ph, seg, total, met, theta, none);
-  else k_char_sweep<ND, D, CONV, AVG, false><<<blocks, 256, 0, s>>>(Q, R, g, ph, seg, total, met, theta, none);
 }
 
 // the last (z) sweep of a 3-D stage fused with the RK update
@@ -1287,35 +1281,35 @@ void launch_sweep_z_rk(int conv, int avg, int mode, const double* Q, double* R, 
 }
 
 template <int ND, int D, int CONV>
-static void launch_sweep_avg(int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg, bool acc,
+static void launch_sweep_avg(int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
                              const double* met, const double* theta, hipStream_t s) {
-  if (avg == OSBL_AVG_ROE) launch_sweep_t<ND, D, CONV, OSBL_AVG_ROE>(Q, R, g, ph, seg, acc, met, theta, s);
-  else launch_sweep_t<ND, D, CONV, OSBL_AVG_SIMPLE>(Q, R, g, ph, seg, acc, met, theta, s);
+  if (avg == OSBL_AVG_ROE) launch_sweep_t<ND, D, CONV, OSBL_AVG_ROE>(Q, R, g, ph, seg, met, theta, s);
+  else launch_sweep_t<ND, D, CONV, OSBL_AVG_SIMPLE>(Q, R, g, ph, seg, met, theta, s);
 }
 
 template <int ND, int D>
 static void launch_sweep_conv(int conv, int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
-                              const double* met, const double* theta, bool acc, hipStream_t s) {
+                              const double* met, const double* theta, hipStream_t s) {
   switch (conv) {
-    case OSBL_CONV_WENO_JS: launch_sweep_avg<ND, D, OSBL_CONV_WENO_JS>(avg, Q, R, g, ph, seg, acc, met, theta, s); break;
-    case OSBL_CONV_WENO_Z: launch_sweep_avg<ND, D, OSBL_CONV_WENO_Z>(avg, Q, R, g, ph, seg, acc, met, theta, s); break;
-    case OSBL_CONV_TENO5: launch_sweep_avg<ND, D, OSBL_CONV_TENO5>(avg, Q, R, g, ph, seg, acc, met, theta, s); break;
+    case OSBL_CONV_WENO_JS: launch_sweep_avg<ND, D, OSBL_CONV_WENO_JS>(avg, Q, R, g, ph, seg, met, theta, s); break;
+    case OSBL_CONV_WENO_Z: launch_sweep_avg<ND, D, OSBL_CONV_WENO_Z>(avg, Q, R, g, ph, seg, met, theta, s); break;
+    case OSBL_CONV_TENO5: launch_sweep_avg<ND, D, OSBL_CONV_TENO5>(avg, Q, R, g, ph, seg, met, theta, s); break;
     case CONV_WFILTER:
       // the WENO filter reconstructs with SimpleAverage (WENO_filter.py:324)
-      if constexpr (ND == 3) launch_sweep_t<ND, D, CONV_WFILTER, OSBL_AVG_SIMPLE>(Q, R, g, ph, seg, acc, met, theta, s);
+      if constexpr (ND == 3) launch_sweep_t<ND, D, CONV_WFILTER, OSBL_AVG_SIMPLE>(Q, R, g, ph, seg, met, theta, s);
       break;
-    default: launch_sweep_avg<ND, D, OSBL_CONV_TENO6>(avg, Q, R, g, ph, seg, acc, met, theta, s); break;
+    default: launch_sweep_avg<ND, D, OSBL_CONV_TENO6>(avg, Q, R, g, ph, seg, met, theta, s); break;
   }
 }
 
 void launch_sweep(int nd, int d, int conv, int avg, const double* Q, double* R, const Grid& g, const Phys& ph, int seg,
-                  const double* met, const double* theta, bool acc, hipStream_t s) {
+                  const double* met, const double* theta, hipStream_t s) {
   if (nd == 3) {
-    if (d == 0) launch_sweep_conv<3, 0>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
-    else if (d == 1) launch_sweep_conv<3, 1>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
-    else launch_sweep_conv<3, 2>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
+    if (d == 0) launch_sweep_conv<3, 0>(conv, avg, Q, R, g, ph, seg, met, theta, s);
+    else if (d == 1) launch_sweep_conv<3, 1>(conv, avg, Q, R, g, ph, seg, met, theta, s);
+    else launch_sweep_conv<3, 2>(conv, avg, Q, R, g, ph, seg, met, theta, s);
   } else {
-    launch_sweep_conv<1, 0>(conv, avg, Q, R, g, ph, seg, met, theta, acc, s);
+    launch_sweep_conv<1, 0>(conv, avg, Q, R, g, ph, seg, met, theta, s);
   }
 }
 
@@ -1332,23 +1326,26 @@ template <int ND>
 static void launch_update_nd(int conv, bool visc, int mode, const double* Q, const double* P, double* R, double* Qo,
                              double* Qn, const Grid& g, const Phys& ph, double cA, double cB, int first,
                              hipStream_t s) {
-  const bool central = conv == OSBL_CONV_CENTRAL_SKEW || conv == OSBL_CONV_CENTRAL_CONS;
-  if (central) {
-    if constexpr (ND == 1) {  // 2-D: k_central2d, 3-D: k_central3d
+  // 1-D blocks, and 3-D Euler blocks of characteristic schemes; the others' stages
+  // end in k_central2d/3d, k_char_tile2d, the viscous or general kernels
+  if constexpr (ND == 1) {
     if (conv == OSBL_CONV_CENTRAL_SKEW) {
       if (visc) launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
       else launch_update_m<ND, OSBL_CONV_CENTRAL_SKEW, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
-    } else {
+      return;
+    }
+    if (conv == OSBL_CONV_CENTRAL_CONS) {
       if (visc) launch_update_m<ND, OSBL_CONV_CENTRAL_CONS, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
       else launch_update_m<ND, OSBL_CONV_CENTRAL_CONS, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
+      return;
     }
+    if (visc) {
+      launch_update_m<ND, OSBL_CONV_WENO_Z, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
+      return;
     }
-  } else if constexpr (ND != 2) {  // 2-D: k_char_tile2d
-    if (visc) launch_update_m<ND, OSBL_CONV_WENO_Z, true>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
-    else launch_update_m<ND, OSBL_CONV_WENO_Z, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
   }
+  launch_update_m<ND, OSBL_CONV_WENO_Z, false>(mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);
 }
-
 void launch_update(int nd, int conv, bool visc, int mode, const double* Q, const double* P, double* R, double* Qo,
                    double* Qn, const Grid& g, const Phys& ph, double cA, double cB, int first, hipStream_t s) {
   if (nd == 3) launch_update_nd<3>(conv, visc, mode, Q, P, R, Qo, Qn, g, ph, cA, cB, first, s);

@@ -387,13 +387,11 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
     // viscous kernel and the y sweep accumulate, and the z sweep adds the last
     // difference and applies the RK update, so the update needs no pass of its own
     timed(c, F_SWEEP_X, [&] {
-      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, false,
-                   c->stream);
+      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, c->stream);
     });
     timed(c, F_UPDATE, [&] { launch_visc_update3d(Q, c->R, c->g, c->ph, c->vsz, c->stream); });
     timed(c, F_SWEEP_Y, [&] {
-      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, true,
-                   c->stream);
+      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, nullptr, theta, c->stream);
     });
     timed(c, F_SWEEP_Z, [&] {
       launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, theta, cA, cB,
@@ -405,16 +403,14 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
     // the same schedule on the general path: tiled viscous terms with closures,
     // metric and mu(T) (z free of both), sweeps with the metric, RK in the z sweep
     timed(c, F_SWEEP_X, [&] {
-      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[0], theta, false,
-                   c->stream);
+      launch_sweep(c->nd, 0, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[0], theta, c->stream);
     });
     timed(c, F_UPDATE, [&] {
       launch_visc_gen3d(Q, c->P, c->R, c->g, c->ph, c->bnd, c->suth ? 1 : 0, c->vsz, c->stream);
       if (c->ph.has_force) launch_body_force3d(Q, c->R, c->g, c->ph, c->stream);
     });
     timed(c, F_SWEEP_Y, [&] {
-      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[1], theta, true,
-                   c->stream);
+      launch_sweep(c->nd, 1, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[1], theta, c->stream);
     });
     timed(c, F_SWEEP_Z, [&] {
       launch_sweep_z_rk(conv, c->cfg.averaging, mode, Q, c->R, c->Qo, Qn, c->g, c->ph, c->seg, theta, cA, cB,
@@ -425,8 +421,7 @@ void stage(osbl_ctx* c, int mode, double cA, double cB, int first, double* pk = 
   if (!is_central(conv)) {
     for (int d = 0; d < c->nd; ++d) {
       timed(c, F_SWEEP_X + d, [&] {
-        launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], theta, d > 0,
-                     c->stream);
+        launch_sweep(c->nd, d, conv, c->cfg.averaging, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], theta, c->stream);
       });
     }
   }
@@ -864,7 +859,7 @@ static void filters(osbl_ctx* c) {
     for (int d = 0; d < c->nd && c->nd == 3; ++d) {
       timed(c, F_FILTER, [&] {
         launch_sweep(c->nd, d, CONV_WFILTER, OSBL_AVG_SIMPLE, Q, c->R, c->g, c->ph, c->seg, c->bnd.dm[d], nullptr,
-                     d > 0, c->stream);
+                     c->stream);
       });
     }
     timed(c, F_FILTER, [&] {

@@ -21,11 +21,8 @@ import json
 # reverse-stage kernels (first match wins)
 FAMILIES = [
     ("k_char_sweep_xl", "char_sweep_x"),
-    ("k_char_sweep<3, 0,", "char_sweep_x"),
     ("k_char_sweep<3, 1,", "char_sweep_y"),
     ("k_char_sweep<3, 2,", "char_sweep_z"),
-    ("k_char_sweep<2, 0,", "char_sweep_x"),
-    ("k_char_sweep<2, 1,", "char_sweep_y"),
     ("k_char_sweep<1, 0,", "char_sweep_x"),
     ("k_char_tile2d", "char_sweep_x"),
     ("k_line_", "char_sweep_x"),
