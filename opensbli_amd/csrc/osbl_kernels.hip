@@ -219,19 +219,21 @@ __global__ void __launch_bounds__(256) k_char_sweep(const double* __restrict__ Q
 constexpr int XW = 4;             // waves per block
 constexpr int XP = 64 + 5;        // points staged per chunk
 
-// Cells per wave: the whole row when the rows alone fill the GPU (1024 SIMDs
-// times the three waves the registers allow), else 64 k - 1 cells (k chunks
-// and the flux left of the first cell) with k as large as that number of
-// waves allows.  400^2 (400 rows, 7 waves each): 21 -> 9 us.
+// Cells per wave: the whole row, or the 63 that one chunk completes, whichever
+// leaves the busiest of the 1024 SIMDs fewer chunks (a row costs a chunk per 64
+// interfaces, one less where the periodic flux is shared; 63 cells per wave
+// cost more of them but spread them out); the whole row once the rows alone
+// give every SIMD the three waves its registers hold.  Measured (us, WENO5-Z,
+// whole row and 63 cells): 512x8x8 29 and 9, 400x20x20 29 and 16, 1000x30x30 59
+// and 47, 128x50x50 periodic 23 and 28, 256x55x55 periodic 39 and 48, 96^3 54
+// and 57.  Two to eight chunks per wave lay between or above the two.
 static int sweep_xl_cells(const Grid& g) {
   const long long rows = (long long)g.n[1] * g.n[2];
   const int n = g.n[0];
   if (rows >= 3072 || n <= 63) return n;
-  for (int k = (n + 63) / 64; k > 1; --k) {
-    const int cells = 64 * k - 1;
-    if (rows * ((n + cells - 1) / cells) >= 3072) return cells >= n ? n : cells;
-  }
-  return 63;
+  const long long whole = (rows + 1023) / 1024 * ((n + (g.periodic_x ? 0 : 1) + 63) / 64);
+  const long long single = (rows * ((n + 62) / 63) + 1023) / 1024;
+  return whole < single ? n : 63;
 }
 
 // (at least three waves per SIMD)

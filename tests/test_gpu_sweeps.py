@@ -59,6 +59,15 @@ def test_3d_shapes(n, conv, oracle):
     _check(problem, q0, oracle, f"3-D {n} {conv}")
 
 
+@pytest.mark.parametrize("bc", ["periodic", "extrap0"])
+@pytest.mark.parametrize("n", [(63, 33, 32), (64, 33, 32), (65, 33, 32), (127, 34, 31), (130, 10, 9), (66, 56, 55)])
+def test_3d_rows(n, bc, oracle):
+    """Rows of one wave (periodic: the flux left of cell 0 is the last one's)
+    and rows split among waves, below and above 1024 and 3072 rows."""
+    problem, q0 = _block(n, "weno_z", bc)
+    _check(problem, q0, oracle, f"3-D rows {n} {bc}")
+
+
 @pytest.mark.parametrize("bc", ["periodic", "symmetry"])
 @pytest.mark.parametrize("conv,rk,viscous", [("central_skew", "ls3", "const"), ("central_skew", "rk3", "none"),
                                              ("central_cons", "rk3", "const"), ("central_cons", "ls3", "none")])
