@@ -717,8 +717,8 @@ __device__ __forceinline__ double recon_gap(const double dcs[5], const double dc
 // The sweeps are bound by FP64 issue (and the clock that its power allows):
 // against projecting every point on the full rows of L this takes the y
 // sweep of WENO5-Z, Roe, 3-D, from ~1300 to ~980 VALU instructions per cell;
-// 256^3: y 0.785 -> 0.64 ms, z with the RK update 0.83 -> 0.70, x 0.89 ->
-// 0.75 (the step 8.9 -> 7.7 ms; TENO6 at 131x97x75 18 % faster).
+// 256^3: y 0.785 -> 0.57 ms, z with the RK update 0.83 -> 0.67, x 0.89 -> 0.62
+// (with its pipelined walk); the step 8.9 -> 7.3 ms, TENO6 12.8 -> 10.8.
 // ---------------------------------------------------------------------------
 template <int ND, int D, int CONV, class W>
 __device__ __forceinline__ void char_fields(const W& w, const Avg<ND>& v, const Phys& ph, double ct,

@@ -441,7 +441,7 @@ def test_channel_with_body_force(n, steps, oracle):
     """The TENO channel structure (apps/channel_flow/compressible_TCF_TENO):
     body force, Sutherland viscosity, isothermal walls on a wall-clustered
     grid, periodic x; 3-D through the tiled general schedule (the force as its
-    own pass), 2-D through the per-point general kernel; against the oracle."""
+    own pass), 2-D through the characteristic tile; against the oracle."""
     from opensbli_amd.native import Block
     from opensbli_amd.problems import channel
     _say(f"case channel with body force {n}, {steps} steps")
