@@ -1,4 +1,4 @@
-// The TENO weights and the short quotients and roots of osbl_device.h on the CPU.
+// The TENO and WENO weights and the short quotients and roots of osbl_device.h on the CPU.
 #include <algorithm>
 
 #include <hip/hip_runtime.h>
@@ -17,6 +17,15 @@ extern "C" void teno(int six, int quirk, long n, const double* d, double eps, do
     if (six && quirk) teno_gap<true, true>(x[0], x[1], x[2], x[3], x[4], eps, ct, num[i], den[i]);
     else if (six) teno_gap<true, false>(x[0], x[1], x[2], x[3], x[4], eps, ct, num[i], den[i]);
     else teno_gap<false, false>(x[0], x[1], x[2], x[3], x[4], eps, ct, num[i], den[i]);
+  }
+}
+
+// the same of WENO5-Z and -JS, from four differences each
+extern "C" void weno(int z, long n, const double* d, double eps, double* num, double* den) {
+  for (long i = 0; i < n; ++i) {
+    const double* x = d + 5 * i;
+    if (z) weno5_gap<true>(x[0], x[1], x[2], x[3], eps, num[i], den[i]);
+    else weno5_gap<false>(x[0], x[1], x[2], x[3], eps, num[i], den[i]);
   }
 }
 

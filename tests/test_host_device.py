@@ -118,6 +118,24 @@ def test_teno_weights_over_the_range_of_the_quotients(recon, scale, eps, six, qu
     assert np.all(err <= 1e-12), (err.max(), int((~(err <= 1e-12)).sum()))
 
 
+@pytest.mark.parametrize("z,eps", [(1, 4e-14), (0, 4e-6)])
+def test_weno_weights_at_the_largest_differences(recon, z, eps):
+    """Differences of 1e22, the bound that the header states (a reconstruction
+    gets the sum or difference of two such): the same weights as in units 2^40
+    times larger."""
+    rs = np.random.RandomState(3)
+    n = 4000
+    d = rs.uniform(-2e22, 2e22, (n, 5))
+    f = ctypes.c_double
+    out = []
+    for unit in (1.0, 2.0 ** -40):
+        num, den = np.empty(n), np.empty(n)
+        recon.weno(z, ctypes.c_long(n), _dp(d * unit), f(eps * unit * unit), _dp(num), _dp(den))
+        assert np.isfinite(num).all() and np.isfinite(den).all()
+        out.append(num / den / unit)
+    assert np.abs(out[0] - out[1]).max() <= 1e-12 * 2e22
+
+
 def test_quotients_and_roots_are_rounded_correctly_or_nearly(recon):
     """a/b, 1/b and sqrt(b) from estimates as coarse as the hardware's: within
     0.501 units in the last place (an IEEE result is within 0.5)."""
