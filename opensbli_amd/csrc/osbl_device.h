@@ -86,11 +86,12 @@ __host__ __device__ __forceinline__ double pow10i(int n) {
 // each operation rounded separately so that floor() sees the same value as a
 // build without contraction
 __device__ __forceinline__ double adaptive_ct(double m, const Phys& ph) {
-  const double t = __dsub_rn(1.0, m);
-  const double t2 = __dmul_rn(t, t);
-  const double t4 = __dmul_rn(t2, t2);
-  const double q = __dmul_rn(t4, __dadd_rn(1.0, __dmul_rn(4.0, m)));
-  const double beta = __dsub_rn(ph.teno_a1, __dmul_rn(ph.teno_a2, __dsub_rn(1.0, q)));
+#pragma clang fp contract(off)
+  const double t = 1.0 - m;
+  const double t2 = t * t;
+  const double t4 = t2 * t2;
+  const double q = t4 * (1.0 + 4.0 * m);
+  const double beta = ph.teno_a1 - ph.teno_a2 * (1.0 - q);
   return 1.0 / pow10i((int)floor(beta));
 }
 
@@ -177,10 +178,11 @@ __device__ __forceinline__ double max_abs(double m, double x) {
   return r;
 }
 
-// Every operation is rounded on its own (no contraction into FMAs), so a
-// point's values are bit-identical wherever a kernel evaluates them -- in a
-// sweep's prologue or in its loop -- and a direction along which the state is
-// uniform keeps exactly zero flux differences.
+// Every kernel and every place in one takes a point's values from here, so they
+// are the same bits in a sweep's prologue and in its loop, and a direction along
+// which the state is uniform keeps exactly zero flux differences.  (The
+// compiler may contract the operations; it does so alike wherever they are
+// inlined.)
 template <int ND>
 __device__ __forceinline__ void finish_pt(Pt<ND>& s, const Phys& ph) {
   const double ir = recip_pos(s.q[0]);
