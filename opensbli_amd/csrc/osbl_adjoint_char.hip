@@ -4,10 +4,9 @@
 //
 // R_i = -sum_d (F_{i+1/2} - F_{i-1/2}) / Delta_d with F_{i+1/2} a function of
 // the six states Q_{i-2..i+3}.  Its vector-Jacobian product with weights mu is
-// sum over interfaces of J_p^T nu, nu = (mu_{i+1} - mu_i)/Delta_d.  A thread
-// slides the forward 6-point window along a grid line; per interface it
-// re-evaluates the forward flux of every characteristic field and runs it
-// backwards:
+// sum over interfaces of J_p^T nu, nu = (mu_{i+1} - mu_i)/Delta_d.  A lane takes
+// one interface, re-evaluates the forward flux of every characteristic field
+// and runs it backwards:
 //   * the reconstructions through a hand-written reverse of the WENO-Z
 //     weights in difference form (tau^2 is smooth; no branch),
 //   * lambda_max = max_p |lambda(p)| to its first maximising point (the

@@ -1,7 +1,8 @@
 // osbl_boundary.hip -- boundary kernels of non-periodic faces and the
-// periodic exchange of one direction.  Each kernel runs over the boundary
-// plane of its face with the other directions' halos included
-// (bc_core.py:163-171); one thread owns one line normal to the face.
+// periodic exchange of one direction.  The faces' kernels run over the boundary
+// planes of both faces of a direction (2-D: of all four faces) with the other
+// directions' halos included (bc_core.py:163-171); one thread owns one line
+// normal to a face.
 #include "osbl_kernels.h"
 
 namespace osbl {

@@ -9,7 +9,8 @@
 //     Der.differentiate (parsing.py:141-186),
 //   * the central convective forms with the same closures,
 // fused with the RK update.  The characteristic fluxes come from the sweeps of
-// osbl_kernels.hip, which apply the metric to their flux differences.
+// osbl_kernels.hip, which apply the metric to their flux differences; 2-D
+// characteristic blocks do all of this in osbl_tile2d.hip.
 #include "osbl_kernels.h"
 #include "osbl_visc.h"
 

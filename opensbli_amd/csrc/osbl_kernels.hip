@@ -1,8 +1,10 @@
 // osbl_kernels.hip -- gfx950 kernels of one RK stage of the OpenSBLI RHS:
-//   * boundary fills (periodic wrap, zeroth-order extrapolation),
-//   * constituent relations for the central/viscous stencils,
-//   * one characteristic LLF sweep per direction (WENO5-JS/Z, TENO5/6),
-//   * the fused central (skew or conservative) + viscous + RK update.
+//   * the periodic halo pass and the constituent relations of what still reads them,
+//   * one characteristic LLF sweep per direction of 1-D and 3-D blocks
+//     (WENO5-JS/Z, TENO5/6), their viscous terms and RK update,
+//   * the central (skew or conservative) stage of 3-D blocks in one kernel, of
+//     1-D blocks as a fused update.
+// (2-D blocks: osbl_tile2d.hip; 1-D lines with extrapolation ends: osbl_line.h.)
 #include "osbl_kernels.h"
 
 namespace osbl {

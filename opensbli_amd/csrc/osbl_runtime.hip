@@ -5,6 +5,7 @@
 // sequence of stream-ordered launches per RK stage:
 //   boundary conditions -> [constituent relations] -> characteristic sweeps
 //   -> fused central/viscous residual + RK update -> boundary conditions.
+// (Tiled stages are one launch and, on periodic blocks, need no boundary pass.)
 #include <algorithm>
 #include <cmath>
 #include <cstdarg>
